@@ -70,7 +70,7 @@ enum mattn_status {
  * every present tile (float16, 32 KiB per 128 x 128 tile) in the workspace and
  * the dQ stage computes dQ = dS K from it instead of recomputing S and dP.
  * The workspace then takes mattn_bwd_workspace_bytes(p, bm) bytes.  For
- * 16-bit inputs at D <= 128 (ignored on the SIMT path).  Faster at D = 128,
+ * 16-bit inputs at D <= 128 (ignored elsewhere).  Faster at D = 128,
  * where recomputing costs more than streaming 2 bytes per allowed pair. */
 #define MATTN_BWD_DS 2
 /* mattn_problem.flags: float32 arithmetic for 16-bit inputs.  The problem runs
@@ -169,8 +169,9 @@ int mattn_validate(const mattn_problem* p, const mattn_blockmap* bm);
  * invalid problem.
  * Head dimensions 64 and 128 with 16-bit inputs run on the MFMA kernels;
  * float32 inputs, D = 256 and 512 for every dtype (the host pads d in (128, 512]
- * with zeros) and MATTN_PRECISE problems run on float32 SIMT kernels, whose
- * workspace is one float32 per query row. */
+ * with zeros) and MATTN_PRECISE problems run on kernels of float32 accuracy
+ * (MFMA on three bfloat16 pieces per float32 operand up to D = 256 without
+ * MATTN_PRECISE, SIMT otherwise), whose workspace is one float32 per query row. */
 size_t mattn_workspace_bytes(const mattn_problem* p);
 
 /* Bytes of device workspace mattn_bwd needs for this map, MATTN_BWD_DS
@@ -216,8 +217,8 @@ int mattn_bwd(const mattn_problem* p, const mattn_blockmap* bm,
  * MATTN_BWD_PRE (delta = rowsum(dO * O) and the float16 copy of dO, into the
  * workspace), MATTN_BWD_DKDV (also writes the float16 copy of K, and with
  * MATTN_BWD_DS every tile's dS, into the workspace), then MATTN_BWD_DQ (reads
- * them).  On the SIMT path MATTN_BWD_PRE does nothing: those kernels take
- * dP - delta as dO . (V - O) per pair.  mattn_bwd == the three stages
+ * them).  On the SIMT path (MATTN_PRECISE, D = 512) MATTN_BWD_PRE does nothing:
+ * those kernels take dP - delta as dO . (V - O) per pair.  mattn_bwd == the three stages
  * in order.  Same arguments as mattn_bwd; exposed so a caller can time the
  * stages. */
 enum mattn_bwd_stage { MATTN_BWD_PRE = 0, MATTN_BWD_DKDV = 1, MATTN_BWD_DQ = 2 };

@@ -13,12 +13,13 @@ Mirrors the public interface of ``/root/reference/jaxmodules/attention.py``:
   enable_gqa, return_lse)`` (attention.py:456-692) on the same kernels, its
   ``BlockMask`` handed over as a tile map (``BlockMask.tile_map``).
 
-The kernels are built for head dimensions 64, 128 and 256; other head
-dimensions up to 256 are zero-padded on the GPU to the next of the three (zero
+The kernels are built for head dimensions 64, 128, 256 and 512; other head
+dimensions up to 512 are zero-padded on the GPU to the next of the four (zero
 columns of Q and K leave every score unchanged, zero columns of V give zero
 output columns, which are sliced off; the scale stays 1/sqrt(true d)).  16-bit
-inputs at 64 and 128 run on the MFMA kernels; float32 inputs, and every dtype
-at 256, on float32 SIMT kernels.
+inputs at 64 and 128 run on float16-operand MFMA kernels; float32 inputs, and
+every dtype at 256, on MFMA kernels of float32 accuracy (three bfloat16 pieces
+per float32 operand); 512, and precision "highest", on SIMT kernels.
 
 Arrays are torch tensors on the GPU (jax is not available in this image; the
 jax.ffi binding a jax user would register is described with the C ABI).  The
@@ -496,8 +497,8 @@ def use_precise(precision: Optional[str], scale: float, d: int) -> bool:
     """Whether a problem runs with MATTN_PRECISE.
 
     "default": 16-bit inputs run on the MFMA kernels, whose computed operands
-    (P, dS, dO) are rounded to float16, 11 significant bits; float32 inputs on
-    the float32 SIMT kernels.  "highest": the float32 SIMT kernels for every
+    (P, dS, dO) are rounded to float16, 11 significant bits (not at d > 128);
+    float32 inputs on kernels of float32 accuracy.  "highest": the float32 SIMT kernels for every
     dtype, with the scores formed as compensated dot products (about twice
     float32's precision).  None picks "highest" for kernels sharper than the
     default scale 1/sqrt(d) (threshold_kernel's is 1, attention.py:18-36):

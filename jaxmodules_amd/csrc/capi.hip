@@ -1,8 +1,9 @@
 // C ABI of the library (declared in include/mattn.h): argument validation,
 // workspace layouts, kernel-argument packing and launch selection.  Host code
 // only; the kernels live in fwd.hip, bwd_pre.hip, bwd_dkdv.hip, bwd_dq.hip
-// (16-bit inputs, D = 64 and 128: MFMA) and simt.hip (float32 inputs, and
-// every input dtype at D = 256 and 512: float32 SIMT arithmetic).
+// (16-bit inputs, D = 64 and 128: MFMA on float16 operands), split3.hip (float32
+// inputs up to D = 256 and 16-bit inputs at D = 256: MFMA at float32 accuracy) and
+// simt.hip (D = 512 and MATTN_PRECISE: SIMT arithmetic).
 #include <math.h>
 
 #include <mutex>
@@ -35,7 +36,7 @@ bool strides_ok(const int64_t s[3], int esz) {
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// problems served by the SIMT kernels (float32 arithmetic), which need no
+// problems served in float32 accuracy (split3.hip, simt.hip), which need no
 // residual and no backward workspace beyond one float per query row
 bool simt_path(const mattn_problem* p) {
   return p->dtype == MATTN_F32 || p->D > 128 || (p->flags & MATTN_PRECISE);

@@ -1,12 +1,10 @@
 // SIMT (no MFMA) masked-attention kernels: the forward and the three backward
 // stages in float32 arithmetic, for
-//   * float32 inputs, whose 1e-5 tolerance rules out 16-bit operands, at head
-//     dimensions 64, 128 and 256;
-//   * 16-bit inputs at head dimensions 256 and 512 (any d in (128, 512],
-//     zero-padded by the host), which the MFMA kernels' register and LDS
-//     tiling does not hold.
-//   * 16-bit inputs at D = 64 and 128 under MATTN_PRECISE (callers whose
-//     kernels are too sharp for float16 operands).
+//   * D = 512 (any d in (256, 512], zero-padded by the host), every input dtype;
+//   * MATTN_PRECISE at every head dimension (callers whose kernels are too
+//     sharp for float16 operands).
+// (float32 inputs, and 16-bit inputs at D = 256, run on the matrix cores:
+// split3.hip; launch_fwd_simt and launch_bwd_simt hand them over.)
 // Same maths and tile walk as the MFMA path (/root/reference/jaxmodules/
 // attention.py:52-105 forward, :266-342 backward): per 32-key (or 32-query)
 // sub-block an online softmax, P = exp2(scale_log2 S - lse) in the backward,
@@ -404,66 +402,66 @@ void bwd_dkdv_simt(KArgs a) {
   }
 }
 
-// the stages of one (D, TPR, input, output) combination
+// the stages of one (D, TPR, input, output) combination; without PREC only D = 512
+// comes here
 template <int D, int TPR, class IT, class OT>
 struct Simt {
   static constexpr int SPLIT = TILE * TPR / 512;
+  template <bool PREC>
   static void fwd(const KArgs& a, int grid, hipStream_t st) {
-    if (a.precise) hipLaunchKernelGGL((fwd_simt<D, TPR, IT, OT, true>), dim3(grid * SPLIT), dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((fwd_simt<D, TPR, IT, OT, false>), dim3(grid * SPLIT), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((fwd_simt<D, TPR, IT, OT, PREC>), dim3(grid * SPLIT), dim3(512), 0, st, a);
   }
+  template <bool PREC>
   static void bwd(const KArgs& a, int stage, int q_grid, int kv_grid, hipStream_t st) {
-    if (stage == MATTN_BWD_PRE) {
-      // nothing: the SIMT kernels form dP - delta per pair from O
-    } else if (stage == MATTN_BWD_DKDV) {
-      if (a.precise)
-        hipLaunchKernelGGL((bwd_dkdv_simt<D, TPR, IT, OT, true>), dim3(kv_grid * SPLIT), dim3(512), 0, st, a);
-      else
-        hipLaunchKernelGGL((bwd_dkdv_simt<D, TPR, IT, OT, false>), dim3(kv_grid * SPLIT), dim3(512), 0, st, a);
-    } else {
-      if (a.precise)
-        hipLaunchKernelGGL((bwd_dq_simt<D, TPR, IT, OT, true>), dim3(q_grid * SPLIT), dim3(512), 0, st, a);
-      else
-        hipLaunchKernelGGL((bwd_dq_simt<D, TPR, IT, OT, false>), dim3(q_grid * SPLIT), dim3(512), 0, st, a);
-    }
+    if (stage == MATTN_BWD_DKDV)
+      hipLaunchKernelGGL((bwd_dkdv_simt<D, TPR, IT, OT, PREC>), dim3(kv_grid * SPLIT), dim3(512), 0, st, a);
+    else if (stage == MATTN_BWD_DQ)
+      hipLaunchKernelGGL((bwd_dq_simt<D, TPR, IT, OT, PREC>), dim3(q_grid * SPLIT), dim3(512), 0, st, a);
+    // MATTN_BWD_PRE: nothing, these kernels form dP - delta per pair from O
   }
 };
 
-// f(Simt<...>{}) for the problem's combination: D = 64, 128 (4 threads per
-// row) or 256 (8); float32 inputs, or 16-bit inputs with a float32 or
+// f(Simt<...>{}, precise) for the problem's combination: 4 threads per row at D = 64
+// and 128, 8 at 256, 16 at 512; float32 inputs, or 16-bit inputs with a float32 or
 // same-dtype output
-template <class Tag, class F>
-void dispatch16(int D, bool of32, F&& f) {
-  if (D == 64) { if (of32) f(Simt<64, 4, Tag, float>{}); else f(Simt<64, 4, Tag, Tag>{}); }
-  else if (D == 128) { if (of32) f(Simt<128, 4, Tag, float>{}); else f(Simt<128, 4, Tag, Tag>{}); }
-  else if (D == 256) { if (of32) f(Simt<256, 8, Tag, float>{}); else f(Simt<256, 8, Tag, Tag>{}); }
-  else { if (of32) f(Simt<512, 16, Tag, float>{}); else f(Simt<512, 16, Tag, Tag>{}); }
+template <class IT, class OT, class F>
+void dispatch_d(int D, bool precise, F&& f) {
+  if (D == 64) f(Simt<64, 4, IT, OT>{}, std::true_type{});
+  else if (D == 128) f(Simt<128, 4, IT, OT>{}, std::true_type{});
+  else if (D == 256) f(Simt<256, 8, IT, OT>{}, std::true_type{});
+  else if (precise) f(Simt<512, 16, IT, OT>{}, std::true_type{});
+  else f(Simt<512, 16, IT, OT>{}, std::false_type{});
 }
 template <class F>
-hipError_t dispatch(int D, int dtype, int o_dtype, F&& f) {
+hipError_t dispatch(int D, int dtype, int o_dtype, bool precise, F&& f) {
   const bool of32 = o_dtype == MATTN_F32;
-  if (dtype == MATTN_F32) {
-    if (D == 64) f(Simt<64, 4, float, float>{});
-    else if (D == 128) f(Simt<128, 4, float, float>{});
-    else if (D == 256) f(Simt<256, 8, float, float>{});
-    else f(Simt<512, 16, float, float>{});
-  } else if (dtype == MATTN_BF16) {
-    dispatch16<bf16_tag>(D, of32, f);
-  } else {
-    dispatch16<f16_tag>(D, of32, f);
-  }
+  if (dtype == MATTN_F32) dispatch_d<float, float>(D, precise, f);
+  else if (dtype == MATTN_BF16 && of32) dispatch_d<bf16_tag, float>(D, precise, f);
+  else if (dtype == MATTN_BF16) dispatch_d<bf16_tag, bf16_tag>(D, precise, f);
+  else if (of32) dispatch_d<f16_tag, float>(D, precise, f);
+  else dispatch_d<f16_tag, f16_tag>(D, precise, f);
   return hipGetLastError();
 }
 
 }  // namespace
 
+bool s3_path(int D, int dtype, bool precise);
+hipError_t launch_fwd_s3(const KArgs& a, int D, int dtype, int o_dtype, int grid, hipStream_t st);
+hipError_t launch_bwd_s3(const KArgs& a, int D, int dtype, int o_dtype, int stage, int q_grid, int kv_grid,
+                         hipStream_t st);
+
 hipError_t launch_fwd_simt(const KArgs& a, int D, int dtype, int o_dtype, int grid, hipStream_t st) {
-  return dispatch(D, dtype, o_dtype, [&](auto s) { decltype(s)::fwd(a, grid, st); });
+  if (s3_path(D, dtype, a.precise)) return launch_fwd_s3(a, D, dtype, o_dtype, grid, st);
+  return dispatch(D, dtype, o_dtype, a.precise,
+                  [&](auto s, auto p) { decltype(s)::template fwd<decltype(p)::value>(a, grid, st); });
 }
 
 hipError_t launch_bwd_simt(const KArgs& a, int D, int dtype, int o_dtype, int stage, int q_grid, int kv_grid,
                            hipStream_t st) {
-  return dispatch(D, dtype, o_dtype, [&](auto s) { decltype(s)::bwd(a, stage, q_grid, kv_grid, st); });
+  if (s3_path(D, dtype, a.precise)) return launch_bwd_s3(a, D, dtype, o_dtype, stage, q_grid, kv_grid, st);
+  return dispatch(D, dtype, o_dtype, a.precise, [&](auto s, auto p) {
+    decltype(s)::template bwd<decltype(p)::value>(a, stage, q_grid, kv_grid, st);
+  });
 }
 
 }  // namespace mattn
