@@ -445,7 +445,7 @@ def summary(r, ms, kern, graph_ms=None):
                                 "masks": r.tm.n_masks, "built_by": r.trace_how,
                                 "build_s": round(r.trace_s, 3)},
                    "bwd_dq": "from stored dS" if r.stored_ds else "recomputes S and dP",
-                   "precision": "highest (float32 SIMT)" if r.precise else "default (float16-operand MFMA)",
+                   "precision": "highest (float64 MFMA)" if r.precise else "default (float16-operand MFMA)",
                    "bwd_workspace_bytes": r.ws_bytes}
 
 
@@ -465,7 +465,7 @@ def main():
     ap.add_argument("--stored-ds", action="store_true",
                     help="run dQ from the stored dS wherever the kernels allow it (head dim <= 128)")
     ap.add_argument("--precise", action="store_true",
-                    help="measure precision=\"highest\" (MATTN_PRECISE: float32 SIMT kernels, compensated "
+                    help="measure precision=\"highest\" (MATTN_PRECISE: float64 MFMA kernels, float64 "
                          "scores) instead of the default MFMA path; not the headline")
     ap.add_argument("--tilemap", action="store_true",
                     help="instead: time the tile-map build of configs 3-5, host tracer vs GPU classifier")

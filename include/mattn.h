@@ -73,9 +73,10 @@ enum mattn_status {
  * 16-bit inputs at D <= 128 (ignored elsewhere).  Faster at D = 128,
  * where recomputing costs more than streaming 2 bytes per allowed pair. */
 #define MATTN_BWD_DS 2
-/* mattn_problem.flags: float32 arithmetic for 16-bit inputs.  The problem runs
- * on the SIMT kernels (every product and sum in float32, the inputs read
- * exactly), as float32 inputs do, instead of the MFMA kernels, whose
+/* mattn_problem.flags: more than float32's precision for every input dtype.  The
+ * problem runs on the float64 matrix cores (D = 512: on SIMT kernels), the inputs
+ * read exactly, instead of the kernels of float32 accuracy (float32 inputs,
+ * D > 128) or the MFMA kernels, whose
  * operands P, dS and dO are rounded to float16 (11 significant bits) -- except
  * in split tiles: 128-row query tiles with a row whose largest attention
  * weight reaches 1/32, whose O, lse and gradient terms the MFMA path forms
@@ -85,9 +86,9 @@ enum mattn_status {
  * For kernels sharper than the default scale 1/sqrt(d) (the reference's
  * threshold_kernel has scale 1, attention.py:18-36), where rows concentrate
  * on single keys and dS = P (dP - delta) cancels below the float16 operand
- * rounding.  The scores are then compensated dot products (about twice
- * float32's precision) for every dtype, O and the row sums accumulate in
- * float64, and the forward's residual (mattn_fwd_workspace_bytes) holds what
+ * rounding.  The scores, O and the row sums then accumulate in float64 (at
+ * D = 512 the scores are compensated dot products, about twice float32's
+ * precision), and the forward's residual (mattn_fwd_workspace_bytes) holds what
  * the stored lse and O round off (one float per query row and per element of
  * O), which the backward reads. */
 #define MATTN_PRECISE 4
@@ -170,8 +171,8 @@ int mattn_validate(const mattn_problem* p, const mattn_blockmap* bm);
  * Head dimensions 64 and 128 with 16-bit inputs run on the MFMA kernels;
  * float32 inputs, D = 256 and 512 for every dtype (the host pads d in (128, 512]
  * with zeros) and MATTN_PRECISE problems run on kernels of float32 accuracy
- * (MFMA on three bfloat16 pieces per float32 operand up to D = 256 without
- * MATTN_PRECISE, SIMT otherwise), whose workspace is one float32 per query row. */
+ * (up to D = 256 MFMA on three bfloat16 pieces per float32 operand, or float64
+ * MFMA with MATTN_PRECISE; SIMT at D = 512), whose workspace is one float32 per query row. */
 size_t mattn_workspace_bytes(const mattn_problem* p);
 
 /* Bytes of device workspace mattn_bwd needs for this map, MATTN_BWD_DS
@@ -217,8 +218,8 @@ int mattn_bwd(const mattn_problem* p, const mattn_blockmap* bm,
  * MATTN_BWD_PRE (delta = rowsum(dO * O) and the float16 copy of dO, into the
  * workspace), MATTN_BWD_DKDV (also writes the float16 copy of K, and with
  * MATTN_BWD_DS every tile's dS, into the workspace), then MATTN_BWD_DQ (reads
- * them).  On the SIMT path (MATTN_PRECISE, D = 512) MATTN_BWD_PRE does nothing:
- * those kernels take dP - delta as dO . (V - O) per pair.  mattn_bwd == the three stages
+ * them).  Under MATTN_PRECISE and at D = 512 MATTN_BWD_PRE does nothing: those
+ * kernels form delta themselves, or dP - delta as dO . (V - O) per pair.  mattn_bwd == the three stages
  * in order.  Same arguments as mattn_bwd; exposed so a caller can time the
  * stages. */
 enum mattn_bwd_stage { MATTN_BWD_PRE = 0, MATTN_BWD_DKDV = 1, MATTN_BWD_DQ = 2 };

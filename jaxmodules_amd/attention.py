@@ -19,7 +19,8 @@ columns of Q and K leave every score unchanged, zero columns of V give zero
 output columns, which are sliced off; the scale stays 1/sqrt(true d)).  16-bit
 inputs at 64 and 128 run on float16-operand MFMA kernels; float32 inputs, and
 every dtype at 256, on MFMA kernels of float32 accuracy (three bfloat16 pieces
-per float32 operand); 512, and precision "highest", on SIMT kernels.
+per float32 operand); precision "highest" on the float64 matrix cores; 512 on
+float32 SIMT kernels.
 
 Arrays are torch tensors on the GPU (jax is not available in this image; the
 jax.ffi binding a jax user would register is described with the C ABI).  The
@@ -357,9 +358,9 @@ def mattn_forward(q, k, v, tm: bmap.TileMap, scale: float, out_dtype=torch.float
     mattn_fwd.  ``heads_major`` lays O out in memory as [B, Hq, N, d] (the
     returned tensor is the [B, N, Hq, d] view of it).  The residual (a uint8
     tensor; None for float32 inputs, at d = 256 and with ``precise``, which
-    the SIMT kernels serve) holds the float16 V copy and, with
+    other kernels serve) holds the float16 V copy and, with
     ``for_backward``, the float16 Q copy that mattn_backward reads.
-    ``precise``: float32 arithmetic for 16-bit inputs (MATTN_PRECISE)."""
+    ``precise``: MATTN_PRECISE (float64 products and sums)."""
     lib = _lib.load()
     B, N, Hq, d = q.shape
     if heads_major:
@@ -498,9 +499,9 @@ def use_precise(precision: Optional[str], scale: float, d: int) -> bool:
 
     "default": 16-bit inputs run on the MFMA kernels, whose computed operands
     (P, dS, dO) are rounded to float16, 11 significant bits (not at d > 128);
-    float32 inputs on kernels of float32 accuracy.  "highest": the float32 SIMT kernels for every
-    dtype, with the scores formed as compensated dot products (about twice
-    float32's precision).  None picks "highest" for kernels sharper than the
+    float32 inputs on kernels of float32 accuracy.  "highest": float64 products
+    and sums for every dtype (d > 256: float32 with compensated scores, about
+    twice float32's precision).  None picks "highest" for kernels sharper than the
     default scale 1/sqrt(d) (threshold_kernel's is 1, attention.py:18-36):
     their logits spread sqrt(d) times wider, rows concentrate on single keys,
     dS = P (dP - delta) cancels below what 11-bit operands resolve, and scores
@@ -625,8 +626,8 @@ def masked_attention_via_map(
         reference returns (its running accumulators are float32,
         attention.py:173); pass Q.dtype for a 16-bit output.
     precision: None, "default" or "highest" (use_precise): 16-bit inputs run
-        on float16-operand MFMA kernels by default and in float32 arithmetic
-        (compensated scores) with "highest", which None selects for kernels
+        on float16-operand MFMA kernels by default and in float64
+        products and sums with "highest", which None selects for kernels
         sharper than default_kernel (threshold_kernel).  Not a reference
         argument.
 
@@ -731,7 +732,7 @@ def flex_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     mismatches, NotImplementedError for ``return_lse``).  ``score_mod`` has no
     kernel here and raises NotImplementedError, as does a value head dimension
     different from the query's.  ``precision`` as for masked_attention_via_map
-    (None selects float32 arithmetic for a ``scale`` above 1/sqrt(E)).
+    (None selects "highest" for a ``scale`` above 1/sqrt(E)).
     """
     if return_lse:
         raise NotImplementedError("return_lse is not supported yet")

@@ -2,8 +2,8 @@
 // workspace layouts, kernel-argument packing and launch selection.  Host code
 // only; the kernels live in fwd.hip, bwd_pre.hip, bwd_dkdv.hip, bwd_dq.hip
 // (16-bit inputs, D = 64 and 128: MFMA on float16 operands), split3.hip (float32
-// inputs up to D = 256 and 16-bit inputs at D = 256: MFMA at float32 accuracy) and
-// simt.hip (D = 512 and MATTN_PRECISE: SIMT arithmetic).
+// inputs up to D = 256 and 16-bit inputs at D = 256: MFMA at float32 accuracy),
+// precise.hip (MATTN_PRECISE up to D = 256: float64 MFMA) and simt.hip (D = 512).
 #include <math.h>
 
 #include <mutex>
@@ -36,7 +36,7 @@ bool strides_ok(const int64_t s[3], int esz) {
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// problems served in float32 accuracy (split3.hip, simt.hip), which need no
+// problems served in float32 accuracy or better (split3.hip, precise.hip, simt.hip), which need no
 // residual and no backward workspace beyond one float per query row
 bool simt_path(const mattn_problem* p) {
   return p->dtype == MATTN_F32 || p->D > 128 || (p->flags & MATTN_PRECISE);
@@ -59,7 +59,7 @@ size_t ds_slots(const mattn_problem* p, const mattn_blockmap* bm) {
 // the float16 rounding of their operands), and per key tile a flag: a split
 // row has an allowed key there (its dK/dV column then takes the split
 // products; cleared by the V' conversion, set by the split rows' walk).
-// MATTN_PRECISE on the SIMT kernels: what the stored lse and O round off
+// MATTN_PRECISE: what the stored lse and O round off
 // (float32, [B, Hq, Lq] and [B, Hq, Lq, D]), which the backward adds back.
 struct FwdWs {
   size_t vh, qh, vsc, vmax, qsc, pmx, srow, scol, lse_lo, o_lo, total;

@@ -95,9 +95,9 @@ struct KArgs {
   const int* col_row;
   int ds_nnz;
   const int* kv_desc;  // per dK/dV launch slot: { item, g, e, e_end, n_sub, qt, mask, row }
-  int precise;         // MATTN_PRECISE: the SIMT kernels form the scores as compensated dot products
-  float* lse_lo;       // MATTN_PRECISE (SIMT, forward residual): [B, Hq, Lq], (m + log2 l) - lse
-  float* o_lo;         // MATTN_PRECISE (SIMT, forward residual): [B, Hq, Lq, D], exact O - stored O
+  int precise;         // MATTN_PRECISE: float64 (D = 512: compensated) scores and sums
+  float* lse_lo;       // MATTN_PRECISE (forward residual): [B, Hq, Lq], (m + log2 l) - lse
+  float* o_lo;         // MATTN_PRECISE (forward residual): [B, Hq, Lq, D], exact O - stored O
   // Split rows (MFMA path): a row whose largest attention weight reaches
   // SPLIT_P.  The forward leaves per query tile the largest weight of its
   // rows (pmx) and a 128-bit mask of its split rows (srow, 4 words, bit i of

@@ -1,10 +1,8 @@
 // SIMT (no MFMA) masked-attention kernels: the forward and the three backward
-// stages in float32 arithmetic, for
-//   * D = 512 (any d in (256, 512], zero-padded by the host), every input dtype;
-//   * MATTN_PRECISE at every head dimension (callers whose kernels are too
-//     sharp for float16 operands).
-// (float32 inputs, and 16-bit inputs at D = 256, run on the matrix cores:
-// split3.hip; launch_fwd_simt and launch_bwd_simt hand them over.)
+// stages in float32 arithmetic for D = 512 (any d in (256, 512], zero-padded by the
+// host), every input dtype, with and without MATTN_PRECISE.  The other problems of
+// float32 accuracy run on the matrix cores: split3.hip and, under MATTN_PRECISE,
+// precise.hip; launch_fwd_simt and launch_bwd_simt hand them over.
 // Same maths and tile walk as the MFMA path (/root/reference/jaxmodules/
 // attention.py:52-105 forward, :266-342 backward): per 32-key (or 32-query)
 // sub-block an online softmax, P = exp2(scale_log2 S - lse) in the backward,
@@ -15,8 +13,7 @@
 // |dO| |V|) would be all that is left of their difference.
 // TPR threads share a row (query or key), each holding D / TPR head dims; a
 // workgroup of 512 threads owns 512 / TPR rows of a 128-row map tile, so a
-// tile takes 128 TPR / 512 workgroups (one for TPR = 4, two for TPR = 8 at
-// D = 256, four for TPR = 16 at D = 512).
+// tile takes 128 TPR / 512 workgroups (four for TPR = 16 at D = 512).
 #include <type_traits>
 
 #include "common.hpp"
@@ -402,11 +399,10 @@ void bwd_dkdv_simt(KArgs a) {
   }
 }
 
-// the stages of one (D, TPR, input, output) combination; without PREC only D = 512
-// comes here
-template <int D, int TPR, class IT, class OT>
+// the stages of one (input, output) combination: D = 512, 16 threads per row
+template <class IT, class OT>
 struct Simt {
-  static constexpr int SPLIT = TILE * TPR / 512;
+  static constexpr int D = 512, TPR = 16, SPLIT = TILE * TPR / 512;
   template <bool PREC>
   static void fwd(const KArgs& a, int grid, hipStream_t st) {
     hipLaunchKernelGGL((fwd_simt<D, TPR, IT, OT, PREC>), dim3(grid * SPLIT), dim3(512), 0, st, a);
@@ -421,45 +417,46 @@ struct Simt {
   }
 };
 
-// f(Simt<...>{}, precise) for the problem's combination: 4 threads per row at D = 64
-// and 128, 8 at 256, 16 at 512; float32 inputs, or 16-bit inputs with a float32 or
-// same-dtype output
+// f(Simt<...>{}, precise) for the problem's combination: float32 inputs, or 16-bit
+// inputs with a float32 or same-dtype output
 template <class IT, class OT, class F>
-void dispatch_d(int D, bool precise, F&& f) {
-  if (D == 64) f(Simt<64, 4, IT, OT>{}, std::true_type{});
-  else if (D == 128) f(Simt<128, 4, IT, OT>{}, std::true_type{});
-  else if (D == 256) f(Simt<256, 8, IT, OT>{}, std::true_type{});
-  else if (precise) f(Simt<512, 16, IT, OT>{}, std::true_type{});
-  else f(Simt<512, 16, IT, OT>{}, std::false_type{});
+void dispatch_p(bool precise, F&& f) {
+  if (precise) f(Simt<IT, OT>{}, std::true_type{});
+  else f(Simt<IT, OT>{}, std::false_type{});
 }
 template <class F>
-hipError_t dispatch(int D, int dtype, int o_dtype, bool precise, F&& f) {
+hipError_t dispatch(int dtype, int o_dtype, bool precise, F&& f) {
   const bool of32 = o_dtype == MATTN_F32;
-  if (dtype == MATTN_F32) dispatch_d<float, float>(D, precise, f);
-  else if (dtype == MATTN_BF16 && of32) dispatch_d<bf16_tag, float>(D, precise, f);
-  else if (dtype == MATTN_BF16) dispatch_d<bf16_tag, bf16_tag>(D, precise, f);
-  else if (of32) dispatch_d<f16_tag, float>(D, precise, f);
-  else dispatch_d<f16_tag, f16_tag>(D, precise, f);
+  if (dtype == MATTN_F32) dispatch_p<float, float>(precise, f);
+  else if (dtype == MATTN_BF16 && of32) dispatch_p<bf16_tag, float>(precise, f);
+  else if (dtype == MATTN_BF16) dispatch_p<bf16_tag, bf16_tag>(precise, f);
+  else if (of32) dispatch_p<f16_tag, float>(precise, f);
+  else dispatch_p<f16_tag, f16_tag>(precise, f);
   return hipGetLastError();
 }
 
 }  // namespace
 
 bool s3_path(int D, int dtype, bool precise);
+hipError_t launch_fwd_f64(const KArgs& a, int D, int dtype, int o_dtype, int grid, hipStream_t st);
+hipError_t launch_bwd_f64(const KArgs& a, int D, int dtype, int o_dtype, int stage, int q_grid, int kv_grid,
+                          hipStream_t st);
 hipError_t launch_fwd_s3(const KArgs& a, int D, int dtype, int o_dtype, int grid, hipStream_t st);
 hipError_t launch_bwd_s3(const KArgs& a, int D, int dtype, int o_dtype, int stage, int q_grid, int kv_grid,
                          hipStream_t st);
 
 hipError_t launch_fwd_simt(const KArgs& a, int D, int dtype, int o_dtype, int grid, hipStream_t st) {
   if (s3_path(D, dtype, a.precise)) return launch_fwd_s3(a, D, dtype, o_dtype, grid, st);
-  return dispatch(D, dtype, o_dtype, a.precise,
+  if (D <= 256) return launch_fwd_f64(a, D, dtype, o_dtype, grid, st);
+  return dispatch(dtype, o_dtype, a.precise,
                   [&](auto s, auto p) { decltype(s)::template fwd<decltype(p)::value>(a, grid, st); });
 }
 
 hipError_t launch_bwd_simt(const KArgs& a, int D, int dtype, int o_dtype, int stage, int q_grid, int kv_grid,
                            hipStream_t st) {
   if (s3_path(D, dtype, a.precise)) return launch_bwd_s3(a, D, dtype, o_dtype, stage, q_grid, kv_grid, st);
-  return dispatch(D, dtype, o_dtype, a.precise, [&](auto s, auto p) {
+  if (D <= 256) return launch_bwd_f64(a, D, dtype, o_dtype, stage, q_grid, kv_grid, st);
+  return dispatch(dtype, o_dtype, a.precise, [&](auto s, auto p) {
     decltype(s)::template bwd<decltype(p)::value>(a, stage, q_grid, kv_grid, st);
   });
 }

@@ -1,7 +1,7 @@
 // Masked attention at float32 accuracy on the matrix cores (split3.hpp): the
 // forward and the backward of float32 inputs at D = 64, 128 and 256 and of 16-bit
-// inputs at D = 256.  MATTN_PRECISE and D = 512 run on the SIMT kernels of
-// simt.hip, which these replaced elsewhere.  Measured against them: float32
+// inputs at D = 256 (MATTN_PRECISE: precise.hip; D = 512: the SIMT kernels of
+// simt.hip, which these replaced).  Measured against them: float32
 // causal [2, 2048, 8, 64] fwd 465 -> 87 us, dK/dV 768 -> 165, dQ 596 -> 126 (the
 // step 16.9 -> 86 TFLOP/s); bfloat16 causal [1, 4096, 8, 256] fwd 4322 -> 326 us,
 // dK/dV 14370 -> 750, dQ 4811 -> 708 (10 -> 139 TFLOP/s).  Their error against
@@ -36,10 +36,6 @@ namespace mattn {
 namespace {
 using namespace s3;
 
-__device__ __forceinline__ const char* head_base(const void* p, const int64_t* s, int b, int h, int es) {
-  return (const char*)p + es * ((int64_t)b * s[0] + (int64_t)h * s[2]);
-}
-
 // own row operands: row r of a tensor slice, k-step kd = columns c0 + 16 kd + 8 hi .. + 7
 template <class T, int N>
 __device__ __forceinline__ void own_rows(Frag<Pieces<T>::n> (&f)[N], const char* base, int64_t rs, int r, int c0, int hi) {
@@ -69,17 +65,6 @@ struct Place {
 };
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
-
-// Sub-blocks of the walk over entries [e0, e1): SPT = 128 / BN per tile.
-template <int BN>
-struct Walk {
-  static constexpr int SPT = TILE / BN;
-  const int* ent;
-  int e0, n;
-  __device__ __forceinline__ Walk(const int* ent_, int e0_, int e1_) : ent(ent_), e0(e0_), n((e1_ - e0_) * SPT) {}
-  __device__ __forceinline__ int first(int s) const { return ent[2 * (e0 + s / SPT)] * TILE + (s % SPT) * BN; }
-  __device__ __forceinline__ int mask(int s) const { return ent[2 * (e0 + s / SPT) + 1]; }
-};
 
 // the 32 mask bits of row `row` (of a tile) against the 32-row block `blk` of the other side
 __device__ __forceinline__ uint32_t bits32(const uint64_t* bits, int mask, int blk, int row) {

@@ -258,5 +258,21 @@ __device__ __forceinline__ void slab_sum_store(const float* slab, void* out, int
   }
 }
 
+// base address of (b, h) in a tensor of element strides s
+__device__ __forceinline__ const char* head_base(const void* p, const int64_t* s, int b, int h, int es) {
+  return (const char*)p + es * ((int64_t)b * s[0] + (int64_t)h * s[2]);
+}
+
+// Sub-blocks of the walk over entries [e0, e1): SPT = 128 / BN per tile.
+template <int BN>
+struct Walk {
+  static constexpr int SPT = TILE / BN;
+  const int* ent;
+  int e0, n;
+  __device__ __forceinline__ Walk(const int* ent_, int e0_, int e1_) : ent(ent_), e0(e0_), n((e1_ - e0_) * SPT) {}
+  __device__ __forceinline__ int first(int s) const { return ent[2 * (e0 + s / SPT)] * TILE + (s % SPT) * BN; }
+  __device__ __forceinline__ int mask(int s) const { return ent[2 * (e0 + s / SPT) + 1]; }
+};
+
 }  // namespace s3
 }  // namespace mattn
