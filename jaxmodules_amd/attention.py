@@ -31,6 +31,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import struct
 from collections import OrderedDict
 from typing import Callable, Optional, Tuple
 
@@ -231,9 +232,19 @@ def _mask_key(mask_fn):
     """Cache key of a mask function: by content when every value it reads is
     one _freeze can describe -- so a new but identical lambda per call (the
     usual way to pass a mask) finds the map already traced -- and the function
-    object itself otherwise."""
+    object itself otherwise.  A closed-form mask (jaxmodules_amd.masks) without
+    arrays is its few numbers, so that the mask the residue rewrite makes anew
+    on every call is not classified again each time (1.1 ms of the strided
+    [1, 131072, 1, 64] step, whose kernels take 0.16); one with document ids or
+    a tile table is the function object (hashing the arrays on every call would
+    cost more than it saves)."""
     import types
 
+    spec = bmap.spec_of(mask_fn)
+    if spec is not None:
+        if spec.doc_q is not None or spec.table is not None:
+            return mask_fn
+        return ("spec", spec.causal, spec.win_left, spec.win_right, spec.period)
     if isinstance(mask_fn, types.FunctionType):
         try:
             return ("content", _fn_content(mask_fn))
@@ -288,7 +299,7 @@ def _check_map(tm: bmap.TileMap, q, k):
 
 def device_blockmap(tm: bmap.TileMap, device) -> _lib.MattnBlockmap:
     """Uploads the tile map once per device and returns the C struct pointing at it."""
-    key = str(torch.device(device))
+    key = device if isinstance(device, torch.device) else torch.device(device)
     hit = tm.device.get(key)
     if hit is not None:
         return hit[1]
@@ -323,33 +334,29 @@ def device_blockmap(tm: bmap.TileMap, device) -> _lib.MattnBlockmap:
 _DT = {torch.bfloat16: _lib.MATTN_BF16, torch.float16: _lib.MATTN_F16, torch.float32: _lib.MATTN_F32}
 
 
-def _strides(t: torch.Tensor):
-    s = t.stride()
-    return (ctypes.c_int64 * 3)(s[0], s[1], s[2])
-
-
 def _ready(t: torch.Tensor) -> torch.Tensor:
     """d contiguous and 16-byte aligned strides/base, as the kernels' vector loads need."""
-    es = t.element_size()
-    ok = t.stride(-1) == 1 and all((s * es) % 16 == 0 for s in t.stride()[:3]) \
-        and t.data_ptr() % 16 == 0
+    s0, s1, s2, s3 = t.stride()
+    ok = s3 == 1 and ((s0 | s1 | s2) * t.element_size()) % 16 == 0 and t.data_ptr() % 16 == 0
     return t if ok else t.contiguous()
+
+
+# mattn_problem as one record: 8 sizes and types, scale, flags, 8 x 3 strides
+_PROBLEM = struct.Struct("=8ifi24q")
+assert _PROBLEM.size == ctypes.sizeof(_lib.MattnProblem)
 
 
 def _problem(q, k, v, o, scale, do=None, dq=None, dk=None, dv=None):
     B, N, Hq, d = q.shape
-    p = _lib.MattnProblem(B=B, Lq=N, Lk=k.shape[1], Hq=Hq, Hkv=k.shape[2], D=d,
-                          dtype=_DT[q.dtype], o_dtype=_DT[o.dtype], scale=scale)
-    p.q_stride, p.k_stride, p.v_stride, p.o_stride = _strides(q), _strides(k), _strides(v), _strides(o)
-    p.do_stride = _strides(do if do is not None else o)
-    p.dq_stride = _strides(dq if dq is not None else q)
-    p.dk_stride = _strides(dk if dk is not None else k)
-    p.dv_stride = _strides(dv if dv is not None else v)
-    return p
+    sq, sk, sv, so = q.stride()[:3], k.stride()[:3], v.stride()[:3], o.stride()[:3]
+    return _lib.MattnProblem.from_buffer_copy(_PROBLEM.pack(
+        B, N, k.shape[1], Hq, k.shape[2], d, _DT[q.dtype], _DT[o.dtype], scale, 0, *sq, *sk, *sv, *so,
+        *(so if do is None else do.stride()[:3]), *(sq if dq is None else dq.stride()[:3]),
+        *(sk if dk is None else dk.stride()[:3]), *(sv if dv is None else dv.stride()[:3])))
 
 
 def _stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def mattn_forward(q, k, v, tm: bmap.TileMap, scale: float, out_dtype=torch.float32,
@@ -374,9 +381,9 @@ def mattn_forward(q, k, v, tm: bmap.TileMap, scale: float, out_dtype=torch.float
     p = _problem(q, k, v, o, scale)
     p.flags = (_lib.MATTN_FWD_FOR_BWD if for_backward else 0) | (_lib.MATTN_PRECISE if precise else 0)
     bm = device_blockmap(tm, q.device)
-    nws = int(lib.mattn_fwd_workspace_bytes(ctypes.byref(p)))
-    res, rptr = _workspace(nws, q.device)
-    _lib.check(lib.mattn_fwd(ctypes.byref(p), ctypes.byref(bm), q.data_ptr(), k.data_ptr(),
+    pr = ctypes.byref(p)
+    res, rptr = _workspace(lib.mattn_fwd_workspace_bytes(pr), q.device)
+    _lib.check(lib.mattn_fwd(pr, ctypes.byref(bm), q.data_ptr(), k.data_ptr(),
                              v.data_ptr(), o.data_ptr(), lse.data_ptr(), rptr, _stream(q.device)),
                "mattn_fwd")
     return o, lse, res
@@ -439,11 +446,12 @@ def mattn_backward(q, k, v, o, lse, do, tm: bmap.TileMap, scale: float, res=None
     p.flags = _lib.MATTN_FWD_FOR_BWD | (_lib.MATTN_PRECISE if precise else 0)
     bm = device_blockmap(tm, q.device)
     p.flags = bwd_flags(p, bm)
-    nws = int(lib.mattn_bwd_workspace_bytes(ctypes.byref(p), ctypes.byref(bm)))
+    pr, br = ctypes.byref(p), ctypes.byref(bm)
+    nws = lib.mattn_bwd_workspace_bytes(pr, br)
     if nws == 0:
-        _lib.check(lib.mattn_validate(ctypes.byref(p), ctypes.byref(bm)), "mattn_bwd")
+        _lib.check(lib.mattn_validate(pr, br), "mattn_bwd")
     ws, wptr = _workspace(max(nws, 256), q.device)
-    _lib.check(lib.mattn_bwd(ctypes.byref(p), ctypes.byref(bm), q.data_ptr(), k.data_ptr(),
+    _lib.check(lib.mattn_bwd(pr, br, q.data_ptr(), k.data_ptr(),
                              v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr(), _aligned(res),
                              wptr, max(nws, 256), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                              _stream(q.device)),
@@ -456,8 +464,10 @@ class _MaskedAttention(torch.autograd.Function):
     (Q, K, V, O, LSE) instead of (Q, K, V): the backward reads the saved
     log-sum-exp rather than re-running the forward scan.
 
-    O is always computed and saved in float32 (the reference's own output
-    dtype); a 16-bit ``out_dtype`` is a rounded copy of it.  The backward's
+    Where a gradient is needed O is computed and saved in float32 (the
+    reference's own output dtype) and a 16-bit ``out_dtype`` is a rounded copy of
+    it; otherwise the kernels round it themselves (the same values: 57 us of a
+    670 us bfloat16 forward at B=4 L=4096 Hq=32 d=128 was the copy).  The backward's
     delta = rowsum(dO * O) then uses the unrounded O: where one key dominates
     a row, dS = P (dP - delta) cancels, and a bfloat16 O would leave its
     rounding (2^-9 of |V|) in dQ and dK."""
@@ -465,8 +475,10 @@ class _MaskedAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, tm, scale, out_dtype, heads_major=False, precise=False):
         grads = any(ctx.needs_input_grad[:3])
-        o, lse, res = mattn_forward(q, k, v, tm, scale, torch.float32, heads_major, for_backward=grads,
-                                    precise=precise)
+        o, lse, res = mattn_forward(q, k, v, tm, scale, torch.float32 if grads else out_dtype, heads_major,
+                                    for_backward=grads, precise=precise)
+        if not grads:
+            return o
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.tm, ctx.scale, ctx.res, ctx.precise = tm, scale, res, precise
         return o if out_dtype == torch.float32 else o.to(out_dtype)
@@ -474,7 +486,7 @@ class _MaskedAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
-        do = _ready(do.to(o.dtype))
+        do = _ready(do if do.dtype == o.dtype else do.to(o.dtype))
         dq, dk, dv = mattn_backward(q, k, v, o, lse, do, ctx.tm, ctx.scale, ctx.res, ctx.precise)
         return dq, dk, dv, None, None, None, None, None
 
@@ -589,7 +601,7 @@ def _residue_rewrite(Q, K, V, is_causal, kernel_fn, mask_fn, block_size, window_
 
 def residue_view(x: torch.Tensor, P: int) -> torch.Tensor:
     """[1, L, H, d] -> the [P, L / P, H, d] view whose [r, s] is position s P + r."""
-    return x[0].reshape(x.shape[1] // P, P, x.shape[2], x.shape[3]).transpose(0, 1)
+    return x.reshape(x.shape[1] // P, P, x.shape[2], x.shape[3]).transpose(0, 1)  # (x[0]'s gradient would be a copy)
 
 
 def residue_unview(y: torch.Tensor) -> torch.Tensor:
@@ -654,25 +666,38 @@ def _via_map(Q, K, V, *, is_causal=False, kernel_fn=default_kernel, mask_fn=None
     scale = kernel_scale(kernel_fn, plan.d)
     if not (Q.is_cuda and K.is_cuda and V.is_cuda):
         raise RuntimeError("masked_attention_via_map runs on the GPU only (no CPU code path)")
-    dt = torch.promote_types(torch.promote_types(Q.dtype, K.dtype), V.dtype)
-    if dt not in _DT:
-        raise TypeError(f"unsupported dtype {dt}")
+    dt = _common_dtype(Q, K, V)
     if plan.squeeze_batch:
         Q, K, V = Q[None], K[None], V[None]
     D = _kernel_dim(plan.d)
-    Q = Q.to(dt)
     # softmax(s q.k) == softmax(|s| (-q).k); s == 0 gives uniform weights: q = 0, scale 1
     if scale < 0:
-        Q, scale = -Q, -scale
+        Q, scale = -Q.to(dt), -scale
     elif scale == 0:
-        Q, scale = Q * 0, 1.0
+        Q, scale = Q.to(dt) * 0, 1.0
     precise = use_precise(precision, scale, plan.d)
-    q, k, v = (_ready(_pad_dim(x.to(dt), D)) for x in (Q, K, V))
+    q, k, v = _operand(Q, dt, D), _operand(K, dt, D), _operand(V, dt, D)
     od = _out_dtype(dt, out_dtype)
     out = _MaskedAttention.apply(q, k, v, tm, scale, od, False, precise)
     if D != plan.d:
         out = out[..., :plan.d]
     return out[0] if plan.squeeze_batch else out
+
+
+def _common_dtype(q, k, v):
+    dt = q.dtype
+    if k.dtype != dt or v.dtype != dt:
+        dt = torch.promote_types(torch.promote_types(dt, k.dtype), v.dtype)
+    if dt not in _DT:
+        raise TypeError(f"unsupported dtype {dt}")
+    return dt
+
+
+def _operand(x, dt, D):
+    """x [B, L, H, d] in dtype dt, padded to D columns, as the kernels can load it."""
+    if x.dtype != dt:
+        x = x.to(dt)
+    return _ready(_pad_dim(x, D))
 
 
 def _out_dtype(dt, out_dtype):
@@ -759,23 +784,20 @@ def flex_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         raise NotImplementedError("value head dimension must equal the query/key head dimension")
     if not (query.is_cuda and key.is_cuda and value.is_cuda):
         raise RuntimeError("flex_attention runs on the GPU only (no CPU code path)")
-    dt = torch.promote_types(torch.promote_types(query.dtype, key.dtype), value.dtype)
-    if dt not in _DT:
-        raise TypeError(f"unsupported dtype {dt}")
+    dt = _common_dtype(query, key, value)
     s = 1.0 / math.sqrt(E) if scale is None else float(scale)
     if not math.isfinite(s):
         raise ValueError(f"scale must be finite, got {s}")
     precise = use_precise(precision, s, E)
     tm = _block_mask_tiles(block_mask, B, Hq, Hkv, L, S, _element_head)
     D = _kernel_dim(E)
-    q = query.to(dt)
     # softmax(s q.k) == softmax(|s| (-q).k); s == 0 gives uniform weights: q = 0, scale 1
     if s < 0:
-        q, s = -q, -s
+        query, s = -query.to(dt), -s
     elif s == 0:
-        q, s = q * 0, 1.0
+        query, s = query.to(dt) * 0, 1.0
     # [B, H, L, E] tensors are strided [B, L, H, E] views for the kernels
-    q, k, v = (_ready(_pad_dim(x, D).transpose(1, 2)) for x in (q, key.to(dt), value.to(dt)))
+    q, k, v = (_ready(_pad_dim(x if x.dtype == dt else x.to(dt), D).transpose(1, 2)) for x in (query, key, value))
     out = _MaskedAttention.apply(q, k, v, tm, s, _out_dtype(dt, out_dtype), True, precise)
     out = out.transpose(1, 2)
     return out[..., :E] if D != E else out

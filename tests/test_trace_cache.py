@@ -120,3 +120,19 @@ def test_numpy_functions_keep_content_keys():
     A.clear_cache()
     maps = [_call(lambda h, q, k: np.where(np.abs(q - k) < 30, True, np.int32(k) <= q)) for _ in range(2)]
     assert maps[0] is maps[1]
+
+
+def test_closed_form_masks_without_arrays_are_keyed_by_value():
+    """masks.* functions made anew per call share a key when their numbers agree
+    (the residue rewrite makes its inner mask on every call); those holding
+    arrays are keyed by the function itself."""
+    import numpy as np
+
+    from jaxmodules_amd import masks
+
+    make = lambda p: masks.intersect(masks.same_residue(p), masks.causal())  # noqa: E731
+    assert A._mask_key(make(4)) == A._mask_key(make(4)) != A._mask_key(make(8))
+    assert A._mask_key(masks.window(3, 0)) != A._mask_key(masks.window(3, 1)) != A._mask_key(masks.window(None, 1))
+    assert A._mask_key(masks.causal()) != A._mask_key(masks.same_residue(2))
+    doc = masks.documents(np.arange(8))
+    assert A._mask_key(doc) is doc
