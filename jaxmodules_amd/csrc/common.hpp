@@ -94,6 +94,7 @@ struct KArgs {
   uint16_t* ds;
   const int* col_row;
   int ds_nnz;
+  int n_slots;         // slots of the launch order the kernel walks (kernels that cut a slot into parts)
   const int* kv_desc;  // per dK/dV launch slot: { item, g, e, e_end, n_sub, qt, mask, row }
   int precise;         // MATTN_PRECISE: float64 (D = 512: compensated) scores and sums
   float* lse_lo;       // MATTN_PRECISE (forward residual): [B, Hq, Lq], (m + log2 l) - lse

@@ -39,6 +39,19 @@ __device__ __forceinline__ f64x4 mfma64(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// Sub-blocks of the walk over entries [e0, e1), SPT per tile.  The entry is read at each
+// step: a step has thousands of cycles of matrix work (held in lanes, as split3.hpp's
+// Walk does, the step ran 1.3% slower).
+template <int BN>
+struct Steps {
+  static constexpr int SPT = TILE / BN;
+  const int* ent;
+  int e0, n;
+  __device__ __forceinline__ Steps(const int* ent_, int e0_, int e1_) : ent(ent_), e0(e0_), n((e1_ - e0_) * SPT) {}
+  __device__ __forceinline__ int first(int s) const { return ent[2 * (e0 + s / SPT)] * TILE + (s % SPT) * BN; }
+  __device__ __forceinline__ int mask(int s) const { return ent[2 * (e0 + s / SPT) + 1]; }
+};
+
 // N consecutive elements (N = 4 or 8) as floats
 template <class T, int N>
 __device__ __forceinline__ void get(const char* p, float* x) {
@@ -168,7 +181,7 @@ void fwd_f64(KArgs a) {
   const int qt = item % a.nqt, bh = item / a.nqt;
   const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.G;
   const int mrow = map_row(a, b, h, a.nqt, qt);
-  const Walk<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
+  const Steps<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
   const int wrow = (blockIdx.x % NSUB) * 16 * WQ;
   if (qt * TILE + wrow >= a.Lq) return;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
@@ -196,7 +209,7 @@ void fwd_f64(KArgs a) {
     bool any = false;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      w[t] = mask >= 0 ? bits16(a.row_bits, mask, (s % Walk<BN>::SPT) * (BN / 16) + wk * NT + t, qloc) : 0xffffu;
+      w[t] = mask >= 0 ? bits16(a.row_bits, mask, (s % Steps<BN>::SPT) * (BN / 16) + wk * NT + t, qloc) : 0xffffu;
       any |= w[t] != 0;
     }
     if (!__any(any)) continue;
@@ -280,7 +293,7 @@ void bwd_dq_f64(KArgs a) {
   const int qt = item % a.nqt, bh = item / a.nqt;
   const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.G;
   const int mrow = map_row(a, b, h, a.nqt, qt);
-  const Walk<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
+  const Steps<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
   const int wrow = (blockIdx.x % NSUB) * 16 * WQ;
   if (qt * TILE + wrow >= a.Lq) return;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
@@ -321,7 +334,7 @@ void bwd_dq_f64(KArgs a) {
     for (int t = 0; t < NT; ++t) {
       const int r0 = 16 * (wk * NT + t);
       const uint32_t w =
-          mask >= 0 ? bits16(a.row_bits, mask, (s % Walk<BN>::SPT) * (BN / 16) + wk * NT + t, qloc) : 0xffffu;
+          mask >= 0 ? bits16(a.row_bits, mask, (s % Steps<BN>::SPT) * (BN / 16) + wk * NT + t, qloc) : 0xffffu;
       if (!__any(w != 0)) continue;
       const f64x4 st = dot_rows<D>(Kl + (r0 + l16) * ld<D>(), qv, g, f64x4{});
       const f64x4 dp = dot_rows<D>(Vl + (r0 + l16) * ld<D>(), gv, g, f64x4{});
@@ -373,7 +386,7 @@ void bwd_dkdv_f64(KArgs a) {
   for (int gh = 0; gh < a.G; ++gh) {
     const int h = hk * a.G + gh;
     const int mc = map_row(a, b, h, a.nkt, kt);
-    const Walk<BN> walk(a.col_ent, a.col_ptr[mc], a.col_ptr[mc + 1]);
+    const Steps<BN> walk(a.col_ent, a.col_ptr[mc], a.col_ptr[mc + 1]);
     const char* qb = head_base(a.q, a.qs, b, h, elt_bytes<IT>());
     const char* gb = head_base(a.dO, a.dos, b, h, elt_bytes<OT>());
     const char* ob = head_base(a.o, a.os, b, h, elt_bytes<OT>());
@@ -408,7 +421,7 @@ void bwd_dkdv_f64(KArgs a) {
       for (int t = 0; t < NT; ++t) {
         const int r0 = 16 * (wk * NT + t);
         const uint32_t w =
-            mask >= 0 ? bits16(a.col_bits, mask, (s % Walk<BN>::SPT) * (BN / 16) + wk * NT + t, kloc) : 0xffffu;
+            mask >= 0 ? bits16(a.col_bits, mask, (s % Steps<BN>::SPT) * (BN / 16) + wk * NT + t, kloc) : 0xffffu;
         if (!__any(w != 0)) continue;
         const f64x4 st = dot_rows<D>(Ql + (r0 + l16) * ld<D>(), kv, g, f64x4{});
         const f64x4 dp = dot_rows<D>(Gl + (r0 + l16) * ld<D>(), vv, g, f64x4{});

@@ -1,33 +1,38 @@
 // Masked attention at float32 accuracy on the matrix cores (split3.hpp): the
 // forward and the backward of float32 inputs at D = 64, 128 and 256 and of 16-bit
 // inputs at D = 256 (MATTN_PRECISE: precise.hip; D = 512: the SIMT kernels of
-// simt.hip, which these replaced).  Measured against them: float32
-// causal [2, 2048, 8, 64] fwd 465 -> 87 us, dK/dV 768 -> 165, dQ 596 -> 126 (the
-// step 16.9 -> 86 TFLOP/s); bfloat16 causal [1, 4096, 8, 256] fwd 4322 -> 326 us,
-// dK/dV 14370 -> 750, dQ 4811 -> 708 (10 -> 139 TFLOP/s).  Their error against
-// float64 is no larger (float32 step: 6.6e-7 of the norm, 1.1e-6 before).
-// Bound by the matrix cores and the split's VALU work together: a 32 x 32 block
-// of the float32 forward at D = 64 takes 48 MFMAs (1536 cycles) and about 300
-// vector instructions.
+// simt.hip, which these replaced).
 //
 // Same maths and tile walk as there (/root/reference/jaxmodules/
-// attention.py:52-105 forward, :266-342 backward).  Every wave owns 32 rows
-// (queries in the forward and dQ, keys in dK/dV), one per lane pair, and walks
-// the present tiles of its map row or column, sub-block by sub-block:
+// attention.py:52-105 forward, :266-342 backward).  Every wave owns 16 rows (queries in
+// the forward and dQ, keys in dK/dV; lane l % 16 = row) and walks the present tiles of
+// its map row or column 32 rows of the other side at a time:
 //   forward  S^T = K Q^T, online softmax, O^T += V^T P^T
 //   dQ       S^T = K Q^T, dP^T = V dO^T, dS = P (dP - delta), dQ^T += K^T dS^T
 //   dK/dV    S = Q K^T, dP = dO V^T, dV^T += dO^T P, dK^T += Q^T dS
-// The streamed tensors are read once per workgroup, split into bfloat16 pieces
-// on the way to LDS (the next sub-block's rows are in registers meanwhile);
-// the wave's own rows are split in registers.  P and dS are split from the
-// C registers, which are the B operand of the next product as they stand.
+// The streamed rows are read once per workgroup and split into bfloat16 pieces on the
+// way to LDS (bfloat16 rows go there directly); the wave's own rows are split in
+// registers.  P and dS are split from the C registers, which are the B operand of the
+// next product as they stand.
 //
-// A workgroup is WQ x WK x DS waves: WQ groups of 32 own rows; WK waves per group
-// that take every WK-th 32-row block of a sub-block and sum their results through
-// LDS at the end; and DS = 2 waves that each hold one half of the columns (of the
-// own rows' operands and of the result), form S and dP over that half and add the
-// partner's through LDS, so that a wave's operands and accumulators fit half the
-// registers and two waves share a SIMD.
+// Why 16 rows (v_mfma_f32_16x16x32_bf16): at D = 256 a wave of 32 rows holds its
+// operands and results only by sharing them with a partner wave (each half of the
+// columns, S and dP summed through LDS with a barrier, the softmax done by both) or by
+// spilling; for float32 at D = 64 its dK/dV spilled at two waves a SIMD.  The price is
+// LDS: a streamed operand is read per 16 rows, 125 bytes a clock and CU at the matrix
+// cores' full rate.
+// Measured, causal steps: float32 [2, 2048, 8, 64] fwd 465 -> 97 us, dK/dV 768 -> 144,
+// dQ 596 -> 113 against the SIMT kernels; bfloat16 [1, 4096, 8, 256] fwd 4322 -> 192 us,
+// dK/dV 14370 -> 579, dQ 4811 -> 248 (32-row waves sharing columns: 326, 750, 708).
+// The error against float64 is no larger than theirs (float32 step: 8.4e-7 of the norm,
+// 1.1e-6 before).  float32 at D = 64 is bound by vector instructions (260 a step and
+// wave against 48 MFMAs of 16 cycles; half of them split the streamed rows).
+//
+// MFMA 16x16x32 layout (lane l, l16 = l % 16, g = l / 16): A row l16, k = 8 g .. 8 g + 7;
+// B column l16, the same k; C column l16, register r row 4 g + r.  The two 16-row
+// blocks t of a 32-row step leave lane (l16, g) with rows 16 t + 4 g + r, taken as the
+// 8 values of the next product's B operand; its A operand (transposed reads) holds the
+// same rows in the same places.
 #include <type_traits>
 
 #include "split3.hpp"
@@ -36,221 +41,511 @@ namespace mattn {
 namespace {
 using namespace s3;
 
-// own row operands: row r of a tensor slice, k-step kd = columns c0 + 16 kd + 8 hi .. + 7
-template <class T, int N>
-__device__ __forceinline__ void own_rows(Frag<Pieces<T>::n> (&f)[N], const char* base, int64_t rs, int r, int c0, int hi) {
+// the two blocks' C registers as a B operand over the 32 rows
+__device__ __forceinline__ Frag<3> c_frag16(const f32x4& c0, const f32x4& c1) {
+  Frag<3> f;
 #pragma unroll
-  for (int kd = 0; kd < N; ++kd) {
+  for (int e = 0; e < 4; ++e) {
+    uint32_t w[3];
+    if (e < 2) split2<3>(c0[2 * e], c0[2 * e + 1], w);
+    else split2<3>(c1[2 * e - 4], c1[2 * e - 3], w);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) f.p[p][e] = w[p];
+  }
+  return f;
+}
+
+constexpr int BN = 32;  // streamed rows a step
+
+// LDS tile of one piece: 16-byte chunk c of row r at c ^ sw(r).  A row read takes one
+// chunk of 16 rows, a transposed read (32 lanes) one chunk pair of 8 aligned rows: both
+// hit 16 (8 pairs of) distinct 16-byte bank groups.  (A row of D = 64 is half the 64
+// banks: its parity is the fourth bit.)
+template <int D>
+__device__ __forceinline__ int sw(int r) {
+  if constexpr (D == 64) return (((r >> 1) & 3) << 1) | ((r >> 3) & 1);
+  else return ((r & 7) << 1) | ((r >> 3) & 1);
+}
+
+// BN rows of a tensor to LDS as planes of pieces.  bfloat16 rows (one piece, as they are)
+// go straight to LDS (DMA); others through registers and split.
+template <int D, class T, int NTH, bool WIDE = false>
+struct Rows {
+  static constexpr int NP = Pieces<T>::n, CPR = D / 8, ELTS = NP * BN * D;
+  static constexpr int CH = BN * CPR / NTH;
+  static constexpr bool DMA = NP == 1;
+  Raw8<T> v[DMA ? 1 : CH];
+  // registers, or (DMA) LDS `dst`; rows past n - 1 re-read row n - 1 (masked)
+  __device__ __forceinline__ void load(const char* base, int64_t rs, int r0, int n, uint16_t* dst) {
+    each_chunk<D, elt_bytes<T>(), BN, NTH, WIDE>(base, rs, r0, n, [&](int c, const char* p, uint32_t off) {
+      const int i = threadIdx.x + NTH * c, r = i / CPR, col = i % CPR;
+      if constexpr (DMA) {
+        const int blk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + c * (NTH / 64);
+        lds_load16(p + (off + 16 * (col ^ sw<D>(r))), dst + blk * 512);  // lane l of block blk: chunk 64 blk + l
+      } else {
+        v[c].load(p + (off + elt_bytes<T>() * 8 * col));
+      }
+    });
+  }
+  __device__ __forceinline__ void store(uint16_t* dst) const {
+    if constexpr (!DMA) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const int i = threadIdx.x + NTH * c, r = i / CPR, col = i % CPR;
+        const Frag<NP> f = v[c].split();
+#pragma unroll
+        for (int p = 0; p < NP; ++p) *(u32x4*)(dst + p * BN * D + r * D + ((col ^ sw<D>(r)) << 3)) = f.p[p];
+      }
+    }
+  }
+};
+
+// LDS byte addresses of the operand reads of a tile at `base` (512-byte aligned): the
+// chunk index is XORed with bits of the row alone, so column steps are XORs too
+//   along d:       rows 16 t + l16, columns 32 kd + 8 g ..: row_addr ^ (64 kd), offset 16 t rows
+//   along the rows: columns 16 mt .., k slot 4 t + j = row 16 t + 4 g + j: tr_addr ^ (32 mt), offset 16 t rows
+template <int D>
+__device__ __forceinline__ uint32_t row_addr(int l16, int g) {
+  return 2 * l16 * D + ((g ^ sw<D>(l16)) << 4);
+}
+template <int D>
+__device__ __forceinline__ uint32_t tr_addr(int l16, int g) {
+  const int r = 4 * g + (l16 >> 2);
+  return 2 * r * D + ((((l16 & 3) >> 1) ^ sw<D>(r)) << 4) + 8 * (l16 & 1);
+}
+
+// S += A X and dP += A2 X2 along d for both 16-row blocks: tiles at byte addresses ra, rb
+template <int WANT, int D, int NA, int NX, int NB, int NY>
+__device__ __forceinline__ void two_dots(uint32_t ra, uint32_t rb, const Frag<NX> (&x)[D / 32], const Frag<NY> (&y)[D / 32],
+                                         f32x4 (&st)[2], f32x4 (&dp)[2]) {
+  constexpr int PF = ahead(WANT, NA + NB), PL = 2 * BN * D;
+  Frag<NA> fa[PF + 1];
+  Frag<NB> fb[PF + 1];
+  pipe<2 * (D / 32), PF, NA + NB>(
+      [&](auto ic, auto sc) {
+        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value, kd = i / 2, t = i % 2;
+        rd<32 * t * D, PL>(fa[sl], ra ^ (uint32_t)(64 * kd));
+        rd<32 * t * D, PL>(fb[sl], rb ^ (uint32_t)(64 * kd));
+      },
+      [&](auto ic, auto sc) {
+        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value, kd = i / 2, t = i % 2;
+        landed(fa[sl]);
+        landed(fb[sl]);
+        mma_two(fa[sl], x[kd], st[t], fb[sl], y[kd], dp[t]);
+      });
+}
+template <int D, int NA, int NX>
+__device__ __forceinline__ void one_dot(uint32_t ra, const Frag<NX> (&x)[D / 32], f32x4 (&st)[2]) {
+  constexpr int PF = ahead(2, 2 * NA), PL = 2 * BN * D;
+  Frag<NA> f0[PF + 1], f1[PF + 1];
+  pipe<D / 32, PF, 2 * NA>(
+      [&](auto ic, auto sc) {
+        constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
+        rd<0, PL>(f0[sl], ra ^ (uint32_t)(64 * kd));
+        rd<32 * D, PL>(f1[sl], ra ^ (uint32_t)(64 * kd));
+      },
+      [&](auto ic, auto sc) {
+        constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
+        landed(f0[sl]);
+        landed(f1[sl]);
+        mma_two(f0[sl], x[kd], st[0], f1[sl], x[kd], st[1]);
+      });
+}
+// acc[mt] += (tile at byte address ta)^T w, the 32 rows of the tile against w
+template <int D, int NA, int WANT = 2>
+__device__ __forceinline__ void add_rows(uint32_t ta, const Frag<3>& w, f32x4 (&acc)[D / 16]) {
+  constexpr int PF = ahead(WANT, 4 * NA), PL = 2 * BN * D;
+  Tr<NA> f0[PF + 1], f1[PF + 1];
+  pipe<D / 32, PF, 4 * NA>(
+      [&](auto ic, auto sc) {
+        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value;
+        static_for<NA>([&](auto pc) {
+          constexpr int p = decltype(pc)::value;
+          f0[sl].lo[p] = ds_read_tr8<p * PL>(ta ^ (uint32_t)(64 * i));
+          f0[sl].up[p] = ds_read_tr8<p * PL + 32 * D>(ta ^ (uint32_t)(64 * i));
+          f1[sl].lo[p] = ds_read_tr8<p * PL>(ta ^ (uint32_t)(64 * i + 32));
+          f1[sl].up[p] = ds_read_tr8<p * PL + 32 * D>(ta ^ (uint32_t)(64 * i + 32));
+        });
+      },
+      [&](auto ic, auto sc) {
+        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value;
+        const Frag<NA> a0 = landed(f0[sl]), a1 = landed(f1[sl]);
+        mma_two(a0, w, acc[2 * i], a1, w, acc[2 * i + 1]);
+      });
+}
+// B operand of the wave's own rows: row r of a tensor slice, columns 32 kd + 8 g .. + 7
+template <int D, class T>
+__device__ __forceinline__ void own16(Frag<Pieces<T>::n> (&f)[D / 32], const char* base, int64_t rs, int r, int g) {
+#pragma unroll
+  for (int kd = 0; kd < D / 32; ++kd) {
     Raw8<T> x;
-    x.load(base + elt_bytes<T>() * ((int64_t)r * rs + c0 + 16 * kd + 8 * hi));
+    x.load(base + elt_bytes<T>() * ((int64_t)r * rs + 32 * kd + 8 * g));
     f[kd] = x.split();
   }
 }
 
-// Place of this wave in its workgroup
-template <int WQ, int WK, int DS>
-struct Place {
-  static constexpr int NTH = 64 * WQ * WK * DS, NSUB = TILE / (32 * WQ);  // workgroups per 128-row tile
-  int lane, l32, hi, wave, wq, wk, ds;
-  __device__ __forceinline__ Place() {
-    lane = threadIdx.x & 63;
-    l32 = lane & 31;
-    hi = lane >> 5;
-    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    wq = wave % WQ;
-    wk = wave / WQ % WK;
-    ds = wave / (WQ * WK);
+// The wave's 16 rows (lane l16 = row, acc[mt][r] = column 16 mt + 4 g + r) times sc to a
+// tensor, through LDS (16 x D float32 a wave) so that rows are stored whole.
+template <int D, class T>
+__device__ __forceinline__ void put16(const f32x4 (&acc)[D / 16], float sc, float* L, void* out, int64_t row0,
+                                      int64_t rstride, int nrows, int lane) {
+  using P = Elt<typename std::conditional<std::is_same<T, float>::value, bf16_tag, T>::type>;
+  const int l16 = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int mt = 0; mt < D / 16; ++mt)
+    *(f32x4*)(L + l16 * D + (((4 * mt + g) ^ l16) << 2)) = acc[mt] * sc;
+#pragma unroll
+  for (int i = 0; i < 16 * D / 8 / 64; ++i) {
+    const int n = 64 * i + lane, row = n / (D / 8), c = 2 * (n % (D / 8));
+    const f32x4 x = *(const f32x4*)(L + row * D + ((c ^ row) << 2));
+    const f32x4 y = *(const f32x4*)(L + row * D + (((c + 1) ^ row) << 2));
+    if (row < nrows) {
+      char* dst = (char*)out + elt_bytes<T>() * (row0 + (int64_t)row * rstride + 4 * c);
+      if constexpr (std::is_same<T, float>::value) {
+        __builtin_nontemporal_store(x, (f32x4*)dst);
+        __builtin_nontemporal_store(y, (f32x4*)dst + 1);
+      } else {
+        __builtin_nontemporal_store(u32x4{P::pack2(x[0], x[1]), P::pack2(x[2], x[3]), P::pack2(y[0], y[1]),
+                                          P::pack2(y[2], y[3])}, (u32x4*)dst);
+      }
+    }
   }
-  __device__ __forceinline__ int partner() const { return wave ^ (WQ * WK); }  // DS = 2: the other half
-};
+}
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-// the 32 mask bits of row `row` (of a tile) against the 32-row block `blk` of the other side
-__device__ __forceinline__ uint32_t bits32(const uint64_t* bits, int mask, int blk, int row) {
-  return (uint32_t)(bits[((int64_t)mask * 2 + (blk >> 1)) * TILE + row] >> (32 * (blk & 1)));
+// the 32 mask bits of row `row` (of a tile) against the 32-row block `blk` of the other
+// side, shifted so that bit 16 t + r is the one of C register r of block t
+__device__ __forceinline__ uint32_t bits32(const uint64_t* bits, int mask, int blk, int row, int g) {
+  return (uint32_t)(bits[((int64_t)mask * 2 + (blk >> 1)) * TILE + row] >> (32 * (blk & 1))) >> (4 * g);
+}
+__device__ __forceinline__ uint32_t ones16(uint32_t w, int t, int r) {
+  uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)w, 16 * t + r, 1);
+  asm("" : "+v"(m));
+  return m;
 }
 
-// The walk over n sub-blocks: with one LDS buffer a sub-block is staged between two
-// barriers, with two it is staged while the one before it is computed.
-template <int NBUF, class S, class C>
-__device__ __forceinline__ void run_walk(int n, S&& stage, C&& compute) {
-  if constexpr (NBUF == 2) {
-    if (n > 0) stage(0);
-    for (int s = 0; s < n; ++s) {
-      __syncthreads();
-      if (s + 1 < n) stage(s + 1);
-      compute(s);
-    }
-  } else {
-    for (int s = 0; s < n; ++s) {
-      __syncthreads();
-      stage(s);
-      __syncthreads();
-      compute(s);
-    }
+// max of x over lanes l and l ^ 16 (no LDS access)
+__device__ __forceinline__ float wave_max16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// P = 0 where the mask bit is clear
+__device__ __forceinline__ void zero16(f32x4 (&p)[2], uint32_t w) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[t][r] = mask_zero(p[t][r], ones16(w, t, r));
+}
+
+// One walk: the streamed rows of step s are in LDS buffer s % NBUF when compute(s) runs.
+// start(s, buf) issues their loads, finish(buf) writes what went through registers.
+template <int NBUF, bool DMA, int BUF, class S, class F, class C>
+__device__ __forceinline__ void walk_rows(int n, uint16_t* L, S&& start, F&& finish, C&& compute) {
+  static_assert(!DMA || NBUF == 2, "");
+  if (n > 0) start(0, L);
+  for (int s = 0; s < n; ++s) {
+    uint16_t* buf = L + (NBUF == 2 ? (s & 1) * BUF : 0);
+    uint16_t* nxt = L + (NBUF == 2 ? ((s + 1) & 1) * BUF : 0);
+    if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of step s have landed
+    if constexpr (NBUF == 1) __syncthreads();          // step s - 1 is consumed
+    finish(s, buf);
+    __syncthreads();  // every wave's part of step s is there (and, NBUF = 2, step s - 1 consumed)
+    if (s + 1 < n) start(s + 1, nxt);
+    compute(s, buf);
   }
 }
 
-// ---------------------------------------------------------------------------
-// forward
-// ---------------------------------------------------------------------------
-template <int D, class IT, class OT, int BN, int WQ, int WK, int DS, int NBUF, int MINW>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * WQ * WK * DS, 64 * WQ * WK * DS), amdgpu_waves_per_eu(MINW, MINW)))
+template <int D, class IT, class OT, int NW, int MINW, int RES>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW), amdgpu_waves_per_eu(MINW, MINW)))
 void fwd_s3(KArgs a) {
-  using W = Place<WQ, WK, DS>;
-  constexpr int NP = Pieces<IT>::n, DW = D / DS, NKD = DW / 16, NMD = DW / 32;
-  constexpr int RPW = 32 * WQ, NT = BN / (32 * WK);
-  static_assert(WK == 1 || DS == 1, "");
-  using St = Stage<D, IT, BN, W::NTH>;
-  constexpr int BUF = 2 * St::ELTS;  // K planes, then V planes
-  constexpr int XCH = DS == 1 ? 0 : W::NTH * 16 * NT * 2;  // S halves (in 16-bit elements)
-  constexpr int OUT = WK == 1 ? WQ * DS * put_bytes<DW>() : WK * RPW * D * 4;
-  __shared__ __attribute__((aligned(16))) uint16_t L[cmax(NBUF * BUF + XCH, OUT / 2)];
-  __shared__ float Ml[2][WK == 1 ? 1 : WQ * WK][32];
+  constexpr int NTH = 64 * NW, NSUB = TILE / (16 * NW), NP = Pieces<IT>::n, NKD = D / 32, NMD = D / 16;
+  using R = Rows<D, IT, NTH>;
+  constexpr int BUF = 2 * R::ELTS, NBUF = R::DMA || 4 * BUF <= 56 * 1024 ? 2 : 1;
+  __shared__ __attribute__((aligned(512))) uint16_t L[cmax(NBUF * BUF, NW * 16 * D * 2)];
 
-  const int item = a.q_order[blockIdx.x / W::NSUB];
+  const Slot slot = launch_slot<NSUB, RES>(a);
+  const int item = slot.ok ? a.q_order[slot.slot] : -1;
   if (item < 0 || item >= a.B * a.Hq * a.nqt) return;  // idle slot (or an entry out of range)
   const int qt = item % a.nqt, bh = item / a.nqt;
   const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.G;
   const int mrow = map_row(a, b, h, a.nqt, qt);
-  const Walk<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
-  const W w;
-  const int wrow = (blockIdx.x % W::NSUB) * RPW;  // workgroup's first row in the tile
-  if (qt * TILE + wrow >= a.Lq) return;           // (a ragged last tile's empty part)
-  const int qloc = wrow + 32 * w.wq + w.l32;
-  const int q = qt * TILE + qloc;
+  Walk<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
+  const int wrow = slot.part * 16 * NW;
+  if (qt * TILE + wrow >= a.Lq) return;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t ra = row_addr<D>(l16, g), ta = tr_addr<D>(l16, g);
+  const int qloc = wrow + 16 * wave + l16, q = qt * TILE + qloc;
 
   const char* kb = head_base(a.k, a.ks, b, hk, elt_bytes<IT>());
   const char* vb = head_base(a.v, a.vs, b, hk, elt_bytes<IT>());
-  St ks, vs;
-  if (walk.n > 0) {
-    ks.load(kb, a.ks[1], walk.first(0), a.Lk);
-    vs.load(vb, a.vs[1], walk.first(0), a.Lk);
-  }
   Frag<NP> qf[NKD];
-  own_rows<IT>(qf, head_base(a.q, a.qs, b, h, elt_bytes<IT>()), a.qs[1], min(q, a.Lq - 1), w.ds * DW, w.hi);
-
-  f32x16 acc[NMD];
+  own16<D, IT>(qf, head_base(a.q, a.qs, b, h, elt_bytes<IT>()), a.qs[1], min(q, a.Lq - 1), g);
+  f32x4 acc[NMD];
 #pragma unroll
-  for (int i = 0; i < NMD; ++i) acc[i] = f32x16{};
+  for (int i = 0; i < NMD; ++i) acc[i] = f32x4{};
   float m2 = NEG_INF, l = 0.f;
   const float c2 = a.scale_log2;
-  float* X = (float*)(L + NBUF * BUF);
 
-  auto stage = [&](int s) {  // registers -> LDS buffer of sub-block s; the next one's rows -> registers
-    uint16_t* buf = L + (NBUF == 2 ? (s & 1) * BUF : 0);
-    ks.store(buf);
-    vs.store(buf + St::ELTS);
-    if (s + 1 < walk.n) {
-      ks.load(kb, a.ks[1], walk.first(s + 1), a.Lk);
-      vs.load(vb, a.vs[1], walk.first(s + 1), a.Lk);
-    }
-  };
-  auto compute = [&](int s) {
-    const uint16_t* Kl = L + (NBUF == 2 ? (s & 1) * BUF : 0);
-    const uint16_t* Vl = Kl + St::ELTS;
-    const int mask = walk.mask(s), blk0 = (s % Walk<BN>::SPT) * (BN / 32) + w.wk * NT;
-    uint32_t w32[NT];
-    bool live = true;
-    if (mask >= 0) {
-      bool any = false;
+  R ks, vs;
+  walk_rows<NBUF, R::DMA, BUF>(walk.n, L,
+      [&](int s, uint16_t* buf) {
+        const int k0 = walk.first(s);
+        ks.load(kb, a.ks[1], k0, a.Lk, buf);
+        vs.load(vb, a.vs[1], k0, a.Lk, buf + R::ELTS);
+      },
+      [&](int, uint16_t* buf) {
+        ks.store(buf);
+        vs.store(buf + R::ELTS);
+      },
+      [&](int s, const uint16_t* Kl) {
+        const uint16_t* Vl = Kl + R::ELTS;
+        const int mask = walk.mask(s);
+        uint32_t w = 0xffffffffu;
+        if (mask >= 0) {
+          w = bits32(a.row_bits, mask, s % Walk<BN>::SPT, qloc, g);
+          if (!__any((w & 0x000f000fu) != 0)) return;  // no allowed key of the wave's rows here
+        }
+        f32x4 st[2] = {f32x4{}, f32x4{}};
+        one_dot<D, NP>(lds_addr(Kl) + ra, qf, st);
+        if (mask >= 0) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        w32[t] = bits32(a.row_bits, mask, blk0 + t, qloc);
-        any |= w32[t] != 0;
-      }
-      live = __any(any);  // an allowed key of the wave's rows here
-    }
-    f32x16 st[NT];
-    if (live) {
+          for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        st[t] = f32x16{};
+            for (int r = 0; r < 4; ++r) st[t][r] = mask_neg_inf(st[t][r], ones16(w, t, r));
+        }
+        float mx = NEG_INF;
 #pragma unroll
-        for (int kd = 0; kd < NKD; ++kd)
-          st[t] = mma(row_frag<D, NP, BN>(Kl, 32 * (w.wk * NT + t) + w.l32, w.ds * NKD + kd, w.hi), qf[kd], st[t]);
-      }
-      if constexpr (DS == 2) half_put(st, X, w.wave, w.lane);
-    }
-    if constexpr (DS == 2) __syncthreads();
-    if (!live) return;
-    if constexpr (DS == 2) half_add(st, X, w.partner(), w.lane);
-    if (mask >= 0) {
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+          for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[t][r]);
+        const float mx2 = wave_max32(wave_max16(mx)) * c2;
+        // the running max is raised only when a row's grows by more than 2^8
+        if (__any(mx2 > m2 + 8.f)) {
+          const float mn = fmaxf(m2, mx2);
+          const float alpha = (mn == NEG_INF) ? 1.f : fast_exp2(m2 - mn);
+          l *= alpha;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) st[t][r] = mask_neg_inf(st[t][r], mask_ones(w32[t] >> (4 * w.hi), r));
-    }
-    float mx = NEG_INF;
+          for (int i = 0; i < NMD; ++i) acc[i] *= alpha;
+          m2 = mn;
+        }
+        const float nmu = (m2 == NEG_INF) ? 0.f : -m2;
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[t][r]);
-    const float mx2 = wave_max32(mx) * c2;
-    // the running max is raised only when a row's grows by more than 2^8 (P <= 2^8
-    // until then; the pieces keep float32's range)
-    if (__any(mx2 > m2 + 8.f)) {
-      const float mn = fmaxf(m2, mx2);
-      const float alpha = (mn == NEG_INF) ? 1.f : fast_exp2(m2 - mn);
-      l *= alpha;
-#pragma unroll
-      for (int i = 0; i < NMD; ++i) acc[i] *= alpha;
-      m2 = mn;
-    }
-    const float nmu = (m2 == NEG_INF) ? 0.f : -m2;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        st[t][r] = fast_exp2(fmaf(st[t][r], c2, nmu));
-        l += st[t][r];
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const Frag<3> pf = c_frag(st[t], j);
-#pragma unroll
-        for (int mt = 0; mt < NMD; ++mt)
-          acc[mt] = mma(tr_frag<D, NP, BN>(Vl, 32 * (w.wk * NT + t) + 16 * j, w.ds * NMD + mt, w.lane), pf, acc[mt]);
-      }
-    }
-  };
-  run_walk<NBUF>(walk.n, stage, compute);
+          for (int r = 0; r < 4; ++r) {
+            st[t][r] = fast_exp2(fmaf(st[t][r], c2, nmu));
+            l += st[t][r];
+          }
+        add_rows<D, NP>(lds_addr(Vl) + ta, c_frag16(st[0], st[1]), acc);
+      });
 
+  l += __shfl_xor(l, 16);
   l = wave_sum32(l);
-  const int nrows = a.Lq - (qt * TILE + wrow);
-  const int64_t orow = (int64_t)b * a.os[0] + (int64_t)(qt * TILE + wrow) * a.os[1] + (int64_t)h * a.os[2];
-  float* lse = a.lse + ((int64_t)b * a.Hq + h) * a.Lq;
+  if (g == 0 && q < a.Lq) a.lse[((int64_t)b * a.Hq + h) * a.Lq + q] = l > 0.f ? m2 + __builtin_log2f(l) : NEG_INF;
   __syncthreads();  // every wave is done with the operand tiles
-  if constexpr (WK == 1) {
-    if (w.ds == 0 && w.hi == 0 && q < a.Lq) lse[q] = l > 0.f ? m2 + __builtin_log2f(l) : NEG_INF;
-    put_rows<DW, OT>(acc, l > 0.f ? 1.f / l : 0.f, (char*)L + w.wave * put_bytes<DW>(), a.out,
-                     orow + (int64_t)32 * w.wq * a.os[1] + w.ds * DW, a.os[1], nrows - 32 * w.wq, w.lane);
-  } else {
-    if (w.hi == 0) {
-      Ml[0][w.wave][w.l32] = m2;
-      Ml[1][w.wave][w.l32] = l;
-    }
-    __syncthreads();
-    float M = NEG_INF, lt = 0.f;
-#pragma unroll
-    for (int k = 0; k < WK; ++k) M = fmaxf(M, Ml[0][k * WQ + w.wq][w.l32]);
-#pragma unroll
-    for (int k = 0; k < WK; ++k) {
-      const float mk = Ml[0][k * WQ + w.wq][w.l32];
-      lt += mk == NEG_INF ? 0.f : Ml[1][k * WQ + w.wq][w.l32] * fast_exp2(mk - M);
-    }
-    const float f = (m2 == NEG_INF || !(lt > 0.f)) ? 0.f : fast_exp2(m2 - M) / lt;
-    if (w.wk == 0 && w.hi == 0 && q < a.Lq) lse[q] = lt > 0.f ? M + __builtin_log2f(lt) : NEG_INF;
-    slab_put<D, WQ>(acc, f, (float*)L, w.wq, w.wk, w.lane);
-    __syncthreads();
-    slab_sum_store<D, OT, WQ, WK, W::NTH>((const float*)L, a.out, orow, a.os[1], nrows);
-  }
+  const int r0 = qt * TILE + wrow + 16 * wave;
+  put16<D, OT>(acc, l > 0.f ? 1.f / l : 0.f, (float*)L + wave * 16 * D, a.out,
+               (int64_t)b * a.os[0] + (int64_t)r0 * a.os[1] + (int64_t)h * a.os[2], a.os[1], a.Lq - r0, lane);
 }
 
-// ---------------------------------------------------------------------------
-// backward
-// ---------------------------------------------------------------------------
+template <int D, class IT, class OT, int NW, int MINW, int RES>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW), amdgpu_waves_per_eu(MINW, MINW)))
+void bwd_dq_s3(KArgs a) {
+  constexpr int NTH = 64 * NW, NSUB = TILE / (16 * NW), NP = Pieces<IT>::n, NG = Pieces<OT>::n;
+  constexpr int NKD = D / 32, NMD = D / 16;
+  using R = Rows<D, IT, NTH>;
+  constexpr int BUF = 2 * R::ELTS, NBUF = R::DMA || 4 * BUF <= 56 * 1024 ? 2 : 1;
+  __shared__ __attribute__((aligned(512))) uint16_t L[cmax(NBUF * BUF, NW * 16 * D * 2)];
+
+  const Slot slot = launch_slot<NSUB, RES>(a);
+  const int item = slot.ok ? a.q_order[slot.slot] : -1;
+  if (item < 0 || item >= a.B * a.Hq * a.nqt) return;  // idle slot (or an entry out of range)
+  const int qt = item % a.nqt, bh = item / a.nqt;
+  const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.G;
+  const int mrow = map_row(a, b, h, a.nqt, qt);
+  Walk<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
+  const int wrow = slot.part * 16 * NW;
+  if (qt * TILE + wrow >= a.Lq) return;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t ra = row_addr<D>(l16, g), ta = tr_addr<D>(l16, g);
+  const int qloc = wrow + 16 * wave + l16, qc = min(qt * TILE + qloc, a.Lq - 1);
+
+  const char* kb = head_base(a.k, a.ks, b, hk, elt_bytes<IT>());
+  const char* vb = head_base(a.v, a.vs, b, hk, elt_bytes<IT>());
+  Frag<NP> qf[NKD];
+  Frag<NG> gf[NKD];
+  own16<D, IT>(qf, head_base(a.q, a.qs, b, h, elt_bytes<IT>()), a.qs[1], qc, g);
+  own16<D, OT>(gf, head_base(a.dO, a.dos, b, h, elt_bytes<OT>()), a.dos[1], qc, g);
+  const int64_t rs = ((int64_t)b * a.Hq + h) * a.Lq + qc;
+  const float lse = a.lse[rs], delta = a.delta[rs], c2 = a.scale_log2;
+  f32x4 acc[NMD];
+#pragma unroll
+  for (int i = 0; i < NMD; ++i) acc[i] = f32x4{};
+
+  R ks, vs;
+  walk_rows<NBUF, R::DMA, BUF>(walk.n, L,
+      [&](int s, uint16_t* buf) {
+        const int k0 = walk.first(s);
+        ks.load(kb, a.ks[1], k0, a.Lk, buf);
+        vs.load(vb, a.vs[1], k0, a.Lk, buf + R::ELTS);
+      },
+      [&](int, uint16_t* buf) {
+        ks.store(buf);
+        vs.store(buf + R::ELTS);
+      },
+      [&](int s, const uint16_t* Kl) {
+        const uint16_t* Vl = Kl + R::ELTS;
+        const int mask = walk.mask(s);
+        uint32_t w = 0xffffffffu;
+        if (mask >= 0) {
+          w = bits32(a.row_bits, mask, s % Walk<BN>::SPT, qloc, g);
+          if (!__any((w & 0x000f000fu) != 0)) return;
+        }
+        f32x4 st[2] = {f32x4{}, f32x4{}}, dp[2] = {f32x4{}, f32x4{}};
+        two_dots<D == 64 ? 2 : 1, D, NP, NP, NP, NG>(lds_addr(Kl) + ra, lds_addr(Vl) + ra, qf, gf, st, dp);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) st[t][r] = fast_exp2(fmaf(st[t][r], c2, -lse));
+        if (mask >= 0) zero16(st, w);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) dp[t][r] = st[t][r] * (dp[t][r] - delta);
+        add_rows<D, NP>(lds_addr(Kl) + ta, c_frag16(dp[0], dp[1]), acc);
+      });
+
+  __syncthreads();
+  const int r0 = qt * TILE + wrow + 16 * wave;
+  put16<D, IT>(acc, a.scale, (float*)L + wave * 16 * D, a.dq,
+               (int64_t)b * a.dqs[0] + (int64_t)r0 * a.dqs[1] + (int64_t)h * a.dqs[2], a.dqs[1], a.Lq - r0, lane);
+}
+
+// two LDS buffers where Q's rows are loaded to LDS directly, or they leave room for
+// two workgroups a CU
+template <int D, class IT, class OT>
+constexpr int dkdv_bufs() {
+  return 4 * (Pieces<IT>::n + Pieces<OT>::n) * BN * D <= (Pieces<IT>::n == 1 ? 158 : 56) * 1024 ? 2 : 1;
+}
+
+// PART: 3 = dV and dK; 1 = dV, 2 = dK: workgroups of their own at D = 256, where both
+// accumulators, K and V would take 192 registers of a wave's 256 (S is then formed
+// twice, 1/14 of the products).
+template <int D, class IT, class OT, int PART, int NW>
+__device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, int sl, int sub) {
+  constexpr bool DV = PART & 1, DK = PART & 2;
+  constexpr int NTH = 64 * NW, NP = Pieces<IT>::n, NG = Pieces<OT>::n;
+  constexpr int NKD = D / 32, NMD = D / 16;
+  using Rq = Rows<D, IT, NTH>;
+  using Rg = Rows<D, OT, NTH, true>;
+  constexpr int BUF = Rq::ELTS + Rg::ELTS, NBUF = dkdv_bufs<D, IT, OT>();
+  const int item = a.kv_order[sl];
+  if (item < 0 || item >= a.B * a.Hkv * a.nkt) return;  // idle slot (or an entry out of range)
+  const int kt = item % a.nkt, bh = item / a.nkt;
+  const int hk = bh % a.Hkv, b = bh / a.Hkv;
+  const int wrow = sub * 16 * NW;
+  if (kt * TILE + wrow >= a.Lk) return;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t ra = row_addr<D>(l16, g), ta = tr_addr<D>(l16, g);
+  const int kloc = wrow + 16 * wave + l16, kc = min(kt * TILE + kloc, a.Lk - 1);
+  const float c2 = a.scale_log2;
+
+  Frag<NP> kf[NKD], vf[DK ? NKD : 1];
+  own16<D, IT>(kf, head_base(a.k, a.ks, b, hk, elt_bytes<IT>()), a.ks[1], kc, g);
+  if constexpr (DK) own16<D, IT>(vf, head_base(a.v, a.vs, b, hk, elt_bytes<IT>()), a.vs[1], kc, g);
+  f32x4 dk[DK ? NMD : 1], dv[DV ? NMD : 1];
+#pragma unroll
+  for (int i = 0; i < NMD; ++i) {
+    if constexpr (DK) dk[i] = f32x4{};
+    if constexpr (DV) dv[i] = f32x4{};
+  }
+
+  for (int gh = 0; gh < a.G; ++gh) {
+    const int h = hk * a.G + gh;
+    const int mc = map_row(a, b, h, a.nkt, kt);
+    Walk<BN> walk(a.col_ent, a.col_ptr[mc], a.col_ptr[mc + 1]);
+    const char* qb = head_base(a.q, a.qs, b, h, elt_bytes<IT>());
+    const char* gb = head_base(a.dO, a.dos, b, h, elt_bytes<OT>());
+    const int64_t rs = ((int64_t)b * a.Hq + h) * a.Lq;
+    Rq rq;
+    Rg rg;
+    float rl = 0.f;  // lse (threads 0 .. BN - 1) or delta (the next BN) of a row
+    __syncthreads();  // the previous head's last step is consumed
+    walk_rows<NBUF, Rq::DMA || Rg::DMA, BUF>(walk.n, L,
+        [&](int s, uint16_t* buf) {
+          const int q0 = walk.first(s);
+          rq.load(qb, a.qs[1], q0, a.Lq, buf);
+          rg.load(gb, a.dos[1], q0, a.Lq, buf + Rq::ELTS);
+          if (threadIdx.x < 2 * BN) {
+            const int64_t r = rs + min(q0 + (int)(threadIdx.x % BN), a.Lq - 1);
+            rl = threadIdx.x < BN ? a.lse[r] : a.delta[r];
+          }
+        },
+        [&](int s, uint16_t* buf) {
+          rq.store(buf);
+          rg.store(buf + Rq::ELTS);
+          if (threadIdx.x < 2 * BN) Rl[(NBUF == 2 ? s & 1 : 0) * 2 * BN + threadIdx.x] = rl;
+        },
+        [&](int s, const uint16_t* Ql) {
+          const uint16_t* Gl = Ql + Rq::ELTS;
+          const float* Rs = Rl + (NBUF == 2 ? s & 1 : 0) * 2 * BN + 4 * g;
+          const int mask = walk.mask(s);
+          uint32_t w = 0xffffffffu;
+          if (mask >= 0) {
+            w = bits32(a.col_bits, mask, s % Walk<BN>::SPT, kloc, g);
+            if (!__any((w & 0x000f000fu) != 0)) return;
+          }
+          f32x4 st[2] = {f32x4{}, f32x4{}}, dp[2] = {f32x4{}, f32x4{}};
+          if constexpr (!DK) one_dot<D, NP>(lds_addr(Ql) + ra, kf, st);
+          else two_dots<D == 128 ? 1 : 2, D, NP, NP, NG, NP>(lds_addr(Ql) + ra, lds_addr(Gl) + ra, kf, vf, st, dp);
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const f32x4 ls = *(const f32x4*)(Rs + 16 * t), dl = *(const f32x4*)(Rs + BN + 16 * t);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              st[t][r] = fast_exp2(fmaf(st[t][r], c2, -ls[r]));
+              if constexpr (DK) dp[t][r] -= dl[r];
+            }
+          }
+          if (mask >= 0) zero16(st, w);
+          if constexpr (DK) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) dp[t] *= st[t];
+          }
+          if constexpr (DV) add_rows<D, NG>(lds_addr(Gl) + ta, c_frag16(st[0], st[1]), dv);
+          if constexpr (DK) add_rows<D, NP>(lds_addr(Ql) + ta, c_frag16(dp[0], dp[1]), dk);
+        });
+  }
+
+  const int r0 = kt * TILE + wrow + 16 * wave;
+  __syncthreads();
+  if constexpr (DV)
+    put16<D, IT>(dv, 1.f, (float*)L + wave * 16 * D, a.dv,
+                 (int64_t)b * a.dvs[0] + (int64_t)r0 * a.dvs[1] + (int64_t)hk * a.dvs[2], a.dvs[1], a.Lk - r0, lane);
+  if constexpr (DK)
+    put16<D, IT>(dk, a.scale, (float*)L + wave * 16 * D, a.dk,
+                 (int64_t)b * a.dks[0] + (int64_t)r0 * a.dks[1] + (int64_t)hk * a.dks[2], a.dks[1], a.Lk - r0, lane);
+}
+
+template <int D, class IT, class OT, int NW, int MINW, int RES>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW), amdgpu_waves_per_eu(MINW, MINW)))
+void bwd_dkdv_s3(KArgs a) {
+  constexpr int NBUF = dkdv_bufs<D, IT, OT>();
+  constexpr int BUF = Rows<D, IT, 64 * NW>::ELTS + Rows<D, OT, 64 * NW>::ELTS;
+  __shared__ __attribute__((aligned(512))) uint16_t L[cmax(NBUF * BUF, NW * 16 * D * 2)];
+  __shared__ __attribute__((aligned(16))) float Rl[NBUF * 2 * BN];  // lse, delta of the step's rows
+  constexpr int NPART = D == 256 ? 2 : 1;
+  const Slot s = launch_slot<NPART * TILE / (16 * NW), RES>(a);
+  if (!s.ok) return;
+  if constexpr (NPART == 1) dkdv_s3<D, IT, OT, 3, NW>(a, L, Rl, s.slot, s.part);
+  else if (s.part & 1) dkdv_s3<D, IT, OT, 1, NW>(a, L, Rl, s.slot, s.part >> 1);
+  else dkdv_s3<D, IT, OT, 2, NW>(a, L, Rl, s.slot, s.part >> 1);
+}
 
 // delta = rowsum(dO * O), summed in float64: D / 8 threads a row, the rows in the
 // order of memory (head fastest where a row of O holds all heads)
@@ -291,300 +586,56 @@ void delta_s3(KArgs a) {
   if (part == 0) a.delta[((int64_t)b * a.Hq + h) * a.Lq + q] = (float)s;
 }
 
-template <int D, class IT, class OT, int BN, int WQ, int WK, int DS, int NBUF, int MINW>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * WQ * WK * DS, 64 * WQ * WK * DS), amdgpu_waves_per_eu(MINW, MINW)))
-void bwd_dq_s3(KArgs a) {
-  using W = Place<WQ, WK, DS>;
-  constexpr int NP = Pieces<IT>::n, NG = Pieces<OT>::n, DW = D / DS, NKD = DW / 16, NMD = DW / 32;
-  constexpr int RPW = 32 * WQ, NT = BN / (32 * WK);
-  static_assert(WK == 1 || DS == 1, "");
-  static_assert(DS == 1 || NT == 1, "one exchange per sub-block");
-  using St = Stage<D, IT, BN, W::NTH>;
-  constexpr int BUF = 2 * St::ELTS;  // K planes, then V planes
-  constexpr int XCH = DS == 1 ? 0 : W::NTH * 32 * 2;  // S and dP halves
-  constexpr int OUT = WK == 1 ? WQ * DS * put_bytes<DW>() : WK * RPW * D * 4;
-  __shared__ __attribute__((aligned(16))) uint16_t L[cmax(NBUF * BUF + XCH, OUT / 2)];
-
-  const int item = a.q_order[blockIdx.x / W::NSUB];
-  if (item < 0 || item >= a.B * a.Hq * a.nqt) return;  // idle slot (or an entry out of range)
-  const int qt = item % a.nqt, bh = item / a.nqt;
-  const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.G;
-  const int mrow = map_row(a, b, h, a.nqt, qt);
-  const Walk<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
-  const W w;
-  const int wrow = (blockIdx.x % W::NSUB) * RPW;
-  if (qt * TILE + wrow >= a.Lq) return;
-  const int qloc = wrow + 32 * w.wq + w.l32;
-  const int q = qt * TILE + qloc, qc = min(q, a.Lq - 1);
-
-  const char* kb = head_base(a.k, a.ks, b, hk, elt_bytes<IT>());
-  const char* vb = head_base(a.v, a.vs, b, hk, elt_bytes<IT>());
-  St ks, vs;
-  if (walk.n > 0) {
-    ks.load(kb, a.ks[1], walk.first(0), a.Lk);
-    vs.load(vb, a.vs[1], walk.first(0), a.Lk);
-  }
-  Frag<NP> qf[NKD];
-  Frag<NG> gf[NKD];
-  own_rows<IT>(qf, head_base(a.q, a.qs, b, h, elt_bytes<IT>()), a.qs[1], qc, w.ds * DW, w.hi);
-  own_rows<OT>(gf, head_base(a.dO, a.dos, b, h, elt_bytes<OT>()), a.dos[1], qc, w.ds * DW, w.hi);
-  const int64_t rs = ((int64_t)b * a.Hq + h) * a.Lq + qc;
-  const float lse = a.lse[rs], delta = a.delta[rs], c2 = a.scale_log2;
-
-  f32x16 acc[NMD];
-#pragma unroll
-  for (int i = 0; i < NMD; ++i) acc[i] = f32x16{};
-  float* X = (float*)(L + NBUF * BUF);
-
-  auto stage = [&](int s) {
-    uint16_t* buf = L + (NBUF == 2 ? (s & 1) * BUF : 0);
-    ks.store(buf);
-    vs.store(buf + St::ELTS);
-    if (s + 1 < walk.n) {
-      ks.load(kb, a.ks[1], walk.first(s + 1), a.Lk);
-      vs.load(vb, a.vs[1], walk.first(s + 1), a.Lk);
-    }
-  };
-  auto compute = [&](int s) {
-    const uint16_t* Kl = L + (NBUF == 2 ? (s & 1) * BUF : 0);
-    const uint16_t* Vl = Kl + St::ELTS;
-    const int mask = walk.mask(s), blk0 = (s % Walk<BN>::SPT) * (BN / 32) + w.wk * NT;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      uint32_t w32 = 0xffffffffu;
-      if (mask >= 0) w32 = bits32(a.row_bits, mask, blk0 + t, qloc);
-      const bool live = __any(w32 != 0);
-      const int r0 = 32 * (w.wk * NT + t);
-      f32x16 sd[2];  // S, dP
-      if (live) {
-        sd[0] = sd[1] = f32x16{};
-#pragma unroll
-        for (int kd = 0; kd < NKD; ++kd) {
-          sd[0] = mma(row_frag<D, NP, BN>(Kl, r0 + w.l32, w.ds * NKD + kd, w.hi), qf[kd], sd[0]);
-          sd[1] = mma(row_frag<D, NP, BN>(Vl, r0 + w.l32, w.ds * NKD + kd, w.hi), gf[kd], sd[1]);
-        }
-        if constexpr (DS == 2) half_put(sd, X, w.wave, w.lane);
-      }
-      if constexpr (DS == 2) __syncthreads();
-      if (!live) continue;
-      if constexpr (DS == 2) half_add(sd, X, w.partner(), w.lane);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float p = fast_exp2(fmaf(sd[0][r], c2, -lse));
-        if (mask >= 0) p = mask_zero(p, mask_ones(w32 >> (4 * w.hi), r));
-        sd[1][r] = p * (sd[1][r] - delta);
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const Frag<3> df = c_frag(sd[1], j);
-#pragma unroll
-        for (int mt = 0; mt < NMD; ++mt)
-          acc[mt] = mma(tr_frag<D, NP, BN>(Kl, r0 + 16 * j, w.ds * NMD + mt, w.lane), df, acc[mt]);
-      }
-    }
-  };
-  run_walk<NBUF>(walk.n, stage, compute);
-
-  const int nrows = a.Lq - (qt * TILE + wrow);
-  const int64_t orow = (int64_t)b * a.dqs[0] + (int64_t)(qt * TILE + wrow) * a.dqs[1] + (int64_t)h * a.dqs[2];
-  __syncthreads();
-  if constexpr (WK == 1) {
-    put_rows<DW, IT>(acc, a.scale, (char*)L + w.wave * put_bytes<DW>(), a.dq,
-                     orow + (int64_t)32 * w.wq * a.dqs[1] + w.ds * DW, a.dqs[1], nrows - 32 * w.wq, w.lane);
-  } else {
-    slab_put<D, WQ>(acc, a.scale, (float*)L, w.wq, w.wk, w.lane);
-    __syncthreads();
-    slab_sum_store<D, IT, WQ, WK, W::NTH>((const float*)L, a.dq, orow, a.dqs[1], nrows);
-  }
-}
-
-// PART: 1 = dV, 2 = dK, 3 = both in one workgroup.  At D = 256 the two run in
-// workgroups of their own (S is then formed twice, 1/14 of the products): both
-// accumulators would take half of a wave's registers.
-template <int D, class IT, class OT, int PART, int WQ, int WK, int DS, int NBUF>
-__device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, int slot, int sub) {
-  using W = Place<WQ, WK, DS>;
-  constexpr int NP = Pieces<IT>::n, NG = Pieces<OT>::n, DW = D / DS, NKD = DW / 16, NMD = DW / 32;
-  constexpr int RPW = 32 * WQ, BN = 32 * WK;  // BN: queries per sub-block
-  constexpr bool DV = PART & 1, DK = PART & 2;
-  static_assert(WK == 1 || DS == 1, "");
-  using Sq = Stage<D, IT, BN, W::NTH>;
-  using Sg = Stage<D, OT, BN, W::NTH>;
-  constexpr int BUF = Sq::ELTS + Sg::ELTS;
-
-  const int item = a.kv_order[slot];
-  if (item < 0 || item >= a.B * a.Hkv * a.nkt) return;  // idle slot (or an entry out of range)
-  const int kt = item % a.nkt, bh = item / a.nkt;
-  const int hk = bh % a.Hkv, b = bh / a.Hkv;
-  const W w;
-  const int wrow = sub * RPW;
-  if (kt * TILE + wrow >= a.Lk) return;
-  const int kloc = wrow + 32 * w.wq + w.l32;
-  const int kc = min(kt * TILE + kloc, a.Lk - 1);
-  const float c2 = a.scale_log2;
-  float* X = (float*)(L + NBUF * BUF);
-
-  Frag<NP> kf[NKD], vf[DK ? NKD : 1];
-  own_rows<IT>(kf, head_base(a.k, a.ks, b, hk, elt_bytes<IT>()), a.ks[1], kc, w.ds * DW, w.hi);
-  if constexpr (DK) own_rows<IT>(vf, head_base(a.v, a.vs, b, hk, elt_bytes<IT>()), a.vs[1], kc, w.ds * DW, w.hi);
-  f32x16 dk[DK ? NMD : 1], dv[DV ? NMD : 1];
-#pragma unroll
-  for (int i = 0; i < NMD; ++i) {
-    if constexpr (DK) dk[i] = f32x16{};
-    if constexpr (DV) dv[i] = f32x16{};
-  }
-
-  for (int g = 0; g < a.G; ++g) {
-    const int h = hk * a.G + g;
-    const int mc = map_row(a, b, h, a.nkt, kt);
-    const Walk<BN> walk(a.col_ent, a.col_ptr[mc], a.col_ptr[mc + 1]);
-    if (walk.n == 0) continue;
-    const char* qb = head_base(a.q, a.qs, b, h, elt_bytes<IT>());
-    const char* gb = head_base(a.dO, a.dos, b, h, elt_bytes<OT>());
-    const int64_t rs = ((int64_t)b * a.Hq + h) * a.Lq;
-    Sq sq;
-    Sg sg;
-    float rl = 0.f;  // lse (threads 0 .. BN - 1) or delta (the next BN) of a row
-    auto load = [&](int s) {
-      const int q0 = walk.first(s);
-      sq.load(qb, a.qs[1], q0, a.Lq);
-      sg.load(gb, a.dos[1], q0, a.Lq);
-      if (threadIdx.x < 2 * BN) {
-        const int64_t r = rs + min(q0 + (int)(threadIdx.x % BN), a.Lq - 1);
-        rl = threadIdx.x < BN ? a.lse[r] : a.delta[r];
-      }
-    };
-    auto stage = [&](int s) {
-      uint16_t* buf = L + (NBUF == 2 ? (s & 1) * BUF : 0);
-      sq.store(buf);
-      sg.store(buf + Sq::ELTS);
-      if (threadIdx.x < 2 * BN) Rl[(NBUF == 2 ? (s & 1) * 2 * BN : 0) + threadIdx.x] = rl;
-      if (s + 1 < walk.n) load(s + 1);
-    };
-    auto compute = [&](int s) {
-      const uint16_t* Ql = L + (NBUF == 2 ? (s & 1) * BUF : 0);
-      const uint16_t* Gl = Ql + Sq::ELTS;
-      const float* R = Rl + (NBUF == 2 ? (s & 1) * 2 * BN : 0) + 32 * w.wk + 4 * w.hi;
-      const int mask = walk.mask(s), blk = (s % Walk<BN>::SPT) * WK + w.wk;
-      uint32_t w32 = 0xffffffffu;
-      if (mask >= 0) w32 = bits32(a.col_bits, mask, blk, kloc);
-      const bool live = __any(w32 != 0);
-      const int r0 = 32 * w.wk;
-      f32x16 sd[DK ? 2 : 1];  // S, dP
-      if (live) {
-#pragma unroll
-        for (int n = 0; n < (DK ? 2 : 1); ++n) sd[n] = f32x16{};
-#pragma unroll
-        for (int kd = 0; kd < NKD; ++kd) {
-          sd[0] = mma(row_frag<D, NP, BN>(Ql, r0 + w.l32, w.ds * NKD + kd, w.hi), kf[kd], sd[0]);
-          if constexpr (DK) sd[1] = mma(row_frag<D, NG, BN>(Gl, r0 + w.l32, w.ds * NKD + kd, w.hi), vf[kd], sd[1]);
-        }
-        if constexpr (DS == 2) half_put(sd, X, w.wave, w.lane);
-      }
-      if constexpr (DS == 2) __syncthreads();
-      if (!live) return;
-      if constexpr (DS == 2) half_add(sd, X, w.partner(), w.lane);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const f32x4 ls = *(const f32x4*)(R + 8 * j), dl = *(const f32x4*)(R + BN + 8 * j);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * j + i;
-          float p = fast_exp2(fmaf(sd[0][r], c2, -ls[i]));
-          if (mask >= 0) p = mask_zero(p, mask_ones(w32 >> (4 * w.hi), r));
-          sd[0][r] = p;
-          if constexpr (DK) sd[1][r] = p * (sd[1][r] - dl[i]);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if constexpr (DV) {
-          const Frag<3> pf = c_frag(sd[0], j);
-#pragma unroll
-          for (int mt = 0; mt < NMD; ++mt)
-            dv[mt] = mma(tr_frag<D, NG, BN>(Gl, r0 + 16 * j, w.ds * NMD + mt, w.lane), pf, dv[mt]);
-        }
-        if constexpr (DK) {
-          const Frag<3> df = c_frag(sd[DK ? 1 : 0], j);
-#pragma unroll
-          for (int mt = 0; mt < NMD; ++mt)
-            dk[mt] = mma(tr_frag<D, NP, BN>(Ql, r0 + 16 * j, w.ds * NMD + mt, w.lane), df, dk[mt]);
-        }
-      }
-    };
-    load(0);
-    __syncthreads();  // the previous head's last sub-block is consumed
-    run_walk<NBUF>(walk.n, stage, compute);
-  }
-
-  const int nrows = a.Lk - (kt * TILE + wrow);
-  auto out = [&](const f32x16(&acc)[NMD], float sc, void* dst, const int64_t* st) {
-    const int64_t row = (int64_t)b * st[0] + (int64_t)(kt * TILE + wrow) * st[1] + (int64_t)hk * st[2];
-    __syncthreads();
-    if constexpr (WK == 1) {
-      put_rows<DW, IT>(acc, sc, (char*)L + w.wave * put_bytes<DW>(), dst,
-                       row + (int64_t)32 * w.wq * st[1] + w.ds * DW, st[1], nrows - 32 * w.wq, w.lane);
-    } else {
-      slab_put<D, WQ>(acc, sc, (float*)L, w.wq, w.wk, w.lane);
-      __syncthreads();
-      slab_sum_store<D, IT, WQ, WK, W::NTH>((const float*)L, dst, row, st[1], nrows);
-    }
-  };
-  if constexpr (DV) out(dv, 1.f, a.dv, a.dvs);
-  if constexpr (DK) out(dk, a.scale, a.dk, a.dks);
-}
-
-template <int D, class IT, class OT, bool BOTH, int WQ, int WK, int DS, int NBUF, int MINW>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * WQ * WK * DS, 64 * WQ * WK * DS), amdgpu_waves_per_eu(MINW, MINW)))
-void bwd_dkdv_s3(KArgs a) {
-  using W = Place<WQ, WK, DS>;
-  constexpr int BN = 32 * WK;
-  constexpr int BUF = Stage<D, IT, BN, W::NTH>::ELTS + Stage<D, OT, BN, W::NTH>::ELTS;
-  constexpr int XCH = DS == 1 ? 0 : W::NTH * 32 * 2;
-  constexpr int OUT = WK == 1 ? WQ * DS * put_bytes<D / DS>() : WK * 32 * WQ * D * 4;
-  __shared__ __attribute__((aligned(16))) uint16_t L[cmax(NBUF * BUF + XCH, OUT / 2)];
-  __shared__ __attribute__((aligned(16))) float Rl[NBUF * 2 * BN];
-  if constexpr (BOTH) {
-    dkdv_s3<D, IT, OT, 3, WQ, WK, DS, NBUF>(a, L, Rl, blockIdx.x / W::NSUB, blockIdx.x % W::NSUB);
-  } else {
-    const int slot = blockIdx.x / (2 * W::NSUB), sub = (blockIdx.x >> 1) % W::NSUB;
-    if (blockIdx.x & 1) dkdv_s3<D, IT, OT, 1, WQ, WK, DS, NBUF>(a, L, Rl, slot, sub);
-    else dkdv_s3<D, IT, OT, 2, WQ, WK, DS, NBUF>(a, L, Rl, slot, sub);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
 
-// <BN, WQ, WK, DS, NBUF, MINW> of the kernels per head dimension
+template <int NSUB, int NW, void (*K)(KArgs)>
+void go(KArgs a, int grid, hipStream_t st) {
+  a.n_slots = grid;
+  hipLaunchKernelGGL(K, dim3((grid + 7) / 8 * 8 * NSUB), dim3(64 * NW), 0, st, a);
+}
+
+// <waves, waves per SIMD the registers are given for, workgroups resident on a CU>: two
+// waves a SIMD where that spills nothing inside the walks, else one (a spill's reload
+// also waits for the loads in flight: at D = 128 the float32 step took 697 us with 41
+// spilled registers in dK/dV, 600 at one wave a SIMD).
 template <int D, class IT, class OT>
 struct S3 {
   static constexpr int N = Pieces<IT>::n;
+  template <int NW, int MINW, int RES>
+  static void f(const KArgs& a, int grid, hipStream_t st) {
+    go<TILE / (16 * NW), NW, fwd_s3<D, IT, OT, NW, MINW, RES>>(a, grid, st);
+  }
+  template <int NW, int MINW, int RES>
+  static void q(const KArgs& a, int grid, hipStream_t st) {
+    go<TILE / (16 * NW), NW, bwd_dq_s3<D, IT, OT, NW, MINW, RES>>(a, grid, st);
+  }
+  template <int NW, int MINW, int RES>
+  static void kv(const KArgs& a, int grid, hipStream_t st) {
+    go<(D == 256 ? 2 : 1) * TILE / (16 * NW), NW, bwd_dkdv_s3<D, IT, OT, NW, MINW, RES>>(a, grid, st);
+  }
   static void fwd(const KArgs& a, int grid, hipStream_t st) {
-    if constexpr (D == 64) go<fwd_s3<D, IT, OT, 64, 4, 2, 1, 1, 2>, Place<4, 2, 1>>(a, grid, st);
-    else if constexpr (D == 128) go<fwd_s3<D, IT, OT, 32, 4, 1, 2, 1, 2>, Place<4, 1, 2>>(a, grid, st);
-    else go<fwd_s3<D, IT, OT, 32, 4, 1, 2, N == 1 ? 2 : 1, 2>, Place<4, 1, 2>>(a, grid, st);
+    if constexpr (D == 64) f<4, 3, 3>(a, grid, st);
+    else if constexpr (D == 128) f<4, 2, 2>(a, grid, st);
+    else if constexpr (N == 1) f<4, 2, 2>(a, grid, st);
+    else f<4, 1, 1>(a, grid, st);
   }
   static void bwd(const KArgs& a, int stage, int q_grid, int kv_grid, hipStream_t st) {
     if (stage == MATTN_BWD_PRE) {
       const int64_t threads = (int64_t)a.B * a.Hq * a.Lq * (D / 8);
       hipLaunchKernelGGL((delta_s3<D, OT>), dim3((threads + 255) / 256), dim3(256), 0, st, a);
     } else if (stage == MATTN_BWD_DKDV) {
-      if constexpr (D == 64) go<bwd_dkdv_s3<D, IT, OT, true, 4, 2, 1, 1, 2>, Place<4, 2, 1>>(a, kv_grid, st);
-      else if constexpr (D == 128) go<bwd_dkdv_s3<D, IT, OT, true, 4, 1, 2, 1, 2>, Place<4, 1, 2>>(a, kv_grid, st);
-      else if constexpr (N == 1) go<bwd_dkdv_s3<D, IT, OT, false, 4, 1, 2, 1, 2>, Place<4, 1, 2>>(a, 2 * kv_grid, st);
-      else go<bwd_dkdv_s3<D, IT, OT, false, 2, 1, 2, 1, 1>, Place<2, 1, 2>>(a, 2 * kv_grid, st);
+      if constexpr (D == 64) kv<4, 2, 2>(a, kv_grid, st);
+      else if constexpr (D == 128) kv<4, 1, 1>(a, kv_grid, st);
+      else if constexpr (N == 1) kv<8, 2, 1>(a, kv_grid, st);
+      else kv<4, 1, 1>(a, kv_grid, st);
     } else {
-      if constexpr (D == 64) go<bwd_dq_s3<D, IT, OT, 64, 4, 2, 1, 1, 2>, Place<4, 2, 1>>(a, q_grid, st);
-      else if constexpr (D == 128) go<bwd_dq_s3<D, IT, OT, 32, 4, 1, 2, 1, 2>, Place<4, 1, 2>>(a, q_grid, st);
-      else if constexpr (N == 1) go<bwd_dq_s3<D, IT, OT, 32, 4, 1, 2, 1, 2>, Place<4, 1, 2>>(a, q_grid, st);
-      else go<bwd_dq_s3<D, IT, OT, 32, 2, 1, 2, 1, 1>, Place<2, 1, 2>>(a, q_grid, st);
+      if constexpr (D == 64) q<4, 2, 2>(a, q_grid, st);
+      else if constexpr (D == 128) q<8, 2, 1>(a, q_grid, st);
+      else if constexpr (N == 1) q<4, 2, 2>(a, q_grid, st);
+      else q<4, 1, 1>(a, q_grid, st);
     }
-  }
-  template <void (*K)(KArgs), class W>
-  static void go(const KArgs& a, int grid, hipStream_t st) {
-    hipLaunchKernelGGL(K, dim3(grid * W::NSUB), dim3(W::NTH), 0, st, a);
   }
 };
 

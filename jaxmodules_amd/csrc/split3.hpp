@@ -36,17 +36,6 @@ struct Frag { u32x4 p[N]; };
 
 using B16 = Elt<bf16_tag>;
 
-// c += a b: the piece products a_i b_j with i + j <= 2, the small ones first
-template <int NA, int NB>
-__device__ __forceinline__ f32x16 mma(const Frag<NA>& a, const Frag<NB>& b, f32x16 c) {
-#pragma unroll
-  for (int s = 2; s >= 0; --s)
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-      if (s - i >= 0 && s - i < NB) c = B16::mfma(a.p[i], b.p[s - i], c);
-  return c;
-}
-
 // The pieces of two values, packed (low half = x0): piece 0 is x rounded, each
 // further one the rest rounded.
 template <int N>
@@ -59,19 +48,6 @@ __device__ __forceinline__ void split2(float x0, float x1, uint32_t (&w)[N]) {
       x1 -= __uint_as_float(w[i] & 0xffff0000u);
     }
   }
-}
-
-// C registers [8 j, 8 j + 8) of a 32x32 result as the B operand of a 16-deep k-step
-__device__ __forceinline__ Frag<3> c_frag(const f32x16& c, int j) {
-  Frag<3> f;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    uint32_t w[3];
-    split2<3>(c[8 * j + 2 * e], c[8 * j + 2 * e + 1], w);
-#pragma unroll
-    for (int p = 0; p < 3; ++p) f.p[p][e] = w[p];
-  }
-  return f;
 }
 
 // 8 consecutive elements as loaded, and their pieces
@@ -119,143 +95,147 @@ struct Raw8<float> {
 template <class T>
 constexpr int elt_bytes() { return Pieces<T>::n == 3 ? 4 : 2; }
 
-// LDS tile of one piece: rows of D 16-bit values, the 16-byte chunk c of row r
-// at chunk c ^ swz(r): ds_read_b128 row reads and ds_read_b64_tr_b16 reads are
-// then free of bank conflicts (as the swizzle of common.hpp, D = 256 like 128:
-// its rows span the banks twice and the low four chunk bits are swizzled).
-template <int D>
-__device__ __forceinline__ int swz3(int r) { return swz<(D == 64 ? 64 : 128)>(r); }
+// f(c, p, off) for this thread's chunks c of ROWS rows from r0 of a [rows, D] tensor:
+// p + off is the start of row r0 + threadIdx / CPR + c RPC (rows past n - 1 are row
+// n - 1: their scores are masked).  p is uniform and off 32 bits a lane, formed anew
+// each time (opaque: hoisted 64-bit addresses, two registers a chunk, spilled the
+// kernels): 64-bit row products were 80 vector instructions a step.  The validated
+// strides (Q, K, V: 128 rows within 2^31 elements) fit; WIDE (dO, not validated) takes
+// 64-bit offsets when its stride needs them.
+template <int D, int ES, int ROWS, int NTH, bool WIDE, class F>
+__device__ __forceinline__ void each_chunk(const char* base, int64_t rs, int r0, int n, F&& f) {
+  constexpr int CPR = D / 8, RPC = NTH / CPR, CH = ROWS / RPC;  // rows a chunk step covers
+  static_assert(NTH % CPR == 0 && ROWS % RPC == 0, "whole rows a step");
+  const int first = min(r0, n - 1), last = n - 1 - first;
+  const char* p = base + ES * ((int64_t)first * rs);
+  const int r = opaque(threadIdx.x / CPR);
+  if (!WIDE || rs < (1 << 24)) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) f(c, p, (uint32_t)(min(r + c * RPC, last) * (ES * (int)rs)));
+  } else {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) f(c, p + ES * ((int64_t)min(r + c * RPC, last) * rs), 0u);
+  }
+}
 
-// ROWS rows of a [rows, D] tensor: loaded into registers, and written to LDS as
-// planes of pieces, by NTH threads.
-template <int D, class T, int ROWS, int NTH>
-struct Stage {
-  static constexpr int CH = ROWS * D / 8 / NTH;
-  static constexpr int NP = Pieces<T>::n;
-  static constexpr int ELTS = NP * ROWS * D;  // LDS elements
-  static_assert(CH >= 1, "one chunk a thread");
-  Raw8<T> v[CH];
-  // rows past n - 1 re-read row n - 1 (their scores are masked)
-  __device__ __forceinline__ void load(const char* base, int64_t rs, int r0, int n) {
+// ---- operand reads pipelined by hand ----------------------------------------------
+// The compiler keeps few LDS reads in flight and waits for each before its MFMAs, so
+// that a step's reads cost their latency one by one.  pipe() issues the reads of step
+// i + PF (asm, in order: common.hpp) ahead of the MFMAs of step i and waits for just
+// those that step i uses.
+
+// a transposed operand as its two 4-row reads leave it (joined after the wait)
+template <int N>
+struct Tr { u32x2 lo[N], up[N]; };
+
+// pieces at LDS byte address x + OFF + i PL
+template <int OFF, int PL, int N>
+__device__ __forceinline__ void rd(Frag<N>& f, uint32_t x) {
+  static_for<N>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    f.p[i] = ds_read128<OFF + i * PL>(x);
+  });
+}
+template <int OFF, int PL, int N>
+__device__ __forceinline__ void rd(Tr<N>& f, uint32_t x0, uint32_t x1) {
+  static_for<N>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    f.lo[i] = ds_read_tr8<OFF + i * PL>(x0);
+    f.up[i] = ds_read_tr8<OFF + i * PL>(x1);
+  });
+}
+template <int N>
+__device__ __forceinline__ void landed(Frag<N>& f) {
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int i = threadIdx.x + NTH * c, r = i / (D / 8), col = i % (D / 8);
-      v[c].load(base + elt_bytes<T>() * ((int64_t)min(r0 + r, n - 1) * rs + 8 * col));
-    }
+  for (int i = 0; i < N; ++i) hold(f.p[i]);
+}
+template <int N>
+__device__ __forceinline__ Frag<N> landed(Tr<N>& t) {
+  Frag<N> f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    hold(t.lo[i]);
+    hold(t.up[i]);
+    f.p[i] = u32x4{t.lo[i][0], t.lo[i][1], t.up[i][0], t.up[i][1]};
   }
-  __device__ __forceinline__ void store(uint16_t* lds) const {
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int i = threadIdx.x + NTH * c, r = i / (D / 8), col = i % (D / 8);
-      const Frag<NP> f = v[c].split();
-#pragma unroll
-      for (int p = 0; p < NP; ++p) *(u32x4*)(lds + p * ROWS * D + r * D + ((col ^ swz3<D>(r)) << 3)) = f.p[p];
+  return f;
+}
+
+// the steps to read ahead: `want`, or as many as lgkmcnt can count (15 reads)
+constexpr int ahead(int want, int rps) { return want * rps <= 15 ? want : 15 / rps; }
+// N steps of RPS reads each, PF steps ahead: rd(step, slot), use(step, slot), both with
+// compile-time arguments, slot = step % (PF + 1)
+template <int N, int PF, int RPS, class R, class U>
+__device__ __forceinline__ void pipe(R&& read, U&& use) {
+  static_for<(PF < N ? PF : N)>([&](auto ic) { read(ic, std::integral_constant<int, decltype(ic)::value % (PF + 1)>{}); });
+  static_for<N>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (i + PF < N)
+      read(std::integral_constant<int, i + PF>{}, std::integral_constant<int, (i + PF) % (PF + 1)>{});
+    lgkm_wait<RPS * (i + PF < N ? PF : N - 1 - i)>();
+    use(ic, std::integral_constant<int, i % (PF + 1)>{});
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+// the n-th piece product (i, j), i + j <= 2, of NA x NB pieces, small ones first (n < products())
+constexpr int products(int na, int nb) {
+  int c = 0;
+  for (int i = 0; i < na; ++i)
+    for (int j = 0; j < nb; ++j) c += i + j <= 2;
+  return c;
+}
+constexpr int product_ij(int na, int nb, int n) {  // 4 i + j
+  for (int s = 2; s >= 0; --s)
+    for (int i = 0; i < na; ++i) {
+      const int j = s - i;
+      if (j < 0 || j >= nb) continue;
+      if (n-- == 0) return 4 * i + j;
     }
-  }
+  return 0;
+}
+__device__ __forceinline__ void mfma1(u32x4 a, u32x4 b, f32x4& c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+// c += a b and c2 += a2 b2, their products in turn (an MFMA that adds to the result of
+// the one before it waits for it)
+template <int NA, int NB, int NC, int ND, class C>
+__device__ __forceinline__ void mma_two(const Frag<NA>& a, const Frag<NB>& b, C& c, const Frag<NC>& a2,
+                                        const Frag<ND>& b2, C& c2) {
+  constexpr int P1 = products(NA, NB), P2 = products(NC, ND);
+  static_for<(P1 > P2 ? P1 : P2)>([&](auto nc) {
+    constexpr int n = decltype(nc)::value;
+    if constexpr (n < P1) {
+      constexpr int ij = product_ij(NA, NB, n);
+      mfma1(a.p[ij / 4], b.p[ij % 4], c);
+    }
+    if constexpr (n < P2) {
+      constexpr int ij = product_ij(NC, ND, n);
+      mfma1(a2.p[ij / 4], b2.p[ij % 4], c2);
+    }
+  });
+}
+
+// Launch slot and part of this workgroup, for kernels that cut a slot of the launch
+// order into NPART workgroups.  The parts of slot s stay on the XCD s % 8 the order
+// means it for (workgroup i runs on XCD i % 8), in the order's sequence.  When all of
+// an XCD's workgroups start at once (up to RES on each of its 32 CUs), every second
+// round of 32 is taken backwards: the order is longest first, so a CU then gets a long
+// and a short row instead of two of the same rank.
+struct Slot {
+  int slot, part;
+  bool ok;
 };
-
-// A operand, k along the columns: row r of the tile, columns 16 kd + 8 hi .. + 7
-template <int D, int NP, int ROWS>
-__device__ __forceinline__ Frag<NP> row_frag(const uint16_t* lds, int r, int kd, int hi) {
-  Frag<NP> f;
-#pragma unroll
-  for (int p = 0; p < NP; ++p)
-    f.p[p] = *(const u32x4*)(lds + p * ROWS * D + r * D + (((2 * kd + hi) ^ swz3<D>(r)) << 3));
-  return f;
-}
-
-// A operand, k along the rows (r0 + 16 ks ..), its 32 rows the columns 32 mt ..: the
-// transposed read of tr_src (common.hpp), k in the order of the C registers
-template <int D, int NP, int ROWS>
-__device__ __forceinline__ Frag<NP> tr_frag(const uint16_t* lds, int r0, int mt, int lane) {
-  Frag<NP> f;
-  const int i = lane & 15, g = lane >> 4, hi = lane >> 5;
-  const int c = 4 * mt + 2 * (g & 1) + ((i & 3) >> 1);
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-#pragma unroll
-    for (int sec = 0; sec < 2; ++sec) {
-      const int r = 4 * hi + 8 * sec + (i >> 2);
-      const uint16_t* src = lds + p * ROWS * D + (r0 + r) * D + ((c ^ swz3<D>(r)) << 3) + 4 * (i & 1);
-      const s16x4 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)src);
-      const u32x2 w = __builtin_bit_cast(u32x2, t);
-      f.p[p][2 * sec] = w[0];
-      f.p[p][2 * sec + 1] = w[1];
-    }
+template <int NPART, int RES>
+__device__ __forceinline__ Slot launch_slot(const KArgs& a) {
+  const int x = blockIdx.x & 7, R = gridDim.x >> 3;
+  int r = blockIdx.x >> 3;
+  if (R <= 32 * RES && (r & 32)) {
+    const int r0 = r & ~31;
+    r = r0 + min(32, R - r0) - 1 - (r & 31);
   }
-  return f;
-}
-
-// 16-bit or float32 output of a row's values, through store_rows (common.hpp), in
-// column blocks of at most 128 so that a wave stages 32 x 128 values at a time
-template <int D, class T>
-__device__ __forceinline__ void put_rows(const f32x16 (&acc)[D / 32], float sc, void* lds, void* out, int64_t row0,
-                                         int64_t rstride, int nrows, int lane) {
-  constexpr int ES = elt_bytes<T>(), DB = D > 128 ? 128 : D;
-  using P = Elt<typename std::conditional<std::is_same<T, float>::value, bf16_tag, T>::type>;
-#pragma unroll
-  for (int c = 0; c < D / DB; ++c)
-    store_rows<DB, ES, true>(*(const f32x16(*)[DB / 32])(&acc[c * (DB / 32)]), sc, lds, out, row0 + c * DB, rstride,
-                             nrows, lane, P::pack2);
-}
-template <int D>
-constexpr int put_bytes() { return 32 * (D > 128 ? 128 : D) * 4; }  // LDS of one wave
-
-// c += the partner wave's c (waves w and w ^ pair, which each formed it over half of
-// d), for N results, through LDS (4 KiB a wave and result): publish, barrier, add.
-template <int N>
-__device__ __forceinline__ void half_put(const f32x16 (&c)[N], float* X, int wave, int lane) {
-#pragma unroll
-  for (int n = 0; n < N; ++n)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *(f32x4*)(X + ((wave * N + n) * 4 + j) * 256 + 4 * lane) =
-          f32x4{c[n][4 * j], c[n][4 * j + 1], c[n][4 * j + 2], c[n][4 * j + 3]};
-}
-template <int N>
-__device__ __forceinline__ void half_add(f32x16 (&c)[N], const float* X, int wave, int lane) {
-#pragma unroll
-  for (int n = 0; n < N; ++n)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4 y = *(const f32x4*)(X + ((wave * N + n) * 4 + j) * 256 + 4 * lane);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[n][4 * j + i] += y[i];
-    }
-}
-
-// Results of the WK waves that shared the same 32 rows (lane = row, registers =
-// columns as in store_rows), summed through LDS and stored: slab [WK][WQ * 32][D]
-// float32; each wave has already scaled its part.
-template <int D, int WQ>
-__device__ __forceinline__ void slab_put(const f32x16 (&acc)[D / 32], float sc, float* slab, int wq, int wk, int lane) {
-  const int r = lane & 31, hi = lane >> 5;
-  float* L = slab + (wk * WQ + wq) * 32 * D + r * D;
-#pragma unroll
-  for (int mt = 0; mt < D / 32; ++mt)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = (32 * mt + 8 * j + 4 * hi) >> 2;
-      *(f32x4*)(L + ((c ^ (r & (D / 4 - 1))) << 2)) =
-          f32x4{acc[mt][4 * j] * sc, acc[mt][4 * j + 1] * sc, acc[mt][4 * j + 2] * sc, acc[mt][4 * j + 3] * sc};
-    }
-}
-template <int D, class T, int WQ, int WK, int NTH>
-__device__ __forceinline__ void slab_sum_store(const float* slab, void* out, int64_t row0, int64_t rstride, int nrows) {
-  using P = Elt<typename std::conditional<std::is_same<T, float>::value, bf16_tag, T>::type>;
-#pragma unroll
-  for (int i = 0; i < 32 * WQ * D / 4 / NTH; ++i) {
-    const int n = threadIdx.x + NTH * i, row = n / (D / 4), c = n % (D / 4);
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < WK; ++k)
-      s += *(const f32x4*)(slab + ((k * WQ * 32 + row) * D) + ((c ^ (row & 31 & (D / 4 - 1))) << 2));
-    if (row < nrows) {
-      char* dst = (char*)out + elt_bytes<T>() * (row0 + (int64_t)row * rstride + 4 * c);
-      if constexpr (std::is_same<T, float>::value) __builtin_nontemporal_store(s, (f32x4*)dst);
-      else __builtin_nontemporal_store(u32x2{P::pack2(s[0], s[1]), P::pack2(s[2], s[3])}, (u32x2*)dst);
-    }
-  }
+  const int s = (r / NPART) * 8 + x;
+  return {s, r % NPART, s < a.n_slots};
 }
 
 // base address of (b, h) in a tensor of element strides s
@@ -263,15 +243,31 @@ __device__ __forceinline__ const char* head_base(const void* p, const int64_t* s
   return (const char*)p + es * ((int64_t)b * s[0] + (int64_t)h * s[2]);
 }
 
-// Sub-blocks of the walk over entries [e0, e1): SPT = 128 / BN per tile.
+// Sub-blocks of the walk over entries [e0, e1): SPT = 128 / BN per tile.  The entries
+// are held 64 at a time, one per lane, and read back at a wave-uniform index: a load
+// per step would cost its latency before the step's own loads can start.
 template <int BN>
 struct Walk {
   static constexpr int SPT = TILE / BN;
   const int* ent;
-  int e0, n;
-  __device__ __forceinline__ Walk(const int* ent_, int e0_, int e1_) : ent(ent_), e0(e0_), n((e1_ - e0_) * SPT) {}
-  __device__ __forceinline__ int first(int s) const { return ent[2 * (e0 + s / SPT)] * TILE + (s % SPT) * BN; }
-  __device__ __forceinline__ int mask(int s) const { return ent[2 * (e0 + s / SPT) + 1]; }
+  int e0, n, base, tile, mk;
+  __device__ __forceinline__ Walk(const int* ent_, int e0_, int e1) : ent(ent_), e0(e0_), n((e1 - e0_) * SPT) {
+    if (n > 0) fill(0);
+  }
+  __device__ __forceinline__ void fill(int i) {
+    base = i;
+    const int e = e0 + min(i + (int)(threadIdx.x & 63), n / SPT - 1);
+    tile = ent[2 * e];
+    mk = ent[2 * e + 1];
+  }
+  __device__ __forceinline__ int at(int i) {  // index of entry i in the window
+    if (i < base || i >= base + 64) fill(i);  // (uniform)
+    return i - base;
+  }
+  __device__ __forceinline__ int first(int s) {
+    return __builtin_amdgcn_readlane(tile, at(s / SPT)) * TILE + (s % SPT) * BN;
+  }
+  __device__ __forceinline__ int mask(int s) { return __builtin_amdgcn_readlane(mk, at(s / SPT)); }
 };
 
 }  // namespace s3
