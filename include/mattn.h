@@ -306,6 +306,24 @@ int mattn_tilemap_bits(const mattn_maskspec* ms, int32_t Lq, int32_t Lk,
                        int32_t n_masks, int32_t write, uint64_t* row_bits,
                        uint64_t* col_bits, int32_t* mismatch, void* stream);
 
+/* Rows [n0][n1][n2] of src_cols elements to rows of dst_cols elements: column c of a
+ * destination row is column c of the source row, or zero for c >= src_cols (source
+ * columns past dst_cols are dropped); converted (round to nearest even) where the types
+ * differ.  Strides are in elements; the columns are contiguous.  Rows may have any
+ * alignment.  The destinations must not overlap anything else the call touches. */
+typedef struct mattn_row_copy {
+  const void* src;
+  void* dst;
+  int64_t src_stride[3], dst_stride[3];
+  int32_t n[3];
+  int32_t src_dtype, dst_dtype;   /* enum mattn_dtype */
+  int32_t src_cols, dst_cols;
+} mattn_row_copy;
+
+/* n (1 to 4) such copies in one launch: the zero-padding of Q, K and V to a kernel head
+ * dimension, and the columns of padded gradients taken back. */
+int mattn_copy_rows(const mattn_row_copy* copies, int32_t n, void* stream);
+
 /* Static text of a status code. */
 const char* mattn_strerror(int status);
 

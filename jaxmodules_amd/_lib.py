@@ -42,7 +42,7 @@ STATUS = {
 EXPORTS = ("mattn_validate", "mattn_workspace_bytes", "mattn_bwd_workspace_bytes", "mattn_fwd_workspace_bytes",
            "mattn_fwd", "mattn_bwd",
            "mattn_bwd_stage", "mattn_strerror", "mattn_abi_version", "mattn_maskspec_validate",
-           "mattn_tilemap_classify", "mattn_tilemap_bits", "mattn_bwd_noalloc")
+           "mattn_tilemap_classify", "mattn_tilemap_bits", "mattn_bwd_noalloc", "mattn_copy_rows")
 SCRATCH_BYTES = 512 << 20  # MATTN_SCRATCH_BYTES
 BWD_PRE, BWD_DKDV, BWD_DQ = 0, 1, 2
 
@@ -81,6 +81,15 @@ class MattnMaskspec(ctypes.Structure):
         ("tab_b", ctypes.c_int32), ("tab_h", ctypes.c_int32), ("tiles", ctypes.c_void_p),
         ("blk_size", ctypes.c_int32), ("blk_left", ctypes.c_int32), ("blk_right", ctypes.c_int32),
         ("blk_nk", ctypes.c_int32), ("res_period", ctypes.c_int32),
+    ]
+
+
+class MattnRowCopy(ctypes.Structure):
+    _fields_ = [
+        ("src", ctypes.c_void_p), ("dst", ctypes.c_void_p),
+        ("src_stride", _I64x3), ("dst_stride", _I64x3), ("n", ctypes.c_int32 * 3),
+        ("src_dtype", ctypes.c_int32), ("dst_dtype", ctypes.c_int32),
+        ("src_cols", ctypes.c_int32), ("dst_cols", ctypes.c_int32),
     ]
 
 
@@ -138,6 +147,8 @@ def load():
         lib.mattn_tilemap_classify.restype = ctypes.c_int
         lib.mattn_tilemap_bits.argtypes = [S, i32, i32, i32, i32, vp, i32, i32, i32, vp, vp, vp, vp]
         lib.mattn_tilemap_bits.restype = ctypes.c_int
+        lib.mattn_copy_rows.argtypes = [ctypes.POINTER(MattnRowCopy), i32, vp]
+        lib.mattn_copy_rows.restype = ctypes.c_int
         lib.mattn_abi_version.argtypes = []
         lib.mattn_abi_version.restype = ctypes.c_int
         if lib.mattn_abi_version() != ABI_VERSION:

@@ -389,6 +389,38 @@ def mattn_forward(q, k, v, tm: bmap.TileMap, scale: float, out_dtype=torch.float
     return o, lse, res
 
 
+# mattn_row_copy as one record (padded to its 8-byte alignment)
+_ROW_COPY = struct.Struct("=2Q6q3i2i2i4x")
+assert _ROW_COPY.size == ctypes.sizeof(_lib.MattnRowCopy)
+
+
+def _copy_rows(pairs):
+    """src's columns into dst for each (src, dst) pair of [B, L, H, *] tensors, zeros
+    where dst is wider, converted where the dtypes differ: one launch."""
+    rec = []
+    for src, dst in pairs:
+        if src.stride(3) != 1:
+            src = src.contiguous()
+        # rows in the order dst has them in memory
+        a, b = (2, 1) if dst.stride(1) < dst.stride(2) else (1, 2)
+        rec.append((src, _ROW_COPY.pack(
+            src.data_ptr(), dst.data_ptr(), src.stride(0), src.stride(a), src.stride(b),
+            dst.stride(0), dst.stride(a), dst.stride(b), dst.shape[0], dst.shape[a], dst.shape[b],
+            _DT[src.dtype], _DT[dst.dtype], src.shape[3], dst.shape[3])))
+    arr = (_lib.MattnRowCopy * len(rec)).from_buffer_copy(b"".join(r for _, r in rec))
+    dev = pairs[0][1].device
+    _lib.check(_lib.load().mattn_copy_rows(arr, len(rec), _stream(dev)), "mattn_copy_rows")
+
+
+def _rows_like(x, cols, heads_major, dtype=None):
+    """An uninitialised [B, L, H, cols] tensor shaped like x, in memory [B, L, H, cols]
+    or, heads_major, [B, H, L, cols]."""
+    B, L, H, _ = x.shape
+    if heads_major:
+        return torch.empty((B, H, L, cols), dtype=dtype or x.dtype, device=x.device).transpose(1, 2)
+    return torch.empty((B, L, H, cols), dtype=dtype or x.dtype, device=x.device)
+
+
 def _workspace(nbytes: int, device):
     """(tensor, 256-byte aligned pointer) of at least nbytes of device memory
     (None, None when nbytes is 0)."""
@@ -470,22 +502,44 @@ class _MaskedAttention(torch.autograd.Function):
     670 us bfloat16 forward at B=4 L=4096 Hq=32 d=128 was the copy).  The backward's
     delta = rowsum(dO * O) then uses the unrounded O: where one key dominates
     a row, dS = P (dP - delta) cancels, and a bfloat16 O would leave its
-    rounding (2^-9 of |V|) in dQ and dK."""
+    rounding (2^-9 of |V|) in dQ and dK.
+
+    Head dimensions between the kernels' are zero-padded here (_copy_rows): Q, K
+    and V in one launch, dO in one (converted to float32 on the way); O's and the
+    gradients' columns are taken back in one each."""
 
     @staticmethod
     def forward(ctx, q, k, v, tm, scale, out_dtype, heads_major=False, precise=False):
         grads = any(ctx.needs_input_grad[:3])
+        d = q.shape[3]
+        D = _kernel_dim(d)
+        if D != d:
+            src = (q, k, v)
+            q, k, v = (_rows_like(x, D, heads_major) for x in src)
+            _copy_rows(list(zip(src, (q, k, v))))
         o, lse, res = mattn_forward(q, k, v, tm, scale, torch.float32 if grads else out_dtype, heads_major,
                                     for_backward=grads, precise=precise)
+        if D != d:
+            out = _rows_like(o, d, heads_major, out_dtype)
+            _copy_rows([(o, out)])
+        else:
+            out = o if o.dtype == out_dtype else o.to(out_dtype)
         if not grads:
-            return o
+            return out
         ctx.save_for_backward(q, k, v, o, lse)
-        ctx.tm, ctx.scale, ctx.res, ctx.precise = tm, scale, res, precise
-        return o if out_dtype == torch.float32 else o.to(out_dtype)
+        ctx.tm, ctx.scale, ctx.res, ctx.precise, ctx.d, ctx.heads_major = tm, scale, res, precise, d, heads_major
+        return out
 
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
+        if ctx.d != q.shape[3]:
+            g = torch.empty_like(o)
+            _copy_rows([(do, g)])
+            padded = mattn_backward(q, k, v, o, lse, g, ctx.tm, ctx.scale, ctx.res, ctx.precise)
+            grads = tuple(_rows_like(x, ctx.d, ctx.heads_major) for x in padded)
+            _copy_rows(list(zip(padded, grads)))
+            return (*grads, None, None, None, None, None)
         do = _ready(do if do.dtype == o.dtype else do.to(o.dtype))
         dq, dk, dv = mattn_backward(q, k, v, o, lse, do, ctx.tm, ctx.scale, ctx.res, ctx.precise)
         return dq, dk, dv, None, None, None, None, None
@@ -497,10 +551,6 @@ def _kernel_dim(d: int) -> int:
         if d <= D:
             return D
     raise NotImplementedError(f"head dimension {d} > 512 is not supported by the HIP kernels")
-
-
-def _pad_dim(x: torch.Tensor, D: int) -> torch.Tensor:
-    return x if x.shape[-1] == D else torch.nn.functional.pad(x, (0, D - x.shape[-1]))
 
 
 PRECISIONS = (None, "default", "highest")
@@ -669,18 +719,15 @@ def _via_map(Q, K, V, *, is_causal=False, kernel_fn=default_kernel, mask_fn=None
     dt = _common_dtype(Q, K, V)
     if plan.squeeze_batch:
         Q, K, V = Q[None], K[None], V[None]
-    D = _kernel_dim(plan.d)
     # softmax(s q.k) == softmax(|s| (-q).k); s == 0 gives uniform weights: q = 0, scale 1
     if scale < 0:
         Q, scale = -Q.to(dt), -scale
     elif scale == 0:
         Q, scale = Q.to(dt) * 0, 1.0
     precise = use_precise(precision, scale, plan.d)
-    q, k, v = _operand(Q, dt, D), _operand(K, dt, D), _operand(V, dt, D)
+    q, k, v = _operand(Q, dt), _operand(K, dt), _operand(V, dt)
     od = _out_dtype(dt, out_dtype)
     out = _MaskedAttention.apply(q, k, v, tm, scale, od, False, precise)
-    if D != plan.d:
-        out = out[..., :plan.d]
     return out[0] if plan.squeeze_batch else out
 
 
@@ -693,11 +740,12 @@ def _common_dtype(q, k, v):
     return dt
 
 
-def _operand(x, dt, D):
-    """x [B, L, H, d] in dtype dt, padded to D columns, as the kernels can load it."""
+def _operand(x, dt):
+    """x [B, L, H, d] in dtype dt as the kernels can load it (any layout where it is
+    padded to a kernel head dimension later)."""
     if x.dtype != dt:
         x = x.to(dt)
-    return _ready(_pad_dim(x, D))
+    return _ready(x) if _kernel_dim(x.shape[3]) == x.shape[3] else x
 
 
 def _out_dtype(dt, out_dtype):
@@ -790,17 +838,15 @@ def flex_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         raise ValueError(f"scale must be finite, got {s}")
     precise = use_precise(precision, s, E)
     tm = _block_mask_tiles(block_mask, B, Hq, Hkv, L, S, _element_head)
-    D = _kernel_dim(E)
     # softmax(s q.k) == softmax(|s| (-q).k); s == 0 gives uniform weights: q = 0, scale 1
     if s < 0:
         query, s = -query.to(dt), -s
     elif s == 0:
         query, s = query.to(dt) * 0, 1.0
     # [B, H, L, E] tensors are strided [B, L, H, E] views for the kernels
-    q, k, v = (_ready(_pad_dim(x if x.dtype == dt else x.to(dt), D).transpose(1, 2)) for x in (query, key, value))
+    q, k, v = (_operand(x.transpose(1, 2), dt) for x in (query, key, value))
     out = _MaskedAttention.apply(q, k, v, tm, s, _out_dtype(dt, out_dtype), True, precise)
-    out = out.transpose(1, 2)
-    return out[..., :E] if D != E else out
+    return out.transpose(1, 2)
 
 
 def flex_attention_slow(query, key, value, score_mod=None, block_mask=None, scale=None,
