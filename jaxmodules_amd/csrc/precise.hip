@@ -13,8 +13,8 @@
 // Bound by the float64 matrix cores: 64 cycles per 16x16x4 product, 128 flop a clock
 // and CU: the rate of the vector float64 FMA, but with the operands of 16 FMAs in one
 // register.  Measured against the compensated SIMT kernels, causal steps at scale 1:
-// [1, 2048, 8, 64] 4.95 -> 0.57 ms, [1, 2048, 8, 128] 10.5 -> 1.06 ms, [1, 1024, 8,
-// 256] 7.06 -> 1.31 ms (the backward's registers spill there: 58 to 87 of them).
+// [1, 2048, 8, 64] 4.95 -> 0.49 ms, [1, 2048, 8, 128] 10.5 -> 1.04 ms, [1, 1024, 8,
+// 256] 7.06 -> 1.17 ms (the backward's registers spill there: 58 to 87 of them).
 //
 // MFMA 16x16x4 layout (lane l, l16 = l % 16, g = l / 16): A row l16, k = g; B column
 // l16, k = g; C column l16, register i row 4 i + g.  Operands along d are read as 4
@@ -70,6 +70,10 @@ __device__ __forceinline__ void get(const char* p, float* x) {
 }
 
 constexpr int WK = 2;
+// workgroups a CU holds (launch_slot): by registers (224 to 256 a wave in dK/dV at D =
+// 64 and the others at 128, twice that beyond), at D = 256 by LDS
+template <int D, bool KV>
+constexpr int resident() { return D == 64 ? (KV ? 2 : 3) : D == 128 && !KV ? 2 : 1; }
 template <int D>
 constexpr int ld() { return D + 4; }  // LDS row stride in floats: 16-byte reads of 16 rows hit 16 bank groups
 
@@ -176,13 +180,14 @@ void fwd_f64(KArgs a) {
   float* Kl = (float*)L;
   float* Vl = Kl + BN * ld<D>();
 
-  const int item = a.q_order[blockIdx.x / NSUB];
+  const Slot slot = launch_slot<NSUB, resident<D, false>()>(a);
+  const int item = slot.ok ? a.q_order[slot.slot] : -1;
   if (item < 0 || item >= a.B * a.Hq * a.nqt) return;  // idle slot (or an entry out of range)
   const int qt = item % a.nqt, bh = item / a.nqt;
   const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.G;
   const int mrow = map_row(a, b, h, a.nqt, qt);
   const Steps<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
-  const int wrow = (blockIdx.x % NSUB) * 16 * WQ;
+  const int wrow = slot.part * 16 * WQ;
   if (qt * TILE + wrow >= a.Lq) return;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wq = wave % WQ, wk = wave / WQ;
@@ -288,13 +293,14 @@ void bwd_dq_f64(KArgs a) {
   float* Kl = (float*)L;
   float* Vl = Kl + BN * ld<D>();
 
-  const int item = a.q_order[blockIdx.x / NSUB];
+  const Slot slot = launch_slot<NSUB, resident<D, false>()>(a);
+  const int item = slot.ok ? a.q_order[slot.slot] : -1;
   if (item < 0 || item >= a.B * a.Hq * a.nqt) return;  // idle slot (or an entry out of range)
   const int qt = item % a.nqt, bh = item / a.nqt;
   const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.G;
   const int mrow = map_row(a, b, h, a.nqt, qt);
   const Steps<BN> walk(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1]);
-  const int wrow = (blockIdx.x % NSUB) * 16 * WQ;
+  const int wrow = slot.part * 16 * WQ;
   if (qt * TILE + wrow >= a.Lq) return;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wq = wave % WQ, wk = wave / WQ;
@@ -365,11 +371,12 @@ void bwd_dkdv_f64(KArgs a) {
   float* Ql = (float*)L;
   float* Gl = Ql + BN * ld<D>();
 
-  const int item = a.kv_order[blockIdx.x / NSUB];
+  const Slot slot = launch_slot<NSUB, resident<D, true>()>(a);
+  const int item = slot.ok ? a.kv_order[slot.slot] : -1;
   if (item < 0 || item >= a.B * a.Hkv * a.nkt) return;  // idle slot (or an entry out of range)
   const int kt = item % a.nkt, bh = item / a.nkt;
   const int hk = bh % a.Hkv, b = bh / a.Hkv;
-  const int wrow = (blockIdx.x % NSUB) * 16 * WQ;
+  const int wrow = slot.part * 16 * WQ;
   if (kt * TILE + wrow >= a.Lk) return;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wq = wave % WQ, wk = wave / WQ;
@@ -457,14 +464,19 @@ struct F64 {
   static constexpr int WQ = 2, NT = D == 256 ? 1 : 2, MINW = D == 64 ? 2 : 1;
   static constexpr int NSUB = TILE / (16 * WQ), NTH = 64 * WQ * WK;
   static void fwd(const KArgs& a, int grid, hipStream_t st) {
-    hipLaunchKernelGGL((fwd_f64<D, IT, OT, WQ, NT, MINW>), dim3(grid * NSUB), dim3(NTH), 0, st, a);
+    go<fwd_f64<D, IT, OT, WQ, NT, MINW>>(a, grid, st);
   }
   static void bwd(const KArgs& a, int stage, int q_grid, int kv_grid, hipStream_t st) {
     if (stage == MATTN_BWD_DKDV)
-      hipLaunchKernelGGL((bwd_dkdv_f64<D, IT, OT, WQ, 1, MINW>), dim3(kv_grid * NSUB), dim3(NTH), 0, st, a);
+      go<bwd_dkdv_f64<D, IT, OT, WQ, 1, MINW>>(a, kv_grid, st);
     else if (stage == MATTN_BWD_DQ)
-      hipLaunchKernelGGL((bwd_dq_f64<D, IT, OT, WQ, NT, MINW>), dim3(q_grid * NSUB), dim3(NTH), 0, st, a);
+      go<bwd_dq_f64<D, IT, OT, WQ, NT, MINW>>(a, q_grid, st);
     // MATTN_BWD_PRE: nothing (delta is formed where it is used)
+  }
+  template <void (*K)(KArgs)>
+  static void go(KArgs a, int grid, hipStream_t st) {
+    a.n_slots = grid;
+    hipLaunchKernelGGL(K, dim3((grid + 7) / 8 * 8 * NSUB), dim3(NTH), 0, st, a);
   }
 };
 
