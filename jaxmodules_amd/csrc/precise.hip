@@ -13,8 +13,8 @@
 // Bound by the float64 matrix cores: 64 cycles per 16x16x4 product, 128 flop a clock
 // and CU: the rate of the vector float64 FMA, but with the operands of 16 FMAs in one
 // register.  Measured against the compensated SIMT kernels, causal steps at scale 1:
-// [1, 2048, 8, 64] 4.95 -> 0.49 ms, [1, 2048, 8, 128] 10.5 -> 1.04 ms, [1, 1024, 8,
-// 256] 7.06 -> 1.17 ms (the backward's registers spill there: 58 to 87 of them).
+// [1, 2048, 8, 64] 4.95 -> 0.47 ms, [1, 2048, 8, 128] 10.5 -> 0.91 ms, [1, 1024, 8,
+// 256] 7.06 -> 1.09 ms (the backward's registers spill there: 58 to 87 of them).
 //
 // MFMA 16x16x4 layout (lane l, l16 = l % 16, g = l / 16): A row l16, k = g; B column
 // l16, k = g; C column l16, register i row 4 i + g.  Operands along d are read as 4
@@ -77,18 +77,30 @@ constexpr int resident() { return D == 64 ? (KV ? 2 : 3) : D == 128 && !KV ? 2 :
 template <int D>
 constexpr int ld() { return D + 4; }  // LDS row stride in floats: 16-byte reads of 16 rows hit 16 bank groups
 
-// ROWS rows of a tensor as float32 rows in LDS (rows past n - 1 re-read row n - 1)
+// ROWS rows of a tensor as float32 rows in LDS (rows past n - 1 re-read row n - 1),
+// through registers: loaded one step ahead where they are few (HELD)
 template <int D, class T, int ROWS, int NTH>
-__device__ __forceinline__ void stage32(float* dst, const char* base, int64_t rs, int r0, int n) {
-#pragma unroll
-  for (int c = 0; c < ROWS * D / 8 / NTH; ++c) {
-    const int i = threadIdx.x + NTH * c, r = i / (D / 8), col = 8 * (i % (D / 8));
-    float x[8];
-    get<T, 8>(base + elt_bytes<T>() * ((int64_t)min(r0 + r, n - 1) * rs + col), x);
-    *(f32x4*)(dst + r * ld<D>() + col) = f32x4{x[0], x[1], x[2], x[3]};
-    *(f32x4*)(dst + r * ld<D>() + col + 4) = f32x4{x[4], x[5], x[6], x[7]};
+struct Rows32 {
+  static constexpr int CH = ROWS * D / 8 / NTH;
+  static constexpr bool HELD = D == 64;
+  Raw8<T> v[CH];
+  __device__ __forceinline__ void load(const char* base, int64_t rs, int r0, int n) {
+    constexpr int ES = elt_bytes<T>();
+    each_chunk<D, ES, ROWS, NTH, false>(base, rs, r0, n, [&](int c, const char* p, uint32_t off) {
+      v[c].load(p + (off + ES * 8 * (threadIdx.x % (D / 8))));
+    });
   }
-}
+  __device__ __forceinline__ void store(float* dst) const {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int i = threadIdx.x + NTH * c, r = i / (D / 8), col = 8 * (i % (D / 8));
+      float x[8];
+      v[c].floats(x);
+      *(f32x4*)(dst + r * ld<D>() + col) = f32x4{x[0], x[1], x[2], x[3]};
+      *(f32x4*)(dst + r * ld<D>() + col + 4) = f32x4{x[4], x[5], x[6], x[7]};
+    }
+  }
+};
 
 // this lane's D / 4 values of row r: x[4 j + e] = column 16 j + 4 g + e
 template <int D, class T>
@@ -204,11 +216,26 @@ void fwd_f64(KArgs a) {
   double l = 0.;
   const double c2 = (double)a.scale_log2;
 
+  using R = Rows32<D, IT, BN, NTH>;
+  R ks, vs;
+  auto load = [&](int k0) {
+    ks.load(kb, a.ks[1], k0, a.Lk);
+    vs.load(vb, a.vs[1], k0, a.Lk);
+  };
+  if (R::HELD && walk.n > 0) load(walk.first(0));
   for (int s = 0; s < walk.n; ++s) {
     const int key0 = walk.first(s), mask = walk.mask(s);
     __syncthreads();
-    stage32<D, IT, BN, NTH>(Kl, kb, a.ks[1], key0, a.Lk);
-    stage32<D, IT, BN, NTH>(Vl, vb, a.vs[1], key0, a.Lk);
+    if constexpr (R::HELD) {
+      ks.store(Kl);
+      vs.store(Vl);
+      if (s + 1 < walk.n) load(walk.first(s + 1));
+    } else {
+      ks.load(kb, a.ks[1], key0, a.Lk);
+      ks.store(Kl);
+      vs.load(vb, a.vs[1], key0, a.Lk);
+      vs.store(Vl);
+    }
     __syncthreads();
     uint32_t w[NT];
     bool any = false;
@@ -330,11 +357,26 @@ void bwd_dq_f64(KArgs a) {
 #pragma unroll
   for (int i = 0; i < D / 16; ++i) acc[i] = f64x4{};
 
+  using R = Rows32<D, IT, BN, NTH>;
+  R ks, vs;
+  auto load = [&](int k0) {
+    ks.load(kb, a.ks[1], k0, a.Lk);
+    vs.load(vb, a.vs[1], k0, a.Lk);
+  };
+  if (R::HELD && walk.n > 0) load(walk.first(0));
   for (int s = 0; s < walk.n; ++s) {
     const int key0 = walk.first(s), mask = walk.mask(s);
     __syncthreads();
-    stage32<D, IT, BN, NTH>(Kl, kb, a.ks[1], key0, a.Lk);
-    stage32<D, IT, BN, NTH>(Vl, vb, a.vs[1], key0, a.Lk);
+    if constexpr (R::HELD) {
+      ks.store(Kl);
+      vs.store(Vl);
+      if (s + 1 < walk.n) load(walk.first(s + 1));
+    } else {
+      ks.load(kb, a.ks[1], key0, a.Lk);
+      ks.store(Kl);
+      vs.load(vb, a.vs[1], key0, a.Lk);
+      vs.store(Vl);
+    }
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -401,7 +443,11 @@ void bwd_dkdv_f64(KArgs a) {
     for (int s = 0; s < walk.n; ++s) {
       const int q0 = walk.first(s), mask = walk.mask(s);
       __syncthreads();
-      stage32<D, IT, BN, NTH>(Ql, qb, a.qs[1], q0, a.Lq);
+      {
+        Rows32<D, IT, BN, NTH> qr;
+        qr.load(qb, a.qs[1], q0, a.Lq);
+        qr.store(Ql);
+      }
       // dO rows, and delta = dO . (O + o_lo) by the D / 8 threads of a row
 #pragma unroll
       for (int c = 0; c < BN * D / 8 / NTH; ++c) {
@@ -461,16 +507,16 @@ void bwd_dkdv_f64(KArgs a) {
 
 template <int D, class IT, class OT>
 struct F64 {
-  static constexpr int WQ = 2, NT = D == 256 ? 1 : 2, MINW = D == 64 ? 2 : 1;
+  static constexpr int WQ = 2, NT = D == 256 ? 1 : 2, MINW = D == 64 ? 2 : 1, MINF = D <= 128 ? 2 : 1;
   static constexpr int NSUB = TILE / (16 * WQ), NTH = 64 * WQ * WK;
   static void fwd(const KArgs& a, int grid, hipStream_t st) {
-    go<fwd_f64<D, IT, OT, WQ, NT, MINW>>(a, grid, st);
+    go<fwd_f64<D, IT, OT, WQ, NT, MINF>>(a, grid, st);
   }
   static void bwd(const KArgs& a, int stage, int q_grid, int kv_grid, hipStream_t st) {
     if (stage == MATTN_BWD_DKDV)
       go<bwd_dkdv_f64<D, IT, OT, WQ, 1, MINW>>(a, kv_grid, st);
     else if (stage == MATTN_BWD_DQ)
-      go<bwd_dq_f64<D, IT, OT, WQ, NT, MINW>>(a, q_grid, st);
+      go<bwd_dq_f64<D, IT, OT, WQ, NT, MINF>>(a, q_grid, st);
     // MATTN_BWD_PRE: nothing (delta is formed where it is used)
   }
   template <void (*K)(KArgs)>

@@ -55,6 +55,10 @@ template <class T>
 struct Raw8 {
   u32x4 x;
   __device__ __forceinline__ void load(const char* p) { x = *(const u32x4*)p; }
+  __device__ __forceinline__ void floats(float* f) const {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = Elt<T>::to_f32(elt16(x, e));
+  }
   __device__ __forceinline__ Frag<Pieces<T>::n> split() const {
     Frag<Pieces<T>::n> f;
     if constexpr (Pieces<T>::n == 1) {
@@ -77,6 +81,13 @@ struct Raw8<float> {
   __device__ __forceinline__ void load(const char* p) {
     x = *(const f32x4*)p;
     y = *(const f32x4*)(p + 16);
+  }
+  __device__ __forceinline__ void floats(float* f) const {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[e] = x[e];
+      f[4 + e] = y[e];
+    }
   }
   __device__ __forceinline__ Frag<3> split() const {
     Frag<3> f;
