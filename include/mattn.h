@@ -41,7 +41,8 @@
 extern "C" {
 #endif
 
-/* Element types.  Q, K, V, dQ, dK, dV share `dtype`; O and dO share `o_dtype`
+/* Element types.  Q, K, V, dQ, dK, dV share `dtype`; O and (without MATTN_DO_16)
+ * dO share `o_dtype`
  * (the reference returns float32 O for bfloat16 inputs, attention.py:173). */
 enum mattn_dtype { MATTN_BF16 = 0, MATTN_F16 = 1, MATTN_F32 = 2 };
 
@@ -92,6 +93,10 @@ enum mattn_status {
  * the stored lse and O round off (one float per query row and per element of
  * O), which the backward reads. */
 #define MATTN_PRECISE 4
+/* mattn_problem.flags: dO has the inputs' 16-bit dtype (do_stride counts its
+ * elements) though O is float32: the gradient of a 16-bit copy of O, read as it is.
+ * 16-bit inputs, D <= 256, without MATTN_PRECISE (else MATTN_ERR_DTYPE). */
+#define MATTN_DO_16 16
 
 /* Tile size of the block map, in queries x keys. */
 #define MATTN_TILE_Q 128
@@ -103,7 +108,8 @@ typedef struct mattn_problem {
   int32_t o_dtype;   /* enum mattn_dtype of O and dO: dtype, or MATTN_F32  */
   float scale;       /* softmax scale; the reference's default_kernel uses
                         1/sqrt(D) (attention.py:39-50)                     */
-  int32_t flags;     /* MATTN_FWD_FOR_BWD | MATTN_BWD_DS | MATTN_PRECISE   */
+  int32_t flags;     /* MATTN_FWD_FOR_BWD | MATTN_BWD_DS | MATTN_PRECISE
+                        | MATTN_DO_16                                      */
   /* element strides {batch, sequence, head}; D is contiguous */
   int64_t q_stride[3], k_stride[3], v_stride[3], o_stride[3];
   int64_t do_stride[3], dq_stride[3], dk_stride[3], dv_stride[3];
@@ -200,7 +206,7 @@ int mattn_fwd(const mattn_problem* p, const mattn_blockmap* bm,
               void* o, float* lse, void* residual, void* stream);
 
 /* Backward (replaces the custom_vjp bwd rule, attention.py:266-342).
- *   do_       : upstream gradient, [B, Lq, Hq, D] of o_dtype
+ *   do_       : upstream gradient, [B, Lq, Hq, D] of o_dtype (MATTN_DO_16: of dtype)
  *   o, lse    : the forward's outputs
  *   residual  : the forward's residual buffer (16-bit inputs at D <= 128;
  *               that forward ran with MATTN_FWD_FOR_BWD, which p->flags must

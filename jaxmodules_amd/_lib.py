@@ -19,6 +19,7 @@ MATTN_BF16, MATTN_F16, MATTN_F32 = 0, 1, 2
 MATTN_FWD_FOR_BWD = 1
 MATTN_BWD_DS = 2
 MATTN_PRECISE = 4
+MATTN_DO_16 = 16
 TILE_Q = TILE_K = 128
 ABI_VERSION = 8
 

@@ -468,14 +468,16 @@ def bwd_flags(p, bm) -> int:
 
 def mattn_backward(q, k, v, o, lse, do, tm: bmap.TileMap, scale: float, res=None, precise: bool = False):
     """(dQ, dK, dV) via mattn_bwd; ``res`` is mattn_forward's residual (run
-    with for_backward=True and the same ``precise``)."""
+    with for_backward=True and the same ``precise``).  ``do`` has o's dtype, or q's
+    beside a float32 o (MATTN_DO_16)."""
     lib = _lib.load()
     _check_map(tm, q, k)
     dq = torch.empty_like(q)
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)
     p = _problem(q, k, v, o, scale, do=do, dq=dq, dk=dk, dv=dv)
-    p.flags = _lib.MATTN_FWD_FOR_BWD | (_lib.MATTN_PRECISE if precise else 0)
+    p.flags = (_lib.MATTN_FWD_FOR_BWD | (_lib.MATTN_PRECISE if precise else 0)
+               | (_lib.MATTN_DO_16 if do.dtype != o.dtype else 0))
     bm = device_blockmap(tm, q.device)
     p.flags = bwd_flags(p, bm)
     pr, br = ctypes.byref(p), ctypes.byref(bm)
@@ -533,14 +535,17 @@ class _MaskedAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
-        if ctx.d != q.shape[3]:
-            g = torch.empty_like(o)
+        # a 16-bit dO is read as it is where the kernels take it (MATTN_DO_16)
+        D = q.shape[3]
+        gt = do.dtype if do.dtype == q.dtype and D <= 256 and not ctx.precise else o.dtype
+        if ctx.d != D:
+            g = torch.empty_like(o, dtype=gt)
             _copy_rows([(do, g)])
             padded = mattn_backward(q, k, v, o, lse, g, ctx.tm, ctx.scale, ctx.res, ctx.precise)
             grads = tuple(_rows_like(x, ctx.d, ctx.heads_major) for x in padded)
             _copy_rows(list(zip(padded, grads)))
             return (*grads, None, None, None, None, None)
-        do = _ready(do if do.dtype == o.dtype else do.to(o.dtype))
+        do = _ready(do if do.dtype == gt else do.to(gt))
         dq, dk, dv = mattn_backward(q, k, v, o, lse, do, ctx.tm, ctx.scale, ctx.res, ctx.precise)
         return dq, dk, dv, None, None, None, None, None
 

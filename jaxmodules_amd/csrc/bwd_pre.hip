@@ -59,25 +59,25 @@ __device__ __forceinline__ void load_vals(const void* base, int64_t off, float* 
   }
 }
 
-// A row's values held by its 4 threads in 16-byte chunks: thread p holds
-// chunks p + 4 j (CS values each: 4 float32 or 8 16-bit values), so that the
-// row's 4 threads read 64 contiguous bytes per access.  g[CS j + e] is value
-// CS (p + 4 j) + e of the row.
-template <int D, class Tag, bool F32>
+// A row's values held by its 4 threads in chunks of CS values (dO's 16-byte
+// chunks: 4 float32 or 8 16-bit values): thread p holds chunks p + 4 j, so that the
+// row's 4 threads read 64 contiguous bytes of dO per access (128 of a float32 O
+// beside a 16-bit dO).  g[CS j + e] is value CS (p + 4 j) + e of the row.
+template <int D, class Tag, bool F32, int CS>
 __device__ __forceinline__ void load_row(const void* base, int64_t row_off, int part, float* g) {
-  constexpr int CS = F32 ? 4 : 8, NJ = D / 4 / CS;
+  constexpr int NJ = D / 4 / CS;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) load_vals<CS, Tag, F32>(base, row_off + CS * (part + 4 * j), g + CS * j);
 }
 
 // One workgroup of 512 threads per (b, head, 128-row query tile), 4 threads
 // per row.  Rows past Lq (up to the tile's end) are written as zeros.
-template <int D, class Tag, bool O_F32>
+template <int D, class Tag, bool O_F32, bool G_F32>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512)))
 void bwd_pre(KArgs a) {
   using H = Elt<f16_tag>;
   constexpr int PER = D / 4;
-  constexpr int CS = O_F32 ? 4 : 8;  // values per 16-byte input chunk
+  constexpr int CS = G_F32 ? 4 : 8;  // values per 16-byte chunk of dO
   __shared__ f32x2 red[8];
   // Launch position -> (b, h, qt).  When a row of O holds all heads ([B, L, H,
   // D]), the head runs fastest, so that the workgroups running together read
@@ -102,8 +102,8 @@ void bwd_pre(KArgs a) {
 #pragma unroll
   for (int i = 0; i < PER; ++i) o[i] = g[i] = 0.f;
   if (live) {
-    load_row<D, Tag, O_F32>(a.o, (int64_t)b * a.os[0] + (int64_t)q * a.os[1] + (int64_t)h * a.os[2], part, o);
-    load_row<D, Tag, O_F32>(a.dO, (int64_t)b * a.dos[0] + (int64_t)q * a.dos[1] + (int64_t)h * a.dos[2], part, g);
+    load_row<D, Tag, O_F32, CS>(a.o, (int64_t)b * a.os[0] + (int64_t)q * a.os[1] + (int64_t)h * a.os[2], part, o);
+    load_row<D, Tag, G_F32, CS>(a.dO, (int64_t)b * a.dos[0] + (int64_t)q * a.dos[1] + (int64_t)h * a.dos[2], part, g);
   }
   float mx = 0.f;
 #pragma unroll
@@ -187,9 +187,14 @@ void bwd_pre(KArgs a) {
 hipError_t launch_dq(const KArgs& a, int D, int dtype, int grid, hipStream_t st);
 hipError_t launch_dkdv(const KArgs& a, int D, int dtype, int grid, hipStream_t st);
 
-template <int D, class Tag, bool OF32>
-static void launch_pre_16(const KArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((bwd_pre<D, Tag, OF32>), dim3(a.B * a.Hq * a.nqt), dim3(512), 0, st, a);
+// (a 16-bit dO beside a float32 O, MATTN_DO_16, is read as it is: converting it first
+// was a launch, a float32 copy of it and 4 instead of 2 bytes an element here)
+template <int D, class Tag>
+static void launch_pre_16(const KArgs& a, bool of32, hipStream_t st) {
+  const dim3 grid(a.B * a.Hq * a.nqt), block(512);
+  if (!of32) hipLaunchKernelGGL((bwd_pre<D, Tag, false, false>), grid, block, 0, st, a);
+  else if (a.do16) hipLaunchKernelGGL((bwd_pre<D, Tag, true, false>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((bwd_pre<D, Tag, true, true>), grid, block, 0, st, a);
 }
 
 hipError_t launch_bwd_simt(const KArgs& a, int D, int dtype, int o_dtype, int stage, int q_grid, int kv_grid,
@@ -202,11 +207,11 @@ hipError_t launch_bwd_stage(const KArgs& a, int D, int dtype, int o_dtype, bool 
   if (stage == MATTN_BWD_DKDV) return launch_dkdv(a, D, dtype, kv_grid, st);
   if (stage == MATTN_BWD_DQ) return launch_dq(a, D, dtype, q_grid, st);
   if (dtype == MATTN_BF16) {
-    if (D == 64) { if (of32) launch_pre_16<64, bf16_tag, true>(a, st); else launch_pre_16<64, bf16_tag, false>(a, st); }
-    else { if (of32) launch_pre_16<128, bf16_tag, true>(a, st); else launch_pre_16<128, bf16_tag, false>(a, st); }
+    if (D == 64) launch_pre_16<64, bf16_tag>(a, of32, st);
+    else launch_pre_16<128, bf16_tag>(a, of32, st);
   } else {
-    if (D == 64) { if (of32) launch_pre_16<64, f16_tag, true>(a, st); else launch_pre_16<64, f16_tag, false>(a, st); }
-    else { if (of32) launch_pre_16<128, f16_tag, true>(a, st); else launch_pre_16<128, f16_tag, false>(a, st); }
+    if (D == 64) launch_pre_16<64, f16_tag>(a, of32, st);
+    else launch_pre_16<128, f16_tag>(a, of32, st);
   }
   return hipGetLastError();
 }

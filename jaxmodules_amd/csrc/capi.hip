@@ -157,6 +157,7 @@ KArgs make_args(const mattn_problem* p, const mattn_blockmap* bm) {
   a.kv_order = bm->kv_order;
   a.kv_desc = bm->kv_desc;
   a.precise = (p->flags & MATTN_PRECISE) ? 1 : 0;
+  a.do16 = (p->flags & MATTN_DO_16) && p->o_dtype == MATTN_F32;
   return a;
 }
 
@@ -194,11 +195,13 @@ int mattn_validate(const mattn_problem* p, const mattn_blockmap* bm) {
   if (p->dtype != MATTN_BF16 && p->dtype != MATTN_F16 && p->dtype != MATTN_F32) return MATTN_ERR_DTYPE;
   if (p->o_dtype != p->dtype && p->o_dtype != MATTN_F32) return MATTN_ERR_DTYPE;
   if (!(p->scale > 0.f) || isinf(p->scale)) return MATTN_ERR_SHAPE;  // positive, finite
-  if (p->flags & ~(MATTN_FWD_FOR_BWD | MATTN_BWD_DS | MATTN_PRECISE)) return MATTN_ERR_SHAPE;
+  if (p->flags & ~(MATTN_FWD_FOR_BWD | MATTN_BWD_DS | MATTN_PRECISE | MATTN_DO_16)) return MATTN_ERR_SHAPE;
+  const bool do16 = p->flags & MATTN_DO_16;
+  if (do16 && (p->dtype == MATTN_F32 || p->D > 256 || (p->flags & MATTN_PRECISE))) return MATTN_ERR_DTYPE;
   const int es = elem_size(p->dtype), eo = elem_size(p->o_dtype);
   if (!strides_ok(p->q_stride, es) || !strides_ok(p->k_stride, es) || !strides_ok(p->v_stride, es) ||
       !strides_ok(p->dq_stride, es) || !strides_ok(p->dk_stride, es) ||
-      !strides_ok(p->dv_stride, es) || !strides_ok(p->o_stride, eo) || !strides_ok(p->do_stride, eo))
+      !strides_ok(p->dv_stride, es) || !strides_ok(p->o_stride, eo) || !strides_ok(p->do_stride, do16 ? es : eo))
     return MATTN_ERR_STRIDE;
   const int64_t nqt = cdiv(p->Lq, MATTN_TILE_Q), nkt = cdiv(p->Lk, MATTN_TILE_K);
   if ((int64_t)p->B * p->Hq * p->Lq >= (1ll << 31) || (int64_t)p->B * p->Hkv * p->Lk >= (1ll << 31) || (int64_t)p->B * p->Hq * nqt >= (1ll << 31) || (int64_t)p->B * p->Hkv * nkt >= (1ll << 31) ||

@@ -96,6 +96,7 @@ struct KArgs {
   int ds_nnz;
   int n_slots;         // slots of the launch order the kernel walks (kernels that cut a slot into parts)
   const int* kv_desc;  // per dK/dV launch slot: { item, g, e, e_end, n_sub, qt, mask, row }
+  int do16;            // MATTN_DO_16: dO has the inputs' 16-bit type beside a float32 O
   int precise;         // MATTN_PRECISE: float64 (D = 512: compensated) scores and sums
   float* lse_lo;       // MATTN_PRECISE (forward residual): [B, Hq, Lq], (m + log2 l) - lse
   float* o_lo;         // MATTN_PRECISE (forward residual): [B, Hq, Lq, D], exact O - stored O

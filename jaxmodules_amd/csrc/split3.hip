@@ -549,7 +549,7 @@ void bwd_dkdv_s3(KArgs a) {
 
 // delta = rowsum(dO * O), summed in float64: D / 8 threads a row, the rows in the
 // order of memory (head fastest where a row of O holds all heads)
-template <int D, class OT>
+template <int D, class OT, class GT>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256)))
 void delta_s3(KArgs a) {
   constexpr int TPR = D / 8;
@@ -567,20 +567,17 @@ void delta_s3(KArgs a) {
     b = i / ((int64_t)a.Hq * a.Lq);
   }
   const char* o = head_base(a.o, a.os, b, h, elt_bytes<OT>()) + elt_bytes<OT>() * ((int64_t)q * a.os[1] + 8 * part);
-  const char* g = head_base(a.dO, a.dos, b, h, elt_bytes<OT>()) + elt_bytes<OT>() * ((int64_t)q * a.dos[1] + 8 * part);
+  const char* g = head_base(a.dO, a.dos, b, h, elt_bytes<GT>()) + elt_bytes<GT>() * ((int64_t)q * a.dos[1] + 8 * part);
+  Raw8<OT> ro;
+  Raw8<GT> rg;
+  ro.load(o);
+  rg.load(g);
+  float x[8], y[8];
+  ro.floats(x);
+  rg.floats(y);
   double s = 0.;
-  if constexpr (std::is_same<OT, float>::value) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const f32x4 x = *(const f32x4*)(o + 16 * j), y = *(const f32x4*)(g + 16 * j);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s += (double)x[e] * (double)y[e];
-    }
-  } else {
-    const u32x4 x = *(const u32x4*)o, y = *(const u32x4*)g;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s += (double)Elt<OT>::to_f32(elt16(x, e)) * (double)Elt<OT>::to_f32(elt16(y, e));
-  }
+  for (int e = 0; e < 8; ++e) s += (double)x[e] * (double)y[e];
 #pragma unroll
   for (int m = 1; m < TPR; m <<= 1) s += __shfl_xor(s, m);
   if (part == 0) a.delta[((int64_t)b * a.Hq + h) * a.Lq + q] = (float)s;
@@ -600,7 +597,7 @@ void go(KArgs a, int grid, hipStream_t st) {
 // waves a SIMD where that spills nothing inside the walks, else one (a spill's reload
 // also waits for the loads in flight: at D = 128 the float32 step took 697 us with 41
 // spilled registers in dK/dV, 600 at one wave a SIMD).
-template <int D, class IT, class OT>
+template <int D, class IT, class OT, class GT = OT>
 struct S3 {
   static constexpr int N = Pieces<IT>::n;
   template <int NW, int MINW, int RES>
@@ -609,11 +606,11 @@ struct S3 {
   }
   template <int NW, int MINW, int RES>
   static void q(const KArgs& a, int grid, hipStream_t st) {
-    go<TILE / (16 * NW), NW, bwd_dq_s3<D, IT, OT, NW, MINW, RES>>(a, grid, st);
+    go<TILE / (16 * NW), NW, bwd_dq_s3<D, IT, GT, NW, MINW, RES>>(a, grid, st);
   }
   template <int NW, int MINW, int RES>
   static void kv(const KArgs& a, int grid, hipStream_t st) {
-    go<(D == 256 ? 2 : 1) * TILE / (16 * NW), NW, bwd_dkdv_s3<D, IT, OT, NW, MINW, RES>>(a, grid, st);
+    go<(D == 256 ? 2 : 1) * TILE / (16 * NW), NW, bwd_dkdv_s3<D, IT, GT, NW, MINW, RES>>(a, grid, st);
   }
   static void fwd(const KArgs& a, int grid, hipStream_t st) {
     if constexpr (D == 64) f<4, 3, 3>(a, grid, st);
@@ -624,7 +621,7 @@ struct S3 {
   static void bwd(const KArgs& a, int stage, int q_grid, int kv_grid, hipStream_t st) {
     if (stage == MATTN_BWD_PRE) {
       const int64_t threads = (int64_t)a.B * a.Hq * a.Lq * (D / 8);
-      hipLaunchKernelGGL((delta_s3<D, OT>), dim3((threads + 255) / 256), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((delta_s3<D, OT, GT>), dim3((threads + 255) / 256), dim3(256), 0, st, a);
     } else if (stage == MATTN_BWD_DKDV) {
       if constexpr (D == 64) kv<4, 2, 2>(a, kv_grid, st);
       else if constexpr (D == 128) kv<4, 1, 1>(a, kv_grid, st);
@@ -639,17 +636,25 @@ struct S3 {
   }
 };
 
+// (16-bit inputs: the same-dtype O of the C interface, a float32 O, and a float32 O
+// whose gradient is 16-bit)
+template <class Tag, class F>
+void dispatch16(bool of32, bool do16, F&& f) {
+  if (!of32) f(S3<256, Tag, Tag>{});
+  else if (do16) f(S3<256, Tag, float, Tag>{});
+  else f(S3<256, Tag, float>{});
+}
 template <class F>
-hipError_t dispatch(int D, int dtype, int o_dtype, F&& f) {
+hipError_t dispatch(const KArgs& a, int D, int dtype, int o_dtype, F&& f) {
   const bool of32 = o_dtype == MATTN_F32;
   if (dtype == MATTN_F32) {
     if (D == 64) f(S3<64, float, float>{});
     else if (D == 128) f(S3<128, float, float>{});
     else f(S3<256, float, float>{});
   } else if (dtype == MATTN_BF16) {
-    if (of32) f(S3<256, bf16_tag, float>{}); else f(S3<256, bf16_tag, bf16_tag>{});
+    dispatch16<bf16_tag>(of32, a.do16, f);
   } else {
-    if (of32) f(S3<256, f16_tag, float>{}); else f(S3<256, f16_tag, f16_tag>{});
+    dispatch16<f16_tag>(of32, a.do16, f);
   }
   return hipGetLastError();
 }
@@ -661,12 +666,12 @@ bool s3_path(int D, int dtype, bool precise) {
 }
 
 hipError_t launch_fwd_s3(const KArgs& a, int D, int dtype, int o_dtype, int grid, hipStream_t st) {
-  return dispatch(D, dtype, o_dtype, [&](auto s) { decltype(s)::fwd(a, grid, st); });
+  return dispatch(a, D, dtype, o_dtype, [&](auto s) { decltype(s)::fwd(a, grid, st); });
 }
 
 hipError_t launch_bwd_s3(const KArgs& a, int D, int dtype, int o_dtype, int stage, int q_grid, int kv_grid,
                          hipStream_t st) {
-  return dispatch(D, dtype, o_dtype, [&](auto s) { decltype(s)::bwd(a, stage, q_grid, kv_grid, st); });
+  return dispatch(a, D, dtype, o_dtype, [&](auto s) { decltype(s)::bwd(a, stage, q_grid, kv_grid, st); });
 }
 
 }  // namespace mattn
