@@ -335,10 +335,12 @@ _DT = {torch.bfloat16: _lib.MATTN_BF16, torch.float16: _lib.MATTN_F16, torch.flo
 
 
 def _ready(t: torch.Tensor) -> torch.Tensor:
-    """d contiguous and 16-byte aligned strides/base, as the kernels' vector loads need."""
+    """d contiguous and 16-byte aligned strides/base, as the kernels' vector loads need.
+    (A copy where they are not: contiguous() would return a dense view at an odd address,
+    or one with any stride on a dimension of one, as it is.)"""
     s0, s1, s2, s3 = t.stride()
     ok = s3 == 1 and ((s0 | s1 | s2) * t.element_size()) % 16 == 0 and t.data_ptr() % 16 == 0
-    return t if ok else t.contiguous()
+    return t if ok else t.clone(memory_format=torch.contiguous_format)
 
 
 # mattn_problem as one record: 8 sizes and types, scale, flags, 8 x 3 strides

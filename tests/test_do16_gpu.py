@@ -37,6 +37,24 @@ def test_16bit_upstream_gradient(dtype, d, N):
             assert (a != b).double().mean() < 0.02, name
 
 
+@pytest.mark.parametrize("d", [64, 80, 256])
+def test_16bit_upstream_gradient_at_an_odd_address(d):
+    """The gradient of a slice of a flat buffer: dense, but not at a 16-byte address; and
+    one expanded over the sequence.  Bitwise the gradients of an ordinary copy."""
+    import jaxmodules_amd as jm
+
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v = (torch.randn((1, 130, 2, d), generator=gen, device="cuda").to(torch.bfloat16).requires_grad_()
+               for _ in range(3))
+    flat = torch.randn(130 * 2 * d + 1, generator=gen, device="cuda").to(torch.bfloat16)
+    for g in (flat[1:].view(1, 130, 2, d), flat[:2 * d].view(1, 1, 2, d).expand(1, 130, 2, d)):
+        o = jm.masked_attention_via_map(q, k, v, is_causal=True, out_dtype=torch.bfloat16)
+        got = torch.autograd.grad(o, (q, k, v), g, retain_graph=True)
+        want = torch.autograd.grad(o, (q, k, v), g.clone(memory_format=torch.contiguous_format))
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+
+
 def test_flag_is_refused_where_no_kernel_takes_it():
     from jaxmodules_amd import _lib
     from tests.test_capi import _problem

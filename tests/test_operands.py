@@ -1,0 +1,28 @@
+"""What the kernels are handed: rows at 16-byte addresses with 16-byte strides
+(attention._ready), on the CPU."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from jaxmodules_amd import attention as A
+
+
+def _views():
+    flat = torch.arange(4 * 6 * 2 * 64 + 8, dtype=torch.float32).to(torch.bfloat16)
+    n = 4 * 6 * 2 * 64
+    dense = flat[:n].view(4, 6, 2, 64)
+    yield "aligned", dense, True
+    yield "strided rows", dense.transpose(0, 1), True
+    yield "expanded over the sequence", dense[:, :1].expand(4, 6, 2, 64), True
+    yield "dense at an odd address", flat[1:n + 1].view(4, 6, 2, 64), False
+    yield "odd stride on a dimension of one", flat[:n].as_strided((1, 6, 2, 64), (n + 3, 128, 64, 1)), False
+    yield "d not contiguous", flat[:n].view(4, 6, 64, 2).transpose(2, 3), False
+
+
+@pytest.mark.parametrize("what,x,as_is", list(_views()), ids=lambda v: v if isinstance(v, str) else "")
+def test_ready(what, x, as_is):
+    y = A._ready(x)
+    assert (y is x) == as_is
+    assert torch.equal(x, y) and y.dtype == x.dtype
+    assert y.data_ptr() % 16 == 0 and y.stride(3) == 1
+    assert all(s * y.element_size() % 16 == 0 for s in y.stride()[:3])
