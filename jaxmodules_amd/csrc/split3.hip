@@ -10,6 +10,7 @@
 //   forward  S^T = K Q^T, online softmax, O^T += V^T P^T
 //   dQ       S^T = K Q^T, dP^T = V dO^T, dS = P (dP - delta), dQ^T += K^T dS^T
 //   dK/dV    S = Q K^T, dP = dO V^T, dV^T += dO^T P, dK^T += Q^T dS
+// (dP - delta of weights of 1/2 and more: dO . (V - O), see HOT).
 // The streamed rows are read once per workgroup and split into bfloat16 pieces on the
 // way to LDS (bfloat16 rows go there directly); the wave's own rows are split in
 // registers.  P and dS are split from the C registers, which are the B operand of the
@@ -24,8 +25,8 @@
 // Measured, causal steps: float32 [2, 2048, 8, 64] fwd 465 -> 97 us, dK/dV 768 -> 144,
 // dQ 596 -> 113 against the SIMT kernels; bfloat16 [1, 4096, 8, 256] fwd 4322 -> 192 us,
 // dK/dV 14370 -> 579, dQ 4811 -> 248 (32-row waves sharing columns: 326, 750, 708).
-// The error against float64 is no larger than theirs (float32 step: 8.4e-7 of the norm,
-// 1.1e-6 before).  float32 at D = 64 is bound by vector instructions (260 a step and
+// The error against float64 of rows whose weights are spread (that float32 step, unit
+// normal inputs: 8.4e-7 of the norm) is below theirs (1.1e-6).  float32 at D = 64 is bound by vector instructions (260 a step and
 // wave against 48 MFMAs of 16 cycles; half of them split the streamed rows).
 //
 // MFMA 16x16x32 layout (lane l, l16 = l % 16, g = l / 16): A row l16, k = 8 g .. 8 g + 7;
@@ -239,6 +240,166 @@ __device__ __forceinline__ void zero16(f32x4 (&p)[2], uint32_t w) {
     for (int r = 0; r < 4; ++r) p[t][r] = mask_zero(p[t][r], ones16(w, t, r));
 }
 
+// 4 consecutive elements as float32
+template <class T>
+__device__ __forceinline__ f32x4 load4(const char* p) {
+  if constexpr (std::is_same<T, float>::value) {
+    return *(const f32x4*)p;
+  } else {
+    const u32x2 x = *(const u32x2*)p;
+    return f32x4{Elt<T>::to_f32(x[0] & 0xffffu), Elt<T>::to_f32(x[0] >> 16), Elt<T>::to_f32(x[1] & 0xffffu),
+                 Elt<T>::to_f32(x[1] >> 16)};
+  }
+}
+// the four 16-lane groups' values, summed (in all of them)
+__device__ __forceinline__ float sum_groups(float x) {
+  x += __shfl_xor(x, 16);
+  return x + __shfl_xor(x, 32);
+}
+// O of a problem whose gradient has type GT: float32 beside a 16-bit dO under MATTN_DO_16
+template <class GT>
+__device__ __forceinline__ bool o_is_f32(const KArgs& a) {
+  return std::is_same<GT, float>::value || a.do16;
+}
+// the rows a hot pair needs, at the lane's first column 4 g
+struct HotRows { const char *g, *v, *o, *x; };
+// dO . (V - O) of three rows, in float32 (every lane of a row's four has the sum).  U: column steps whose loads are in flight together (left alone, the compiler waits for
+// each step's three before it issues the next)
+template <int U, int D, class IT, class GT>
+__device__ __forceinline__ float dot_vo(const HotRows& p, bool of32) {
+  f32x4 s = {};
+#pragma unroll 1
+  for (int j = 0; j < D / 16; j += U) {
+    f32x4 x[U], y[U], z[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      x[u] = load4<GT>(p.g + 16 * elt_bytes<GT>() * (j + u));
+      y[u] = load4<IT>(p.v + 16 * elt_bytes<IT>() * (j + u));
+    }
+    if (std::is_same<GT, float>::value || of32) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) z[u] = load4<float>(p.o + 64 * (j + u));
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) z[u] = load4<GT>(p.o + 16 * elt_bytes<GT>() * (j + u));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = fmaf(x[u][e], y[u][e] - z[u][e], s[e]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return sum_groups((s[0] + s[1]) + (s[2] + s[3]));
+}
+
+// Pairs whose weight reaches HOT take dP - delta as dO . (V - O).  Where one key
+// dominates a row its dP and delta are nearly the same number, and their roundings
+// (2^-24 of |dO| |V|) would be all that is left of the difference; V - O is small there
+// and exact to O's own rounding.  (Left to the difference, dQ and dK of rows with a weight
+// of 0.9 or more were 2.4 to 4.9 times as far off.)
+// The check and the list cost dK/dV 2 to 5% and dQ 0 to 4% where no row is dominated (144
+// -> 149 and 115 -> 116 us for float32 [2, 2048, 8, 64]; 589 -> 600 and 254 -> 264 for
+// bfloat16 [1, 4096, 8, 256]); at 1/4 instead of 1/2 they found no error to take away.
+// A step leaves its hot pairs out of dS and notes them, up to MAX for each of the wave's
+// rows; they are added after the walk, when its operands' registers are free and all 16
+// rows have theirs formed at once (dK/dV of such float32 rows at D = 64, one dominant key
+// each: 207 us; formed in each step, 16 rows of one pair: 236).  A query (dQ) has no more than two.  A key that more
+// than eight queries lean on (the first one of a sequence, often) has the rest formed in
+// their step, hot_rest().
+constexpr float HOT = 0.5f;
+constexpr int HOT_Q = 2, HOT_K = 8;
+template <int MAX>
+struct HotList {
+  int n[16];
+  int2 pair[16][MAX];  // streamed row, weight
+};
+__device__ __forceinline__ bool any_hot(const f32x4 (&p)[2]) {
+  float mx = 0.f;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, p[t][r]);
+  return __builtin_expect(__any(mx >= HOT), 0);  // (laid out of the walk's way)
+}
+// The step's pairs: p weights, d = dP - delta, r0 the first streamed row.  Returns the
+// lane's hot pairs that found no place, bit 4 t + r.
+template <int MAX>
+__device__ __forceinline__ uint32_t note_hot(const f32x4 (&p)[2], f32x4 (&d)[2], HotList<MAX>& list, int r0) {
+  // (re-defined here: what depends on the lane alone would be formed before the walk and kept)
+  const int lane = opaque(threadIdx.x) & 63, l16 = lane & 15, g = lane >> 4;
+  uint32_t own = 0, rest = 0;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) own |= (p[t][r] >= HOT ? 1u : 0u) << (4 * t + r);
+  uint32_t m = own << (8 * g);  // the row's: bit 8 g + 4 t + r
+  m |= __shfl_xor(m, 16);
+  m |= __shfl_xor(m, 32);
+  const int n = list.n[l16];
+  int at = n + (int)__builtin_popcount(m & ((1u << (8 * g)) - 1u));  // place of this lane's next one
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if ((own >> (4 * t + r)) & 1u) {
+        if (at < MAX) {
+          list.pair[l16][at++] = make_int2(r0 + 16 * t + 4 * g + r, __float_as_int(p[t][r]));
+          d[t][r] = 0.f;
+        } else {
+          rest |= 1u << (4 * t + r);
+        }
+      }
+  list.n[l16] = min(n + (int)__builtin_popcount(m), MAX);
+  return rest;
+}
+// d of the pairs note_hot had no place for, 16 at a time whatever rows they belong to.
+// rows(own, i): the rows of own row `own` (0 .. 15) and streamed row i (0 .. 31) at lane group g.
+template <int D, class IT, class GT, class F>
+__device__ __forceinline__ void hot_rest(f32x4 (&d)[2], uint32_t rest, bool of32, F&& rows) {
+  while (__any(rest != 0)) {
+    const int lane = opaque(threadIdx.x) & 63, g = lane >> 4;
+    const uint64_t b = __ballot(rest != 0);
+    const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+    const bool mine = rest != 0 && rank < 16;
+    const int e = rest ? (int)__builtin_ctz(rest) : 0;
+    // pair `rank` to the four lanes l16 = rank (lanes without one form pair (0, 0))
+    const int pair = __builtin_amdgcn_ds_permute(4 * (mine ? rank : 63), mine ? (lane & 15) | (16 * (e >> 2) + 4 * g + (e & 3)) << 4 : 0);
+    const int got = __shfl(pair, lane & 15);
+    const float x = __shfl(dot_vo<2, D, IT, GT>(rows(got & 15, got >> 4, g), of32), rank & 15);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (mine && e == 4 * t + r) d[t][r] = x;
+    if (mine) rest &= rest - 1;
+  }
+}
+// acc[mt] += the noted pairs' dS times their streamed rows x; rows(i): those of streamed row i
+template <int D, class IT, class GT, int MAX, class F>
+__device__ __forceinline__ void add_hot(f32x4 (&acc)[D / 16], HotList<MAX>& list, int l16, bool of32, F&& rows) {
+  const int nh = list.n[l16];
+  for (int n = 0; __any(n < nh); ++n) {
+    const bool on = n < nh;
+    const int2 pw = list.pair[l16][n];
+    const HotRows p = rows(on ? pw.x : 0);
+    // every load of a round in flight at once, where there are registers (D = 256: not)
+    constexpr int U = D == 256 ? 2 : D / 16;
+    f32x4 x[D / 16];
+    if constexpr (D != 256) {
+#pragma unroll
+      for (int mt = 0; mt < D / 16; ++mt) x[mt] = load4<IT>(p.x + 16 * elt_bytes<IT>() * mt);
+    }
+    const float ds = __int_as_float(pw.y) * dot_vo<U, D, IT, GT>(p, of32);
+#pragma unroll
+    for (int mt = 0; mt < D / 16; ++mt) {
+      if constexpr (D == 256) x[mt] = load4<IT>(p.x + 16 * elt_bytes<IT>() * mt);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[mt][e] = on ? fmaf(ds, x[mt][e], acc[mt][e]) : acc[mt][e];
+    }
+  }
+}
+
 // One walk: the streamed rows of step s are in LDS buffer s % NBUF when compute(s) runs.
 // start(s, buf) issues their loads, finish(buf) writes what went through registers.
 template <int NBUF, bool DMA, int BUF, class S, class F, class C>
@@ -359,6 +520,7 @@ void bwd_dq_s3(KArgs a) {
   using R = Rows<D, IT, NTH>;
   constexpr int BUF = 2 * R::ELTS, NBUF = R::DMA || 4 * BUF <= 56 * 1024 ? 2 : 1;
   __shared__ __attribute__((aligned(512))) uint16_t L[cmax(NBUF * BUF, NW * 16 * D * 2)];
+  __shared__ HotList<HOT_Q> Hl[NW];
 
   const Slot slot = launch_slot<NSUB, RES>(a);
   const int item = slot.ok ? a.q_order[slot.slot] : -1;
@@ -382,6 +544,7 @@ void bwd_dq_s3(KArgs a) {
   own16<D, OT>(gf, head_base(a.dO, a.dos, b, h, elt_bytes<OT>()), a.dos[1], qc, g);
   const int64_t rs = ((int64_t)b * a.Hq + h) * a.Lq + qc;
   const float lse = a.lse[rs], delta = a.delta[rs], c2 = a.scale_log2;
+  if (lane < 16) Hl[wave].n[lane] = 0;
   f32x4 acc[NMD];
 #pragma unroll
   for (int i = 0; i < NMD; ++i) acc[i] = f32x4{};
@@ -399,7 +562,7 @@ void bwd_dq_s3(KArgs a) {
       },
       [&](int s, const uint16_t* Kl) {
         const uint16_t* Vl = Kl + R::ELTS;
-        const int mask = walk.mask(s);
+        const int mask = walk.mask(s), k0 = walk.first(s);
         uint32_t w = 0xffffffffu;
         if (mask >= 0) {
           w = bits32(a.row_bits, mask, s % Walk<BN>::SPT, qloc, g);
@@ -415,11 +578,21 @@ void bwd_dq_s3(KArgs a) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) dp[t][r] = st[t][r] * (dp[t][r] - delta);
+          for (int r = 0; r < 4; ++r) dp[t][r] -= delta;
+        if (any_hot(st)) note_hot(st, dp, Hl[wave], k0);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) dp[t] *= st[t];
         add_rows<D, NP>(lds_addr(Kl) + ta, c_frag16(dp[0], dp[1]), acc);
       });
 
   __syncthreads();
+  const bool of32 = o_is_f32<OT>(a);
+  add_hot<D, IT, OT>(acc, Hl[wave], l16, of32, [&](int key) {
+    return HotRows{head_base(a.dO, a.dos, b, h, elt_bytes<OT>()) + elt_bytes<OT>() * ((int64_t)qc * a.dos[1] + 4 * g),
+                   vb + elt_bytes<IT>() * ((int64_t)key * a.vs[1] + 4 * g),
+                   head_base(a.o, a.os, b, h, of32 ? 4 : 2) + (of32 ? 4 : 2) * ((int64_t)qc * a.os[1] + 4 * g),
+                   kb + elt_bytes<IT>() * ((int64_t)key * a.ks[1] + 4 * g)};
+  });
   const int r0 = qt * TILE + wrow + 16 * wave;
   put16<D, IT>(acc, a.scale, (float*)L + wave * 16 * D, a.dq,
                (int64_t)b * a.dqs[0] + (int64_t)r0 * a.dqs[1] + (int64_t)h * a.dqs[2], a.dqs[1], a.Lq - r0, lane);
@@ -436,7 +609,7 @@ constexpr int dkdv_bufs() {
 // accumulators, K and V would take 192 registers of a wave's 256 (S is then formed
 // twice, 1/14 of the products).
 template <int D, class IT, class OT, int PART, int NW>
-__device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, int sl, int sub) {
+__device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, HotList<HOT_K>* Hl, int sl, int sub) {
   constexpr bool DV = PART & 1, DK = PART & 2;
   constexpr int NTH = 64 * NW, NP = Pieces<IT>::n, NG = Pieces<OT>::n;
   constexpr int NKD = D / 32, NMD = D / 16;
@@ -454,6 +627,7 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
   const uint32_t ra = row_addr<D>(l16, g), ta = tr_addr<D>(l16, g);
   const int kloc = wrow + 16 * wave + l16, kc = min(kt * TILE + kloc, a.Lk - 1);
   const float c2 = a.scale_log2;
+  const bool of32 = o_is_f32<OT>(a);
 
   Frag<NP> kf[NKD], vf[DK ? NKD : 1];
   own16<D, IT>(kf, head_base(a.k, a.ks, b, hk, elt_bytes<IT>()), a.ks[1], kc, g);
@@ -474,6 +648,13 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
     const int64_t rs = ((int64_t)b * a.Hq + h) * a.Lq;
     Rq rq;
     Rg rg;
+    const auto hot_rows = [&](int key, int q, int g4) {
+      return HotRows{gb + elt_bytes<OT>() * ((int64_t)q * a.dos[1] + 4 * g4),
+                     head_base(a.v, a.vs, b, hk, elt_bytes<IT>()) + elt_bytes<IT>() * ((int64_t)key * a.vs[1] + 4 * g4),
+                     head_base(a.o, a.os, b, h, of32 ? 4 : 2) + (of32 ? 4 : 2) * ((int64_t)q * a.os[1] + 4 * g4),
+                     qb + elt_bytes<IT>() * ((int64_t)q * a.qs[1] + 4 * g4)};
+    };
+    if (DK && lane < 16) Hl[wave].n[lane] = 0;
     float rl = 0.f;  // lse (threads 0 .. BN - 1) or delta (the next BN) of a row
     __syncthreads();  // the previous head's last step is consumed
     walk_rows<NBUF, Rq::DMA || Rg::DMA, BUF>(walk.n, L,
@@ -494,7 +675,7 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
         [&](int s, const uint16_t* Ql) {
           const uint16_t* Gl = Ql + Rq::ELTS;
           const float* Rs = Rl + (NBUF == 2 ? s & 1 : 0) * 2 * BN + 4 * g;
-          const int mask = walk.mask(s);
+          const int mask = walk.mask(s), q0 = walk.first(s);
           uint32_t w = 0xffffffffu;
           if (mask >= 0) {
             w = bits32(a.col_bits, mask, s % Walk<BN>::SPT, kloc, g);
@@ -513,13 +694,19 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
             }
           }
           if (mask >= 0) zero16(st, w);
+          if constexpr (DV) add_rows<D, NG>(lds_addr(Gl) + ta, c_frag16(st[0], st[1]), dv);
           if constexpr (DK) {
+            if (any_hot(st))
+              hot_rest<D, IT, OT>(dp, note_hot(st, dp, Hl[wave], q0), of32, [&](int own, int i, int g4) {
+                return hot_rows(min(kt * TILE + wrow + 16 * wave + own, a.Lk - 1), min(q0 + i, a.Lq - 1), g4);
+              });
 #pragma unroll
             for (int t = 0; t < 2; ++t) dp[t] *= st[t];
           }
-          if constexpr (DV) add_rows<D, NG>(lds_addr(Gl) + ta, c_frag16(st[0], st[1]), dv);
           if constexpr (DK) add_rows<D, NP>(lds_addr(Ql) + ta, c_frag16(dp[0], dp[1]), dk);
         });
+    if constexpr (DK)
+      add_hot<D, IT, OT>(dk, Hl[wave], l16, of32, [&](int q) { return hot_rows(kc, q, g); });
   }
 
   const int r0 = kt * TILE + wrow + 16 * wave;
@@ -539,12 +726,13 @@ void bwd_dkdv_s3(KArgs a) {
   constexpr int BUF = Rows<D, IT, 64 * NW>::ELTS + Rows<D, OT, 64 * NW>::ELTS;
   __shared__ __attribute__((aligned(512))) uint16_t L[cmax(NBUF * BUF, NW * 16 * D * 2)];
   __shared__ __attribute__((aligned(16))) float Rl[NBUF * 2 * BN];  // lse, delta of the step's rows
+  __shared__ HotList<HOT_K> Hl[NW];
   constexpr int NPART = D == 256 ? 2 : 1;
   const Slot s = launch_slot<NPART * TILE / (16 * NW), RES>(a);
   if (!s.ok) return;
-  if constexpr (NPART == 1) dkdv_s3<D, IT, OT, 3, NW>(a, L, Rl, s.slot, s.part);
-  else if (s.part & 1) dkdv_s3<D, IT, OT, 1, NW>(a, L, Rl, s.slot, s.part >> 1);
-  else dkdv_s3<D, IT, OT, 2, NW>(a, L, Rl, s.slot, s.part >> 1);
+  if constexpr (NPART == 1) dkdv_s3<D, IT, OT, 3, NW>(a, L, Rl, Hl, s.slot, s.part);
+  else if (s.part & 1) dkdv_s3<D, IT, OT, 1, NW>(a, L, Rl, Hl, s.slot, s.part >> 1);
+  else dkdv_s3<D, IT, OT, 2, NW>(a, L, Rl, Hl, s.slot, s.part >> 1);
 }
 
 // delta = rowsum(dO * O), summed in float64: D / 8 threads a row, the rows in the
