@@ -25,9 +25,12 @@
 // Measured, causal steps: float32 [2, 2048, 8, 64] fwd 465 -> 97 us, dK/dV 768 -> 144,
 // dQ 596 -> 113 against the SIMT kernels; bfloat16 [1, 4096, 8, 256] fwd 4322 -> 192 us,
 // dK/dV 14370 -> 579, dQ 4811 -> 248 (32-row waves sharing columns: 326, 750, 708).
-// The error against float64 of rows whose weights are spread (that float32 step, unit
-// normal inputs: 8.4e-7 of the norm) is below theirs (1.1e-6).  float32 at D = 64 is bound by vector instructions (260 a step and
-// wave against 48 MFMAs of 16 cycles; half of them split the streamed rows).
+// The error against float64 is 0.6 to 1.0 times that of the SIMT kernels they replaced
+// (0.7 and 0.8 of it for O and the gradients of that float32 step) over logits of standard
+// deviation 1 to 32; where one key of a large positive dot product has nearly all of a
+// row's weight, O is up to 1.3 and dQ up to 1.4 times as far off (1e-7 of the norm).
+// float32 at D = 64 is bound by vector instructions (270 a step and wave against 48 MFMAs
+// of 16 cycles; half of them split the streamed rows).
 //
 // MFMA 16x16x32 layout (lane l, l16 = l % 16, g = l / 16): A row l16, k = 8 g .. 8 g + 7;
 // B column l16, the same k; C column l16, register r row 4 g + r.  The two 16-row
@@ -115,30 +118,108 @@ __device__ __forceinline__ uint32_t tr_addr(int l16, int g) {
   return 2 * r * D + ((((l16 & 3) >> 1) ^ sw<D>(r)) << 4) + 8 * (l16 & 1);
 }
 
-// S += A X and dP += A2 X2 along d for both 16-row blocks: tiles at byte addresses ra, rb
-template <int WANT, int D, int NA, int NX, int NB, int NY>
+// A dot product along d in the making (C registers of one 16-row block), over D / 32 steps.
+// A 16x16x32 MFMA rounds its result four times (measured: off by 0.58 units in the last
+// place in the mean square, one rounding is 0.29), so one chain of all piece products
+// carries 4 x 6 roundings a step at the size the sum has reached: O of float32 problems
+// with logits of 10 and more was 1.3, 1.9 and 3.1 times as far off at D = 64, 128 and 256
+// as sums of 16 or 32 FMAs a lane had left it.  So the small products (2^-8 of the size
+// and less) come first, or apart from the leading ones:
+//   LAST    one chain, the first step's leading product at its end (D = 64, where two
+//           more additions an element are 5% of the backward)
+//   HALVES  a: the leading products of the first half of the steps, b: the small ones
+//           and the other half; a + b (D = 128)
+//   LINKS   the leading products two steps at a time in a, summed here, but for the last
+//           two, which follow the small ones in b (D = 256)
+//   ONE     one chain in the order of the steps
+enum Chains { ONE, LAST, HALVES, LINKS };
+template <int D, int NA, int NB, Chains C>
+struct Dot {
+  static constexpr int N = D / 32, TAIL = C == HALVES ? N / 2 : N - 2;  // leading products from TAIL on: b
+  static_assert(C != LAST || N == 2, "");
+  f32x4 a, b, sum;
+  u32x4 x0, y0;  // LAST: the first step's leading operands
+  template <int KD>
+  __device__ __forceinline__ void begin() {
+    if constexpr (KD == 0 || (C == LINKS && KD < TAIL && KD % 2 == 0)) a = f32x4{};
+    if constexpr (C >= HALVES && KD == 0) b = f32x4{};
+  }
+  // product n of step KD
+  template <int KD, int n>
+  __device__ __forceinline__ void mma(const Frag<NA>& x, const Frag<NB>& y) {
+    constexpr int ij = product_ij(NA, NB, n);
+    if constexpr (C == LAST && KD == 0 && ij == 0) {
+      x0 = x.p[0];
+      y0 = y.p[0];
+    } else {
+      mfma1(x.p[ij / 4], y.p[ij % 4], C < HALVES || (ij == 0 && KD < TAIL) ? a : b);
+    }
+  }
+  template <int KD>
+  __device__ __forceinline__ void end() {
+    if constexpr (C == LAST && KD == N - 1) mfma1(x0, y0, a);
+    if constexpr (C == LINKS && KD < TAIL && KD % 2 == 1) {
+      if constexpr (KD == 1) sum = a;
+      else sum += a;
+    }
+  }
+  __device__ __forceinline__ f32x4 total() const { return C < HALVES ? a : C == HALVES ? a + b : sum + b; }
+};
+// x and y's products of step KD in turn (an MFMA that adds to the result of the one before
+// it waits for it)
+template <int KD, int D, int NA, int NB, int NC, int ND, Chains C>
+__device__ __forceinline__ void dot_step(Dot<D, NA, NB, C>& x, const Frag<NA>& a, const Frag<NB>& b,
+                                         Dot<D, NC, ND, C>& y, const Frag<NC>& c, const Frag<ND>& d) {
+  constexpr int P1 = products(NA, NB), P2 = products(NC, ND);
+  x.template begin<KD>();
+  y.template begin<KD>();
+  static_for<(P1 > P2 ? P1 : P2)>([&](auto nc) {
+    constexpr int n = decltype(nc)::value;
+    if constexpr (n < P1) x.template mma<KD, n>(a, b);
+    if constexpr (n < P2) y.template mma<KD, n>(c, d);
+  });
+  x.template end<KD>();
+  y.template end<KD>();
+}
+
+// S = A X and dP = A2 X2 along d for both 16-row blocks t: tiles at byte addresses ra, rb
+// (block by block, or, ONE, both at each step)
+template <int WANT, Chains C, int D, int NA, int NX, int NB, int NY>
 __device__ __forceinline__ void two_dots(uint32_t ra, uint32_t rb, const Frag<NX> (&x)[D / 32], const Frag<NY> (&y)[D / 32],
                                          f32x4 (&st)[2], f32x4 (&dp)[2]) {
-  constexpr int PF = ahead(WANT, NA + NB), PL = 2 * BN * D;
+  constexpr int PF = ahead(WANT, NA + NB), PL = 2 * BN * D, N = D / 32;
   Frag<NA> fa[PF + 1];
   Frag<NB> fb[PF + 1];
-  pipe<2 * (D / 32), PF, NA + NB>(
+  Dot<D, NA, NX, C> s[C == ONE ? 2 : 1];
+  Dot<D, NB, NY, C> p[C == ONE ? 2 : 1];
+  pipe<2 * N, PF, NA + NB>(
       [&](auto ic, auto sc) {
-        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value, kd = i / 2, t = i % 2;
+        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value;
+        constexpr int kd = C == ONE ? i / 2 : i % N, t = C == ONE ? i % 2 : i / N;
+        if constexpr (C != ONE && i == N) {  // the second block's addresses are formed anew (kept: 2 N registers)
+          ra = opaque(ra);
+          rb = opaque(rb);
+        }
         rd<32 * t * D, PL>(fa[sl], ra ^ (uint32_t)(64 * kd));
         rd<32 * t * D, PL>(fb[sl], rb ^ (uint32_t)(64 * kd));
       },
       [&](auto ic, auto sc) {
-        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value, kd = i / 2, t = i % 2;
+        constexpr int i = decltype(ic)::value, sl = decltype(sc)::value;
+        constexpr int kd = C == ONE ? i / 2 : i % N, t = C == ONE ? i % 2 : i / N, u = C == ONE ? t : 0;
         landed(fa[sl]);
         landed(fb[sl]);
-        mma_two(fa[sl], x[kd], st[t], fb[sl], y[kd], dp[t]);
+        dot_step<kd>(s[u], fa[sl], x[kd], p[u], fb[sl], y[kd]);
+        if constexpr (kd == N - 1) {
+          st[t] = s[u].total();
+          dp[t] = p[u].total();
+        }
       });
 }
-template <int D, int NA, int NX>
+template <Chains C, int D, int NA, int NX>
 __device__ __forceinline__ void one_dot(uint32_t ra, const Frag<NX> (&x)[D / 32], f32x4 (&st)[2]) {
   constexpr int PF = ahead(2, 2 * NA), PL = 2 * BN * D;
   Frag<NA> f0[PF + 1], f1[PF + 1];
+  Dot<D, NA, NX, C> s0, s1;
   pipe<D / 32, PF, 2 * NA>(
       [&](auto ic, auto sc) {
         constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
@@ -149,9 +230,17 @@ __device__ __forceinline__ void one_dot(uint32_t ra, const Frag<NX> (&x)[D / 32]
         constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
         landed(f0[sl]);
         landed(f1[sl]);
-        mma_two(f0[sl], x[kd], st[0], f1[sl], x[kd], st[1]);
+        dot_step<kd>(s0, f0[sl], x[kd], s1, f1[sl], x[kd]);
       });
+  st[0] = s0.total();
+  st[1] = s1.total();
 }
+// (forward and backward alike where gradients are float32: P = exp2(S - lse) takes S as
+// lse has it.  16-bit gradients at D = 256 hide the difference by their own rounding.)
+template <int D>
+constexpr Chains fwd_chains() { return D == 64 ? LAST : D == 128 ? HALVES : LINKS; }
+template <int D, class IT>
+constexpr Chains bwd_chains() { return D == 256 && !std::is_same<IT, float>::value ? ONE : fwd_chains<D>(); }
 // acc[mt] += (tile at byte address ta)^T w, the 32 rows of the tile against w
 template <int D, int NA, int WANT = 2>
 __device__ __forceinline__ void add_rows(uint32_t ta, const Frag<3>& w, f32x4 (&acc)[D / 16]) {
@@ -447,8 +536,8 @@ void fwd_s3(KArgs a) {
   f32x4 acc[NMD];
 #pragma unroll
   for (int i = 0; i < NMD; ++i) acc[i] = f32x4{};
-  float m2 = NEG_INF, l = 0.f;
-  const float c2 = a.scale_log2;
+  float m = NEG_INF, l = 0.f;
+  const float c2 = a.scale_log2, up = fminf(8.f / c2, 3.4e38f);  // (finite: -inf + up < any score)
 
   R ks, vs;
   walk_rows<NBUF, R::DMA, BUF>(walk.n, L,
@@ -469,8 +558,8 @@ void fwd_s3(KArgs a) {
           w = bits32(a.row_bits, mask, s % Walk<BN>::SPT, qloc, g);
           if (!__any((w & 0x000f000fu) != 0)) return;  // no allowed key of the wave's rows here
         }
-        f32x4 st[2] = {f32x4{}, f32x4{}};
-        one_dot<D, NP>(lds_addr(Kl) + ra, qf, st);
+        f32x4 st[2];
+        one_dot<fwd_chains<D>(), D, NP>(lds_addr(Kl) + ra, qf, st);
         if (mask >= 0) {
 #pragma unroll
           for (int t = 0; t < 2; ++t)
@@ -482,22 +571,22 @@ void fwd_s3(KArgs a) {
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[t][r]);
-        const float mx2 = wave_max32(wave_max16(mx)) * c2;
-        // the running max is raised only when a row's grows by more than 2^8
-        if (__any(mx2 > m2 + 8.f)) {
-          const float mn = fmaxf(m2, mx2);
-          const float alpha = (mn == NEG_INF) ? 1.f : fast_exp2(m2 - mn);
+        mx = wave_max32(wave_max16(mx));
+        // the running max is raised only when a row's weights grow by more than 2^8
+        if (__any(mx > m + up)) {
+          const float mn = fmaxf(m, mx);
+          const float alpha = (mn == NEG_INF) ? 1.f : fast_exp2((m - mn) * c2);
           l *= alpha;
 #pragma unroll
           for (int i = 0; i < NMD; ++i) acc[i] *= alpha;
-          m2 = mn;
+          m = mn;
         }
-        const float nmu = (m2 == NEG_INF) ? 0.f : -m2;
+        const float mu = (m == NEG_INF) ? 0.f : m;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            st[t][r] = fast_exp2(fmaf(st[t][r], c2, nmu));
+            st[t][r] = fast_exp2((st[t][r] - mu) * c2);  // exactly 1 for the key that set m
             l += st[t][r];
           }
         add_rows<D, NP>(lds_addr(Vl) + ta, c_frag16(st[0], st[1]), acc);
@@ -505,7 +594,7 @@ void fwd_s3(KArgs a) {
 
   l += __shfl_xor(l, 16);
   l = wave_sum32(l);
-  if (g == 0 && q < a.Lq) a.lse[((int64_t)b * a.Hq + h) * a.Lq + q] = l > 0.f ? m2 + __builtin_log2f(l) : NEG_INF;
+  if (g == 0 && q < a.Lq) a.lse[((int64_t)b * a.Hq + h) * a.Lq + q] = l > 0.f ? fmaf(m, c2, __builtin_log2f(l)) : NEG_INF;
   __syncthreads();  // every wave is done with the operand tiles
   const int r0 = qt * TILE + wrow + 16 * wave;
   put16<D, OT>(acc, l > 0.f ? 1.f / l : 0.f, (float*)L + wave * 16 * D, a.out,
@@ -568,8 +657,8 @@ void bwd_dq_s3(KArgs a) {
           w = bits32(a.row_bits, mask, s % Walk<BN>::SPT, qloc, g);
           if (!__any((w & 0x000f000fu) != 0)) return;
         }
-        f32x4 st[2] = {f32x4{}, f32x4{}}, dp[2] = {f32x4{}, f32x4{}};
-        two_dots<D == 64 ? 2 : 1, D, NP, NP, NP, NG>(lds_addr(Kl) + ra, lds_addr(Vl) + ra, qf, gf, st, dp);
+        f32x4 st[2], dp[2];
+        two_dots<D == 64 ? 2 : 1, bwd_chains<D, IT>(), D, NP, NP, NP, NG>(lds_addr(Kl) + ra, lds_addr(Vl) + ra, qf, gf, st, dp);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -681,9 +770,9 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
             w = bits32(a.col_bits, mask, s % Walk<BN>::SPT, kloc, g);
             if (!__any((w & 0x000f000fu) != 0)) return;
           }
-          f32x4 st[2] = {f32x4{}, f32x4{}}, dp[2] = {f32x4{}, f32x4{}};
-          if constexpr (!DK) one_dot<D, NP>(lds_addr(Ql) + ra, kf, st);
-          else two_dots<D == 128 ? 1 : 2, D, NP, NP, NG, NP>(lds_addr(Ql) + ra, lds_addr(Gl) + ra, kf, vf, st, dp);
+          f32x4 st[2], dp[2];
+          if constexpr (!DK) one_dot<bwd_chains<D, IT>(), D, NP>(lds_addr(Ql) + ra, kf, st);
+          else two_dots<D == 128 ? 1 : 2, bwd_chains<D, IT>(), D, NP, NP, NG, NP>(lds_addr(Ql) + ra, lds_addr(Gl) + ra, kf, vf, st, dp);
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             const f32x4 ls = *(const f32x4*)(Rs + 16 * t), dl = *(const f32x4*)(Rs + BN + 16 * t);

@@ -25,7 +25,8 @@ def _check(q, k, v, do, key, **kw):
     """key [N]: the key each query's weight is on."""
     import jaxmodules_amd as jm
 
-    if q.dtype == torch.float16:  # gradients of 1e-7 times 2^7, clear of float16's subnormals
+    half = q.dtype == torch.float16
+    if half:  # gradients of 1e-7 times 2^7: float16's subnormals end at 6e-8
         do = do * 128
     q, k, v = (x.requires_grad_() for x in (q, k, v))
     o = jm.masked_attention_via_map(q, k, v, **kw)
@@ -33,14 +34,17 @@ def _check(q, k, v, do, key, **kw):
     G, rel = q.shape[2] // k.shape[2], 1e-3 if q.dtype == torch.float32 else 4e-3
     q, k, v, o, do = (x.detach().double() for x in (q, k, v, o, do))
     kx, vx = (x.repeat_interleave(G, 2)[:, key] for x in (k, v))
-    # P V over the sum of the weights: a few roundings of V
+    # P V over the sum of the weights: a few roundings of V at most
     assert ((o - vx).abs() <= 8 * U * vx.abs()).all()
     x = (do * (vx - o)).sum(-1, keepdim=True) / math.sqrt(q.shape[-1])
     per_key = lambda y: torch.zeros_like(k).index_add_(1, key, y.unflatten(2, (-1, G)).sum(3))  # noqa: E731
     for name, got, want in (("dQ", dq, x * kx), ("dK", dk, per_key(x * q)), ("dV", dv, per_key(do))):
-        err = ((got - want).norm() / want.norm()).item()
-        print(f"[dominated] d {q.shape[-1]} {name}: {err:.1e}, {(want.norm() / got.norm()).item():.2f}", flush=True)
-        assert err < rel, name
+        err, bound = (got - want).norm().item(), rel * want.norm().item()
+        if name != "dV":  # the weights of the other keys, and a float16 output's subnormals
+            bound += 1e-3 * U * ((do * vx).norm(dim=-1, keepdim=True) * {"dQ": kx, "dK": q}[name]).norm().item()
+            bound += 2.0 ** -25 * got.numel() ** 0.5 if half else 0.0
+        print(f"[dominated] d {q.shape[-1]} {name}: off by {err:.1e} of {want.norm().item():.1e}", flush=True)
+        assert err <= bound, name
 
 
 @pytest.mark.parametrize("dtype,d", KINDS)

@@ -65,3 +65,19 @@ def test_norm_relative_error(dtype, d):
         rel = np.linalg.norm(a - b) / np.linalg.norm(b)
         print(f"[norm] {dtype} d={d} {name}: {rel:.2e}")
         assert rel < 2e-6, name
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_large_logits(d):
+    """Logits with a standard deviation of 10 (up to 50): a weight is off by its score's
+    error times ln 2, so the scores' sums over d decide whether O meets the gate."""
+    import jaxmodules_amd as jm
+    from tests.helpers import assert_close
+
+    for seed in range(3):
+        Q, K, V, dO = seeded_inputs(1, 512, 512, 4, 2, d, seed, scaled=False)
+        Q = (10 * Q).astype(np.float32)
+        q, k, v = (torch.from_numpy(x).cuda() for x in (Q, K, V))
+        o = jm.masked_attention_via_map(q, k, v, is_causal=True, precision="default")
+        O_ref, _, _, _ = oracle(Q, K, V, dO, CAUSAL, grads=False)
+        assert_close(o.cpu().numpy(), O_ref, "float32", f"d {d}")
