@@ -345,10 +345,22 @@ __device__ __forceinline__ float sum_groups(float x) {
   x += __shfl_xor(x, 16);
   return x + __shfl_xor(x, 32);
 }
+// The kernel's arguments read anew: what only rarely taken paths need of them would
+// otherwise be read at the kernel's start and held over the walk.
+__device__ __forceinline__ const KArgs& args_again() {
+  uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const KArgs*)(const __attribute__((address_space(4))) KArgs*)p;
+}
 // O of a problem whose gradient has type GT: float32 beside a 16-bit dO under MATTN_DO_16
 template <class GT>
 __device__ __forceinline__ bool o_is_f32(const KArgs& a) {
   return std::is_same<GT, float>::value || a.do16;
+}
+// row r of a tensor slice at lane group g's first column
+template <class T>
+__device__ __forceinline__ const char* row_at(const char* base, int64_t rs, int r, int g) {
+  return base + elt_bytes<T>() * ((int64_t)r * rs + 4 * g);
 }
 // the rows a hot pair needs, at the lane's first column 4 g
 struct HotRows { const char *g, *v, *o, *x; };
@@ -489,6 +501,146 @@ __device__ __forceinline__ void add_hot(f32x4 (&acc)[D / 16], HotList<MAX>& list
   }
 }
 
+// ---- results that are not finite ---------------------------------------------------
+// The pieces of an infinity do not add up to it (Inf - Inf), those of a float32 past
+// bfloat16's largest value neither, an infinite piece times a zero one is NaN, and so is
+// the weight 0 of a masked key times an infinite V.  All of this ends as Inf or NaN in the
+// results of the rows it meets, never as a wrong finite value; so a wave that finds either
+// there forms its 16 rows again in plain float32, pair by allowed pair, which gives the
+// infinities and NaNs that the arithmetic of the inputs has.  Lanes as before: l16 the row,
+// g its columns 16 j + 4 g .. + 3.  (g is re-defined for each pair, so that the own row's
+// columns are not held over the loop.)
+template <int N>
+__device__ __forceinline__ bool not_finite(const f32x4 (&acc)[N]) {
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t = fmaf(acc[i][e], 0.f, t);
+  return __builtin_expect(__any(!(t == 0.f)), 0);
+}
+// f(other, on): every position `other` < n of the present tiles of a map row (or column)
+// with an allowed pair in the wave, on where the lane's own row has it
+template <class F>
+__device__ __forceinline__ void each_pair(const int* ent, int e0, int e1, const uint64_t* bits, int row, int n, F&& f) {
+#pragma unroll 1
+  for (int e = e0; e < e1; ++e) {
+    const int first = ent[2 * e] * TILE, mask = ent[2 * e + 1];
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+      const uint64_t w = mask < 0 ? ~0ull : bits[((int64_t)mask * 2 + half) * TILE + row];
+#pragma unroll 1
+      for (int i = 0; i < 64 && first + 64 * half + i < n; ++i) {
+        const bool on = (w >> i) & 1u;
+        if (__any(on)) f(first + 64 * half + i, on);
+      }
+    }
+  }
+}
+template <int D, class T>
+__device__ __forceinline__ float dot_plain(const char* x, const char* y) {
+  f32x4 s = {};
+#pragma unroll 2
+  for (int j = 0; j < D / 16; ++j) {
+    const f32x4 u = load4<T>(x + 16 * elt_bytes<T>() * j), v = load4<T>(y + 16 * elt_bytes<T>() * j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = fmaf(u[e], v[e], s[e]);
+  }
+  return sum_groups((s[0] + s[1]) + (s[2] + s[3]));
+}
+// acc += w x where on
+template <int D, class T>
+__device__ __forceinline__ void add_plain(f32x4 (&acc)[D / 16], float w, const char* x, bool on) {
+#pragma unroll
+  for (int j = 0; j < D / 16; ++j) {
+    const f32x4 u = load4<T>(x + 16 * elt_bytes<T>() * j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[j][e] = on ? fmaf(w, u[e], acc[j][e]) : acc[j][e];
+  }
+}
+template <int N>
+__device__ __forceinline__ void clear(f32x4 (&acc)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) acc[i] = f32x4{};
+}
+// The wave's 16 rows from row0 (of tile qt or kt: TILE t + row0) once more.
+// forward: O times the weights' sum l, and lse
+template <int D, class IT>
+__device__ __forceinline__ void plain_fwd(const KArgs& a, int b, int h, int qt, int row0, f32x4 (&acc)[D / 16], float& l,
+                                          float& lse) {
+  const int row = row0 + (opaque(threadIdx.x) & 15), qc = min(qt * TILE + row, a.Lq - 1), hk = h / a.G;
+  const int mrow = map_row(a, b, h, a.nqt, qt);
+  const char* qb = head_base(a.q, a.qs, b, h, elt_bytes<IT>());
+  const char* kb = head_base(a.k, a.ks, b, hk, elt_bytes<IT>());
+  const char* vb = head_base(a.v, a.vs, b, hk, elt_bytes<IT>());
+  float m = NEG_INF;
+  l = 0.f;
+  clear(acc);
+  each_pair(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1], a.row_bits, row, a.Lk, [&](int key, bool on) {
+    const int g = (opaque(threadIdx.x) & 63) >> 4;
+    const float s = dot_plain<D, IT>(row_at<IT>(qb, a.qs[1], qc, g), row_at<IT>(kb, a.ks[1], key, g));
+    const float mn = on ? fmaxf(m, s) : m, mu = mn == NEG_INF ? 0.f : mn;
+    const float alpha = on ? fast_exp2((m - mu) * a.scale_log2) : 1.f, p = fast_exp2((s - mu) * a.scale_log2);
+    m = mn;
+    l = on ? fmaf(l, alpha, p) : l;
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) acc[i] *= alpha;
+    add_plain<D, IT>(acc, p, row_at<IT>(vb, a.vs[1], key, g), on);
+  });
+  lse = l > 0.f ? fmaf(m, a.scale_log2, __builtin_log2f(l)) : NEG_INF;
+}
+// dQ (without its scale)
+template <int D, class IT, class GT>
+__device__ __forceinline__ void plain_dq(const KArgs& a, int b, int h, int qt, int row0, f32x4 (&acc)[D / 16]) {
+  const int row = row0 + (opaque(threadIdx.x) & 15), qc = min(qt * TILE + row, a.Lq - 1), hk = h / a.G;
+  const int mrow = map_row(a, b, h, a.nqt, qt);
+  const bool of32 = o_is_f32<GT>(a);
+  const char* qb = head_base(a.q, a.qs, b, h, elt_bytes<IT>());
+  const char* kb = head_base(a.k, a.ks, b, hk, elt_bytes<IT>());
+  const char* vb = head_base(a.v, a.vs, b, hk, elt_bytes<IT>());
+  const char* gb = head_base(a.dO, a.dos, b, h, elt_bytes<GT>());
+  const char* ob = head_base(a.o, a.os, b, h, of32 ? 4 : 2);
+  const float lse = a.lse[((int64_t)b * a.Hq + h) * a.Lq + qc];
+  clear(acc);
+  each_pair(a.row_ent, a.row_ptr[mrow], a.row_ptr[mrow + 1], a.row_bits, row, a.Lk, [&](int key, bool on) {
+    const int g = (opaque(threadIdx.x) & 63) >> 4;
+    const char* kr = row_at<IT>(kb, a.ks[1], key, g);
+    const float s = dot_plain<D, IT>(row_at<IT>(qb, a.qs[1], qc, g), kr);
+    const float x = dot_vo<2, D, IT, GT>(HotRows{row_at<GT>(gb, a.dos[1], qc, g), row_at<IT>(vb, a.vs[1], key, g),
+                                                 ob + (of32 ? 4 : 2) * ((int64_t)qc * a.os[1] + 4 * g), kr}, of32);
+    add_plain<D, IT>(acc, fast_exp2(fmaf(s, a.scale_log2, -lse)) * x, kr, on);
+  });
+}
+// PART: 1 = dV, 2 = dK (without its scale)
+template <int D, class IT, class GT, int PART>
+__device__ __forceinline__ void plain_dkdv(const KArgs& a, int b, int hk, int kt, int row0, f32x4 (&acc)[D / 16]) {
+  const int row = row0 + (opaque(threadIdx.x) & 15), kc = min(kt * TILE + row, a.Lk - 1);
+  const bool of32 = o_is_f32<GT>(a);
+  const char* kb = head_base(a.k, a.ks, b, hk, elt_bytes<IT>());
+  const char* vb = head_base(a.v, a.vs, b, hk, elt_bytes<IT>());
+  clear(acc);
+#pragma unroll 1
+  for (int h = hk * a.G; h < (hk + 1) * a.G; ++h) {
+    const int mc = map_row(a, b, h, a.nkt, kt);
+    const char* qb = head_base(a.q, a.qs, b, h, elt_bytes<IT>());
+    const char* gb = head_base(a.dO, a.dos, b, h, elt_bytes<GT>());
+    const char* ob = head_base(a.o, a.os, b, h, of32 ? 4 : 2);
+    each_pair(a.col_ent, a.col_ptr[mc], a.col_ptr[mc + 1], a.col_bits, row, a.Lq, [&](int q, bool on) {
+      const int g = (opaque(threadIdx.x) & 63) >> 4;
+      const char *qr = row_at<IT>(qb, a.qs[1], q, g), *gr = row_at<GT>(gb, a.dos[1], q, g);
+      const float s = dot_plain<D, IT>(qr, row_at<IT>(kb, a.ks[1], kc, g));
+      const float p = fast_exp2(fmaf(s, a.scale_log2, -a.lse[((int64_t)b * a.Hq + h) * a.Lq + q]));
+      if constexpr (PART == 1) {
+        add_plain<D, GT>(acc, p, gr, on);
+      } else {
+        const float x = dot_vo<2, D, IT, GT>(HotRows{gr, row_at<IT>(vb, a.vs[1], kc, g),
+                                                     ob + (of32 ? 4 : 2) * ((int64_t)q * a.os[1] + 4 * g), qr}, of32);
+        add_plain<D, IT>(acc, p * x, qr, on);
+      }
+    });
+  }
+}
+
 // One walk: the streamed rows of step s are in LDS buffer s % NBUF when compute(s) runs.
 // start(s, buf) issues their loads, finish(buf) writes what went through registers.
 template <int NBUF, bool DMA, int BUF, class S, class F, class C>
@@ -594,7 +746,9 @@ void fwd_s3(KArgs a) {
 
   l += __shfl_xor(l, 16);
   l = wave_sum32(l);
-  if (g == 0 && q < a.Lq) a.lse[((int64_t)b * a.Hq + h) * a.Lq + q] = l > 0.f ? fmaf(m, c2, __builtin_log2f(l)) : NEG_INF;
+  float lse = l > 0.f ? fmaf(m, c2, __builtin_log2f(l)) : NEG_INF;
+  if (not_finite(acc)) plain_fwd<D, IT>(args_again(), b, h, qt, wrow + 16 * wave, acc, l, lse);
+  if (g == 0 && q < a.Lq) a.lse[((int64_t)b * a.Hq + h) * a.Lq + q] = lse;
   __syncthreads();  // every wave is done with the operand tiles
   const int r0 = qt * TILE + wrow + 16 * wave;
   put16<D, OT>(acc, l > 0.f ? 1.f / l : 0.f, (float*)L + wave * 16 * D, a.out,
@@ -677,11 +831,13 @@ void bwd_dq_s3(KArgs a) {
   __syncthreads();
   const bool of32 = o_is_f32<OT>(a);
   add_hot<D, IT, OT>(acc, Hl[wave], l16, of32, [&](int key) {
-    return HotRows{head_base(a.dO, a.dos, b, h, elt_bytes<OT>()) + elt_bytes<OT>() * ((int64_t)qc * a.dos[1] + 4 * g),
-                   vb + elt_bytes<IT>() * ((int64_t)key * a.vs[1] + 4 * g),
+    const KArgs& a = args_again();
+    return HotRows{row_at<OT>(head_base(a.dO, a.dos, b, h, elt_bytes<OT>()), a.dos[1], qc, g),
+                   row_at<IT>(vb, a.vs[1], key, g),
                    head_base(a.o, a.os, b, h, of32 ? 4 : 2) + (of32 ? 4 : 2) * ((int64_t)qc * a.os[1] + 4 * g),
-                   kb + elt_bytes<IT>() * ((int64_t)key * a.ks[1] + 4 * g)};
+                   row_at<IT>(kb, a.ks[1], key, g)};
   });
+  if (not_finite(acc)) plain_dq<D, IT, OT>(args_again(), b, h, qt, wrow + 16 * wave, acc);
   const int r0 = qt * TILE + wrow + 16 * wave;
   put16<D, IT>(acc, a.scale, (float*)L + wave * 16 * D, a.dq,
                (int64_t)b * a.dqs[0] + (int64_t)r0 * a.dqs[1] + (int64_t)h * a.dqs[2], a.dqs[1], a.Lq - r0, lane);
@@ -738,10 +894,12 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
     Rq rq;
     Rg rg;
     const auto hot_rows = [&](int key, int q, int g4) {
-      return HotRows{gb + elt_bytes<OT>() * ((int64_t)q * a.dos[1] + 4 * g4),
-                     head_base(a.v, a.vs, b, hk, elt_bytes<IT>()) + elt_bytes<IT>() * ((int64_t)key * a.vs[1] + 4 * g4),
+      const KArgs& a = args_again();
+      const bool of32 = o_is_f32<OT>(a);
+      return HotRows{row_at<OT>(head_base(a.dO, a.dos, b, h, elt_bytes<OT>()), a.dos[1], q, g4),
+                     row_at<IT>(head_base(a.v, a.vs, b, hk, elt_bytes<IT>()), a.vs[1], key, g4),
                      head_base(a.o, a.os, b, h, of32 ? 4 : 2) + (of32 ? 4 : 2) * ((int64_t)q * a.os[1] + 4 * g4),
-                     qb + elt_bytes<IT>() * ((int64_t)q * a.qs[1] + 4 * g4)};
+                     row_at<IT>(head_base(a.q, a.qs, b, h, elt_bytes<IT>()), a.qs[1], q, g4)};
     };
     if (DK && lane < 16) Hl[wave].n[lane] = 0;
     float rl = 0.f;  // lse (threads 0 .. BN - 1) or delta (the next BN) of a row
@@ -798,6 +956,10 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
       add_hot<D, IT, OT>(dk, Hl[wave], l16, of32, [&](int q) { return hot_rows(kc, q, g); });
   }
 
+  if constexpr (DV)
+    if (not_finite(dv)) plain_dkdv<D, IT, OT, 1>(args_again(), b, hk, kt, wrow + 16 * wave, dv);
+  if constexpr (DK)
+    if (not_finite(dk)) plain_dkdv<D, IT, OT, 2>(args_again(), b, hk, kt, wrow + 16 * wave, dk);
   const int r0 = kt * TILE + wrow + 16 * wave;
   __syncthreads();
   if constexpr (DV)

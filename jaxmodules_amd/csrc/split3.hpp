@@ -5,7 +5,10 @@
 //
 // A float32 value is the exact sum of three bfloat16 pieces (8 significant
 // bits each, rounded to nearest, so of either sign), with float32's own
-// exponent range: no scales, and nothing to bound beforehand.  A float16 value
+// exponent range: no scales, and nothing to bound beforehand.  (At its ends:
+// below 2^-110 the last pieces are lost to the subnormals; infinities and what
+// rounds past bfloat16's largest value have no such pieces and leave Inf or NaN
+// in the products, which the kernels look for and form anew.)  A float16 value
 // is the sum of two, a bfloat16 value is one.  A product of two such sums takes
 // the piece products down to 2^-16 of the largest (six for two float32
 // operands, three for float32 times bfloat16); what is left out is about 2^-25
