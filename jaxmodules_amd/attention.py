@@ -474,6 +474,8 @@ def mattn_backward(q, k, v, o, lse, do, tm: bmap.TileMap, scale: float, res=None
     beside a float32 o (MATTN_DO_16)."""
     lib = _lib.load()
     _check_map(tm, q, k)
+    if do.dtype != o.dtype and (do.dtype != q.dtype or o.dtype != torch.float32):
+        raise TypeError(f"dO must have O's dtype {o.dtype}, or the inputs' {q.dtype} beside a float32 O, got {do.dtype}")
     dq = torch.empty_like(q)
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)

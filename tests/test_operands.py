@@ -26,3 +26,16 @@ def test_ready(what, x, as_is):
     assert torch.equal(x, y) and y.dtype == x.dtype
     assert y.data_ptr() % 16 == 0 and y.stride(3) == 1
     assert all(s * y.element_size() % 16 == 0 for s in y.stride()[:3])
+
+
+@pytest.mark.parametrize("q,o,do", [("float16", "float32", "bfloat16"), ("float16", "float16", "float32"),
+                                    ("bfloat16", "bfloat16", "float16"), ("float32", "float32", "bfloat16")])
+def test_upstream_gradient_of_another_dtype_is_refused(q, o, do):
+    """A dO that is neither of O's dtype nor of the inputs' beside a float32 O would be
+    read as something else."""
+    from types import SimpleNamespace
+
+    t = [torch.zeros((1, 128, 1, 64), dtype=getattr(torch, n)) for n in (q, o, do)]
+    tm = SimpleNamespace(B=1, Lq=128, Hq=1, Lk=128, Hkv=1)
+    with pytest.raises(TypeError, match="dO must have"):
+        A.mattn_backward(t[0], t[0], t[0], t[1], torch.zeros(1, 1, 128), t[2], tm, 0.125)
