@@ -94,7 +94,8 @@ enum mattn_status {
  * O), which the backward reads. */
 #define MATTN_PRECISE 4
 /* mattn_problem.flags: dO has the inputs' 16-bit dtype (do_stride counts its
- * elements) though O is float32: the gradient of a 16-bit copy of O, read as it is.
+ * elements) where O is float32: the gradient of a 16-bit copy of O, read as it is.
+ * (Beside an O of the inputs' dtype it says what holds anyway.)
  * 16-bit inputs, D <= 256, without MATTN_PRECISE (else MATTN_ERR_DTYPE). */
 #define MATTN_DO_16 16
 
@@ -333,7 +334,8 @@ int mattn_copy_rows(const mattn_row_copy* copies, int32_t n, void* stream);
 /* Static text of a status code. */
 const char* mattn_strerror(int status);
 
-/* Library ABI version (bumped on any change of the structs above). */
+/* Library ABI version (bumped on any change of the structs, flags or functions above;
+ * 9: MATTN_DO_16 and mattn_copy_rows). */
 int mattn_abi_version(void);
 
 #ifdef __cplusplus

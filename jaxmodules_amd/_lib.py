@@ -21,7 +21,7 @@ MATTN_BWD_DS = 2
 MATTN_PRECISE = 4
 MATTN_DO_16 = 16
 TILE_Q = TILE_K = 128
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 STATUS = {
     0: "MATTN_OK",

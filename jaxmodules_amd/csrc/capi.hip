@@ -20,7 +20,7 @@ using namespace mattn;
 
 namespace {
 
-constexpr int kAbiVersion = 8;
+constexpr int kAbiVersion = 9;
 
 int elem_size(int dt) { return dt == MATTN_F32 ? 4 : 2; }
 
