@@ -351,6 +351,8 @@ assert _PROBLEM.size == ctypes.sizeof(_lib.MattnProblem)
 def _problem(q, k, v, o, scale, do=None, dq=None, dk=None, dv=None):
     B, N, Hq, d = q.shape
     sq, sk, sv, so = q.stride()[:3], k.stride()[:3], v.stride()[:3], o.stride()[:3]
+    if scale > 3.4028234e38:  # past float32: infinite, which mattn_validate refuses (pack raises its own error)
+        scale = math.inf
     return _lib.MattnProblem.from_buffer_copy(_PROBLEM.pack(
         B, N, k.shape[1], Hq, k.shape[2], d, _DT[q.dtype], _DT[o.dtype], scale, 0, *sq, *sk, *sv, *so,
         *(so if do is None else do.stride()[:3]), *(sq if dq is None else dq.stride()[:3]),

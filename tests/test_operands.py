@@ -39,3 +39,15 @@ def test_upstream_gradient_of_another_dtype_is_refused(q, o, do):
     tm = SimpleNamespace(B=1, Lq=128, Hq=1, Lk=128, Hkv=1)
     with pytest.raises(TypeError, match="dO must have"):
         A.mattn_backward(t[0], t[0], t[0], t[1], torch.zeros(1, 1, 128), t[2], tm, 0.125)
+
+
+def test_scale_past_float32_is_the_library_s_to_refuse():
+    import ctypes
+
+    from jaxmodules_amd import _lib
+
+    q = torch.zeros((1, 128, 1, 64))
+    p = A._problem(q, q, q, q, 1e39)
+    assert p.scale == float("inf")
+    assert _lib.load().mattn_validate(ctypes.byref(p), None) == -2  # MATTN_ERR_SHAPE
+    assert A._problem(q, q, q, q, 3e38).scale > 2.9e38
