@@ -351,7 +351,7 @@ assert _PROBLEM.size == ctypes.sizeof(_lib.MattnProblem)
 def _problem(q, k, v, o, scale, do=None, dq=None, dk=None, dv=None):
     B, N, Hq, d = q.shape
     sq, sk, sv, so = q.stride()[:3], k.stride()[:3], v.stride()[:3], o.stride()[:3]
-    if scale > 3.4028234e38:  # past float32: infinite, which mattn_validate refuses (pack raises its own error)
+    if scale >= 3.4028235677973366e38:  # float32 rounds it to inf, which mattn_validate refuses (pack would raise)
         scale = math.inf
     return _lib.MattnProblem.from_buffer_copy(_PROBLEM.pack(
         B, N, k.shape[1], Hq, k.shape[2], d, _DT[q.dtype], _DT[o.dtype], scale, 0, *sq, *sk, *sv, *so,
@@ -504,21 +504,23 @@ class _MaskedAttention(torch.autograd.Function):
     (Q, K, V, O, LSE) instead of (Q, K, V): the backward reads the saved
     log-sum-exp rather than re-running the forward scan.
 
-    Where a gradient is needed O is computed and saved in float32 (the
-    reference's own output dtype) and a 16-bit ``out_dtype`` is a rounded copy of
-    it; otherwise the kernels round it themselves (the same values: 57 us of a
+    Where a gradient is needed (an input requires one and ``grad_mode``,
+    torch.is_grad_enabled() at the call, is on) O is computed and saved in float32
+    (the reference's own output dtype) and a 16-bit ``out_dtype`` is a rounded copy
+    of it; otherwise the kernels round it themselves (the same values: 57 us of a
     670 us bfloat16 forward at B=4 L=4096 Hq=32 d=128 was the copy).  The backward's
     delta = rowsum(dO * O) then uses the unrounded O: where one key dominates
     a row, dS = P (dP - delta) cancels, and a bfloat16 O would leave its
     rounding (2^-9 of |V|) in dQ and dK.
 
     Head dimensions between the kernels' are zero-padded here (_copy_rows): Q, K
-    and V in one launch, dO in one (converted to float32 on the way); O's and the
-    gradients' columns are taken back in one each."""
+    and V in one launch, dO in one (to float32 only where the kernels do not read it
+    in 16 bits); O's and the gradients' columns are taken back in one each."""
 
     @staticmethod
-    def forward(ctx, q, k, v, tm, scale, out_dtype, heads_major=False, precise=False):
-        grads = any(ctx.needs_input_grad[:3])
+    def forward(ctx, q, k, v, tm, scale, out_dtype, heads_major, precise, grad_mode):
+        # (needs_input_grad is set by the inputs alone, and the mode is off in here)
+        grads = grad_mode and any(ctx.needs_input_grad[:3])
         d = q.shape[3]
         D = _kernel_dim(d)
         if D != d:
@@ -550,10 +552,10 @@ class _MaskedAttention(torch.autograd.Function):
             padded = mattn_backward(q, k, v, o, lse, g, ctx.tm, ctx.scale, ctx.res, ctx.precise)
             grads = tuple(_rows_like(x, ctx.d, ctx.heads_major) for x in padded)
             _copy_rows(list(zip(padded, grads)))
-            return (*grads, None, None, None, None, None)
+            return (*grads, *(None,) * 6)
         do = _ready(do if do.dtype == gt else do.to(gt))
         dq, dk, dv = mattn_backward(q, k, v, o, lse, do, ctx.tm, ctx.scale, ctx.res, ctx.precise)
-        return dq, dk, dv, None, None, None, None, None
+        return (dq, dk, dv, *(None,) * 6)
 
 
 def _kernel_dim(d: int) -> int:
@@ -738,7 +740,7 @@ def _via_map(Q, K, V, *, is_causal=False, kernel_fn=default_kernel, mask_fn=None
     precise = use_precise(precision, scale, plan.d)
     q, k, v = _operand(Q, dt), _operand(K, dt), _operand(V, dt)
     od = _out_dtype(dt, out_dtype)
-    out = _MaskedAttention.apply(q, k, v, tm, scale, od, False, precise)
+    out = _MaskedAttention.apply(q, k, v, tm, scale, od, False, precise, torch.is_grad_enabled())
     return out[0] if plan.squeeze_batch else out
 
 
@@ -856,7 +858,7 @@ def flex_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         query, s = query.to(dt) * 0, 1.0
     # [B, H, L, E] tensors are strided [B, L, H, E] views for the kernels
     q, k, v = (_operand(x.transpose(1, 2), dt) for x in (query, key, value))
-    out = _MaskedAttention.apply(q, k, v, tm, s, _out_dtype(dt, out_dtype), True, precise)
+    out = _MaskedAttention.apply(q, k, v, tm, s, _out_dtype(dt, out_dtype), True, precise, torch.is_grad_enabled())
     return out.transpose(1, 2)
 
 
