@@ -278,10 +278,15 @@ struct Walk {
     if (i < base || i >= base + 64) fill(i);  // (uniform)
     return i - base;
   }
+  // (at() first, in a statement of its own: it may replace the window that is then read)
   __device__ __forceinline__ int first(int s) {
-    return __builtin_amdgcn_readlane(tile, at(s / SPT)) * TILE + (s % SPT) * BN;
+    const int i = at(s / SPT);
+    return __builtin_amdgcn_readlane(tile, i) * TILE + (s % SPT) * BN;
   }
-  __device__ __forceinline__ int mask(int s) { return __builtin_amdgcn_readlane(mk, at(s / SPT)); }
+  __device__ __forceinline__ int mask(int s) {
+    const int i = at(s / SPT);
+    return __builtin_amdgcn_readlane(mk, i);
+  }
 };
 
 }  // namespace s3
