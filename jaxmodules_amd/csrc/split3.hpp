@@ -114,7 +114,8 @@ constexpr int elt_bytes() { return Pieces<T>::n == 3 ? 4 : 2; }
 // n - 1: their scores are masked).  p is uniform and off 32 bits a lane, formed anew
 // each time (opaque: hoisted 64-bit addresses, two registers a chunk, spilled the
 // kernels): 64-bit row products were 80 vector instructions a step.  The validated
-// strides (Q, K, V: 128 rows within 2^31 elements) fit; WIDE (dO, not validated) takes
+// strides (Q, K, V: 128 rows within 2^31 elements, so 64 rows of float32 within 2^32
+// bytes) fit, unsigned; WIDE (dO, not validated) takes
 // 64-bit offsets when its stride needs them.
 template <int D, int ES, int ROWS, int NTH, bool WIDE, class F>
 __device__ __forceinline__ void each_chunk(const char* base, int64_t rs, int r0, int n, F&& f) {
@@ -125,7 +126,7 @@ __device__ __forceinline__ void each_chunk(const char* base, int64_t rs, int r0,
   const int r = opaque(threadIdx.x / CPR);
   if (!WIDE || rs < (1 << 24)) {
 #pragma unroll
-    for (int c = 0; c < CH; ++c) f(c, p, (uint32_t)(min(r + c * RPC, last) * (ES * (int)rs)));
+    for (int c = 0; c < CH; ++c) f(c, p, (uint32_t)min(r + c * RPC, last) * (uint32_t)(ES * (int)rs));
   } else {
 #pragma unroll
     for (int c = 0; c < CH; ++c) f(c, p + ES * ((int64_t)min(r + c * RPC, last) * rs), 0u);
