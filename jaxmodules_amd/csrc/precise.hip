@@ -14,7 +14,7 @@
 // and CU: the rate of the vector float64 FMA, but with the operands of 16 FMAs in one
 // register.  Measured against the compensated SIMT kernels, causal steps at scale 1:
 // [1, 2048, 8, 64] 4.95 -> 0.47 ms, [1, 2048, 8, 128] 10.5 -> 0.91 ms, [1, 1024, 8,
-// 256] 7.06 -> 1.09 ms (the backward's registers spill there: 58 to 87 of them).
+// 256] 7.06 -> 1.09 ms (the backward spills 58 to 76 of its 512 registers there).
 //
 // MFMA 16x16x4 layout (lane l, l16 = l % 16, g = l / 16): A row l16, k = g; B column
 // l16, k = g; C column l16, register i row 4 i + g.  Operands along d are read as 4

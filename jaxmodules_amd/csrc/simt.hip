@@ -11,9 +11,8 @@
 // dominates a row, V_k - O is small and exact to float32 rounding, while
 // dO . V_k and dO . O are two large dot products whose roundings (2^-24 of
 // |dO| |V|) would be all that is left of their difference.
-// TPR threads share a row (query or key), each holding D / TPR head dims; a
-// workgroup of 512 threads owns 512 / TPR rows of a 128-row map tile, so a
-// tile takes 128 TPR / 512 workgroups (four for TPR = 16 at D = 512).
+// 16 threads share a row (query or key), each holding 32 head dims; a workgroup
+// of 512 threads owns 32 rows of a 128-row map tile, so a tile takes four.
 #include <type_traits>
 
 #include "common.hpp"
@@ -53,22 +52,21 @@ struct Mem<bf16_tag> : Mem16<bf16_tag> {};
 template <>
 struct Mem<f16_tag> : Mem16<f16_tag> {};
 
-// keys (forward, dQ) or queries (dK/dV) per sub-block: 32, or 16 at D = 512,
-// where four [SB, D] float32 LDS tiles (the dK/dV kernel's Q, dO, O and O's
-// low parts) must fit 160 KiB
-template <int D>
-constexpr int sub_block() { return D > 256 ? 16 : 32; }
+constexpr int D = 512, TPR = 16;  // head dimension, threads per row
+constexpr int DP = D / TPR;       // head dims a thread
+constexpr int RPW = 512 / TPR, SPLIT = TILE / RPW;  // rows a workgroup, workgroups a tile
+// keys (forward, dQ) or queries (dK/dV) per sub-block: four [SB, D] float32 LDS tiles
+// (the dK/dV kernel's Q, dO, O and O's low parts) must fit 160 KiB
+constexpr int SB = 16;
 
 // mask bits of sub-block sb (SB keys or queries) of a partial tile's 128-bit
 // row (or column) at `row`, one bit per element (words [mask][64-half][row])
-template <int SB>
 __device__ __forceinline__ uint32_t sub_bits(const uint64_t* bits, int mask, int sb, int row) {
   const int first = sb * SB;
   return (uint32_t)(bits[((int64_t)mask * 2 + (first >> 6)) * TILE + row] >> (first & 63));
 }
 
 // sum over the TPR lanes of a row (consecutive lanes)
-template <int TPR>
 __device__ __forceinline__ float row_sum(float x) {
 #pragma unroll
   for (int o = 1; o < TPR; o <<= 1) x += __shfl_xor(x, o);
@@ -90,13 +88,12 @@ __device__ __forceinline__ void two_sum(float a, float b, float& s, float& e) {
 // float32's precision.  The scores of a kernel sharper than 1/sqrt(d) reach
 // tens of units (base 2 after scaling), where float32's 2^-24 relative
 // rounding alone moves the weights exp2(S - lse) by 1e-5; otherwise lo = 0.
-template <int DP, int TPR>
 __device__ __forceinline__ void score(const float* qv, const float* y, bool comp, float& hi, float& lo) {
   if (!comp) {
     float p = 0.f;
 #pragma unroll
     for (int i = 0; i < DP; ++i) p = fmaf(qv[i], y[i], p);
-    hi = row_sum<TPR>(p);
+    hi = row_sum(p);
     lo = 0.f;
     return;
   }
@@ -122,7 +119,7 @@ __device__ __forceinline__ void score(const float* qv, const float* y, bool comp
 
 // rows [r0, r0 + SB) of a [rows, D] tensor slice (row stride rs) as floats in
 // LDS; rows past n - 1 re-read row n - 1 (their scores are masked)
-template <int D, class T, int SB = sub_block<D>()>
+template <class T>
 __device__ __forceinline__ void stage_rows(float* dst, const void* base, int64_t rs, int r0, int n) {
   for (int c = threadIdx.x; c < SB * D / 4; c += 512) {
     const int r = c / (D / 4), col = 4 * (c % (D / 4));
@@ -136,11 +133,10 @@ __device__ __forceinline__ void stage_rows(float* dst, const void* base, int64_t
 // backward's dP - delta = dO . (V_k - O) then sees O to float64 accuracy,
 // which a row dominated by one key needs (V_k - O is then a small fraction of
 // |V|, and O's own float32 rounding a large part of it).
-template <int D, int TPR, class IT, class OT, bool PREC>
+template <class IT, class OT, bool PREC>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512)))
 void fwd_simt(KArgs a) {
   using acc_t = typename std::conditional<PREC, double, float>::type;
-  constexpr int DP = D / TPR, RPW = 512 / TPR, SPLIT = TILE / RPW, SB = sub_block<D>();
   constexpr int ES = std::is_same<IT, float>::value ? 4 : 2;
   __shared__ __attribute__((aligned(16))) float Ks[SB * D];
   __shared__ __attribute__((aligned(16))) float Vs[SB * D];
@@ -176,18 +172,18 @@ void fwd_simt(KArgs a) {
       const int key0 = kt * TILE + sb * SB;
       if (key0 >= a.Lk) break;
       __syncthreads();
-      stage_rows<D, IT>(Ks, kb, a.ks[1], key0, a.Lk);
-      stage_rows<D, IT>(Vs, vb, a.vs[1], key0, a.Lk);
+      stage_rows<IT>(Ks, kb, a.ks[1], key0, a.Lk);
+      stage_rows<IT>(Vs, vb, a.vs[1], key0, a.Lk);
       __syncthreads();
       uint32_t bits = 0xffffffffu;
       if (mask >= 0)
-        bits = sub_bits<SB>(a.row_bits, mask, sb, row);
+        bits = sub_bits(a.row_bits, mask, sb, row);
       float sc[SB], sl[SB];  // scores s (scaled: s * scale_log2 = sc + sl)
       float mx = NEG_INF;
 #pragma unroll
       for (int j = 0; j < SB; ++j) {
         float hi, lo;
-        score<DP, TPR>(qv, Ks + j * D + part * DP, PREC, hi, lo);
+        score(qv, Ks + j * D + part * DP, PREC, hi, lo);
         float x = hi * a.scale_log2;
         sl[j] = fmaf(hi, a.scale_log2, -x) + lo * a.scale_log2;  // rounding of x, and the low part
         if (!((bits >> j) & 1u)) x = NEG_INF;
@@ -237,10 +233,9 @@ void fwd_simt(KArgs a) {
   }
 }
 
-template <int D, int TPR, class IT, class OT, bool PREC>
+template <class IT, class OT, bool PREC>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512)))
 void bwd_dq_simt(KArgs a) {
-  constexpr int DP = D / TPR, RPW = 512 / TPR, SPLIT = TILE / RPW, SB = sub_block<D>();
   constexpr int ES = std::is_same<IT, float>::value ? 4 : 2;
   __shared__ __attribute__((aligned(16))) float Ks[SB * D];
   __shared__ __attribute__((aligned(16))) float Vs[SB * D];
@@ -281,19 +276,19 @@ void bwd_dq_simt(KArgs a) {
       const int key0 = kt * TILE + sb * SB;
       if (key0 >= a.Lk) break;
       __syncthreads();
-      stage_rows<D, IT>(Ks, kb, a.ks[1], key0, a.Lk);
-      stage_rows<D, IT>(Vs, vb, a.vs[1], key0, a.Lk);
+      stage_rows<IT>(Ks, kb, a.ks[1], key0, a.Lk);
+      stage_rows<IT>(Vs, vb, a.vs[1], key0, a.Lk);
       __syncthreads();
       uint32_t bits = 0xffffffffu;
       if (mask >= 0)
-        bits = sub_bits<SB>(a.row_bits, mask, sb, row);
+        bits = sub_bits(a.row_bits, mask, sb, row);
       for (int j = 0; j < SB; ++j) {
         float g = 0.f;
 #pragma unroll
         for (int i = 0; i < DP; ++i) g = fmaf(gv[i], (Vs[j * D + part * DP + i] - ov[i]) - ol[i], g);  // dP - delta
-        g = row_sum<TPR>(g);
+        g = row_sum(g);
         float hi, lo;
-        score<DP, TPR>(qv, Ks + j * D + part * DP, PREC, hi, lo);
+        score(qv, Ks + j * D + part * DP, PREC, hi, lo);
         float p = exp2f(fmaf(hi, a.scale_log2, -lse) + fmaf(lo, a.scale_log2, -lse_lo));
         if (!((bits >> j) & 1u)) p = 0.f;
         const float ds = p * g;
@@ -308,10 +303,9 @@ void bwd_dq_simt(KArgs a) {
   for (int i = 0; i < DP; ++i) Mem<IT>::put(a.dq, qo2 + i, dq[i] * a.scale);
 }
 
-template <int D, int TPR, class IT, class OT, bool PREC>
+template <class IT, class OT, bool PREC>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512)))
 void bwd_dkdv_simt(KArgs a) {
-  constexpr int DP = D / TPR, RPW = 512 / TPR, SPLIT = TILE / RPW, SB = sub_block<D>();
   constexpr int ES = std::is_same<IT, float>::value ? 4 : 2;
   constexpr int EO = std::is_same<OT, float>::value ? 4 : 2;
   __shared__ __attribute__((aligned(16))) float Qs[SB * D];
@@ -353,10 +347,10 @@ void bwd_dkdv_simt(KArgs a) {
         const int q0 = qt * TILE + sb * SB;
         if (q0 >= a.Lq) break;
         __syncthreads();
-        stage_rows<D, IT>(Qs, qb, a.qs[1], q0, a.Lq);
-        stage_rows<D, OT>(Gs, gb, a.dos[1], q0, a.Lq);
-        stage_rows<D, OT>(Os, ob, a.os[1], q0, a.Lq);
-        if constexpr (PREC) stage_rows<D, float>(Ol, a.o_lo + ((int64_t)b * a.Hq + h) * a.Lq * D, D, q0, a.Lq);
+        stage_rows<IT>(Qs, qb, a.qs[1], q0, a.Lq);
+        stage_rows<OT>(Gs, gb, a.dos[1], q0, a.Lq);
+        stage_rows<OT>(Os, ob, a.os[1], q0, a.Lq);
+        if constexpr (PREC) stage_rows<float>(Ol, a.o_lo + ((int64_t)b * a.Hq + h) * a.Lq * D, D, q0, a.Lq);
         if (tid < SB) {
           const int64_t rs = ((int64_t)b * a.Hq + h) * a.Lq + min(q0 + tid, a.Lq - 1);
           Ls[tid] = a.lse[rs];
@@ -365,7 +359,7 @@ void bwd_dkdv_simt(KArgs a) {
         __syncthreads();
         uint32_t bits = 0xffffffffu;
         if (mask >= 0)
-          bits = sub_bits<SB>(a.col_bits, mask, sb, row);
+          bits = sub_bits(a.col_bits, mask, sb, row);
         for (int j = 0; j < SB; ++j) {
           float gd = 0.f;
 #pragma unroll
@@ -374,9 +368,9 @@ void bwd_dkdv_simt(KArgs a) {
             if constexpr (PREC) dvo -= Ol[j * D + part * DP + i];
             gd = fmaf(dvo, Gs[j * D + part * DP + i], gd);  // dP - delta
           }
-          gd = row_sum<TPR>(gd);
+          gd = row_sum(gd);
           float hi, lo;
-          score<DP, TPR>(kv, Qs + j * D + part * DP, PREC, hi, lo);
+          score(kv, Qs + j * D + part * DP, PREC, hi, lo);
           float p = exp2f(fmaf(hi, a.scale_log2, -Ls[j]) + fmaf(lo, a.scale_log2, -Llo[j]));
           if (!((bits >> j) & 1u)) p = 0.f;
           const float ds = p * gd;
@@ -399,20 +393,19 @@ void bwd_dkdv_simt(KArgs a) {
   }
 }
 
-// the stages of one (input, output) combination: D = 512, 16 threads per row
+// the stages of one (input, output) combination
 template <class IT, class OT>
 struct Simt {
-  static constexpr int D = 512, TPR = 16, SPLIT = TILE * TPR / 512;
   template <bool PREC>
   static void fwd(const KArgs& a, int grid, hipStream_t st) {
-    hipLaunchKernelGGL((fwd_simt<D, TPR, IT, OT, PREC>), dim3(grid * SPLIT), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((fwd_simt<IT, OT, PREC>), dim3(grid * SPLIT), dim3(512), 0, st, a);
   }
   template <bool PREC>
   static void bwd(const KArgs& a, int stage, int q_grid, int kv_grid, hipStream_t st) {
     if (stage == MATTN_BWD_DKDV)
-      hipLaunchKernelGGL((bwd_dkdv_simt<D, TPR, IT, OT, PREC>), dim3(kv_grid * SPLIT), dim3(512), 0, st, a);
+      hipLaunchKernelGGL((bwd_dkdv_simt<IT, OT, PREC>), dim3(kv_grid * SPLIT), dim3(512), 0, st, a);
     else if (stage == MATTN_BWD_DQ)
-      hipLaunchKernelGGL((bwd_dq_simt<D, TPR, IT, OT, PREC>), dim3(q_grid * SPLIT), dim3(512), 0, st, a);
+      hipLaunchKernelGGL((bwd_dq_simt<IT, OT, PREC>), dim3(q_grid * SPLIT), dim3(512), 0, st, a);
     // MATTN_BWD_PRE: nothing, these kernels form dP - delta per pair from O
   }
 };

@@ -99,8 +99,8 @@ def test_causal_fwd_bwd(dtype, d):
     run_case((2, 384, 384, 2, 2, d), dict(is_causal=True, block_size=128), dtype)
 
 
-# head dimension 256: the float32 SIMT kernels for every input dtype (ragged
-# lengths, grouped heads, a partial-tile mask, both output dtypes)
+# head dimension 256: the float32-accuracy matrix-core kernels for every input dtype
+# (ragged lengths, grouped heads, a partial-tile mask, both output dtypes)
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
 def test_d256_causal_gqa_fwd_bwd(dtype):
     run_case((2, 300, 300, 4, 2, 256), dict(is_causal=True, block_size=128), dtype,
