@@ -272,8 +272,10 @@ struct Walk {
   __device__ __forceinline__ void fill(int i) {
     base = i;
     const int e = e0 + min(i + (int)(threadIdx.x & 63), n / SPT - 1);
-    tile = ent[2 * e];
-    mk = ent[2 * e + 1];
+    // waited for here: left to where they are next read, the wait stands in every step's
+    // way, and for the rows it has in flight too (float32 step 330 -> 360 us)
+    tile = opaque(ent[2 * e]);
+    mk = opaque(ent[2 * e + 1]);
   }
   __device__ __forceinline__ int at(int i) {  // index of entry i in the window
     if (i < base || i >= base + 64) fill(i);  // (uniform)
