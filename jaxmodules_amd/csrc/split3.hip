@@ -182,11 +182,39 @@ __device__ __forceinline__ void dot_step(Dot<D, NA, NB, C>& x, const Frag<NA>& a
   y.template end<KD>();
 }
 
+// S = A X along d for both 16-row blocks: tile at byte address ra
+template <int WANT, Chains C, int D, int NA, int NX>
+__device__ __forceinline__ void one_dot(uint32_t ra, const Frag<NX> (&x)[D / 32], f32x4 (&st)[2]) {
+  constexpr int PF = ahead(WANT, 2 * NA), PL = 2 * BN * D;
+  Frag<NA> f0[PF + 1], f1[PF + 1];
+  Dot<D, NA, NX, C> s0, s1;
+  pipe<D / 32, PF, 2 * NA>(
+      [&](auto ic, auto sc) {
+        constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
+        rd<0, PL>(f0[sl], ra ^ (uint32_t)(64 * kd));
+        rd<32 * D, PL>(f1[sl], ra ^ (uint32_t)(64 * kd));
+      },
+      [&](auto ic, auto sc) {
+        constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
+        landed(f0[sl]);
+        landed(f1[sl]);
+        dot_step<kd>(s0, f0[sl], x[kd], s1, f1[sl], x[kd]);
+      });
+  st[0] = s0.total();
+  st[1] = s1.total();
+}
 // S = A X and dP = A2 X2 along d for both 16-row blocks t: tiles at byte addresses ra, rb
-// (block by block, or, ONE, both at each step)
+// (block by block; ONE: both blocks at each step; LINKS: one product after the other, whose
+// operands in flight then leave room for the chains: side by side, float32 at D = 256
+// spilled 88 and 117 registers, dK/dV 360 -> 460 and dQ 321 -> 476 us of [1, 2048, 8])
 template <int WANT, Chains C, int D, int NA, int NX, int NB, int NY>
 __device__ __forceinline__ void two_dots(uint32_t ra, uint32_t rb, const Frag<NX> (&x)[D / 32], const Frag<NY> (&y)[D / 32],
                                          f32x4 (&st)[2], f32x4 (&dp)[2]) {
+  if constexpr (C == LINKS) {
+    one_dot<1, C, D, NA>(ra, x, st);
+    one_dot<1, C, D, NB>(rb, y, dp);
+    return;
+  }
   constexpr int PF = ahead(WANT, NA + NB), PL = 2 * BN * D, N = D / 32;
   Frag<NA> fa[PF + 1];
   Frag<NB> fb[PF + 1];
@@ -214,26 +242,6 @@ __device__ __forceinline__ void two_dots(uint32_t ra, uint32_t rb, const Frag<NX
           dp[t] = p[u].total();
         }
       });
-}
-template <Chains C, int D, int NA, int NX>
-__device__ __forceinline__ void one_dot(uint32_t ra, const Frag<NX> (&x)[D / 32], f32x4 (&st)[2]) {
-  constexpr int PF = ahead(2, 2 * NA), PL = 2 * BN * D;
-  Frag<NA> f0[PF + 1], f1[PF + 1];
-  Dot<D, NA, NX, C> s0, s1;
-  pipe<D / 32, PF, 2 * NA>(
-      [&](auto ic, auto sc) {
-        constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
-        rd<0, PL>(f0[sl], ra ^ (uint32_t)(64 * kd));
-        rd<32 * D, PL>(f1[sl], ra ^ (uint32_t)(64 * kd));
-      },
-      [&](auto ic, auto sc) {
-        constexpr int kd = decltype(ic)::value, sl = decltype(sc)::value;
-        landed(f0[sl]);
-        landed(f1[sl]);
-        dot_step<kd>(s0, f0[sl], x[kd], s1, f1[sl], x[kd]);
-      });
-  st[0] = s0.total();
-  st[1] = s1.total();
 }
 // (forward and backward alike where gradients are float32: P = exp2(S - lse) takes S as
 // lse has it.  16-bit gradients at D = 256 hide the difference by their own rounding.)
@@ -711,7 +719,7 @@ void fwd_s3(KArgs a) {
           if (!__any((w & 0x000f000fu) != 0)) return;  // no allowed key of the wave's rows here
         }
         f32x4 st[2];
-        one_dot<fwd_chains<D>(), D, NP>(lds_addr(Kl) + ra, qf, st);
+        one_dot<2, fwd_chains<D>(), D, NP>(lds_addr(Kl) + ra, qf, st);
         if (mask >= 0) {
 #pragma unroll
           for (int t = 0; t < 2; ++t)
@@ -929,7 +937,7 @@ __device__ __forceinline__ void dkdv_s3(const KArgs& a, uint16_t* L, float* Rl, 
             if (!__any((w & 0x000f000fu) != 0)) return;
           }
           f32x4 st[2], dp[2];
-          if constexpr (!DK) one_dot<bwd_chains<D, IT>(), D, NP>(lds_addr(Ql) + ra, kf, st);
+          if constexpr (!DK) one_dot<2, bwd_chains<D, IT>(), D, NP>(lds_addr(Ql) + ra, kf, st);
           else two_dots<D == 128 ? 1 : 2, bwd_chains<D, IT>(), D, NP, NP, NG, NP>(lds_addr(Ql) + ra, lds_addr(Gl) + ra, kf, vf, st, dp);
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
