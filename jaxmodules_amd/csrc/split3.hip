@@ -492,17 +492,18 @@ __device__ __forceinline__ void add_hot(f32x4 (&acc)[D / 16], HotList<MAX>& list
     const bool on = n < nh;
     const int2 pw = list.pair[l16][n];
     const HotRows p = rows(on ? pw.x : 0);
-    // every load of a round in flight at once, where there are registers (D = 256: not)
-    constexpr int U = D == 256 ? 2 : D / 16;
+    // at D = 64 every load of a round in flight at once; beyond, the registers that takes cost
+    // the walk more (D = 128: 86 moves a step to and from the accumulation registers)
+    constexpr int U = D == 64 ? 4 : 2;
     f32x4 x[D / 16];
-    if constexpr (D != 256) {
+    if constexpr (D == 64) {
 #pragma unroll
       for (int mt = 0; mt < D / 16; ++mt) x[mt] = load4<IT>(p.x + 16 * elt_bytes<IT>() * mt);
     }
     const float ds = __int_as_float(pw.y) * dot_vo<U, D, IT, GT>(p, of32);
 #pragma unroll
     for (int mt = 0; mt < D / 16; ++mt) {
-      if constexpr (D == 256) x[mt] = load4<IT>(p.x + 16 * elt_bytes<IT>() * mt);
+      if constexpr (D != 64) x[mt] = load4<IT>(p.x + 16 * elt_bytes<IT>() * mt);
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[mt][e] = on ? fmaf(ds, x[mt][e], acc[mt][e]) : acc[mt][e];
     }
