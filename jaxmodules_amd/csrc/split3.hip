@@ -22,13 +22,19 @@
 // spilling; for float32 at D = 64 its dK/dV spilled at two waves a SIMD.  The price is
 // LDS: a streamed operand is read per 16 rows, 125 bytes a clock and CU at the matrix
 // cores' full rate.
-// Measured, causal steps: float32 [2, 2048, 8, 64] fwd 465 -> 97 us, dK/dV 768 -> 144,
-// dQ 596 -> 113 against the SIMT kernels; bfloat16 [1, 4096, 8, 256] fwd 4322 -> 192 us,
-// dK/dV 14370 -> 579, dQ 4811 -> 248 (32-row waves sharing columns: 326, 750, 708).
-// The error against float64 is 0.6 to 1.0 times that of the SIMT kernels they replaced
+// Measured, causal steps, kernel by kernel in a trace (with gaps between them, at another
+// clock than a whole step's, so they don't add up to one): float32 [2, 2048, 8, 64]
+// fwd 465 -> 97 us, dK/dV 768 -> 150, dQ 596 -> 115 against the SIMT kernels; bfloat16
+// [1, 4096, 8, 256] fwd 4322 -> 204 us, dK/dV 14370 -> 588, dQ 4811 -> 264.  32-row waves
+// sharing columns: 326, 750, 708 beside 192, 579, 248.  (Those before the shorter chains
+// of Dot, the pairs of HOT and the check for Inf and NaN, which together cost 0 to 6%,
+// 12% for float32 dK/dV at D = 256.  Logits of standard deviation 8, most rows dominated
+// by one key: dK/dV 199 and 677 us, dQ 129 and 274.)
+// The error against float64 is 0.6 to 1.1 times that of the SIMT kernels they replaced
 // (0.7 and 0.8 of it for O and the gradients of that float32 step) over logits of standard
-// deviation 1 to 32; where one key of a large positive dot product has nearly all of a
-// row's weight, O is up to 1.3 and dQ up to 1.4 times as far off (1e-7 of the norm).
+// deviation 1 to 32 and windows of two keys; rows of one key give dQ = dK = 0 exactly.
+// Where one key of a large positive dot product has nearly all of a row's weight, O is up
+// to 1.3 and dQ up to 1.4 times as far off (1e-7 of the norm).
 // float32 at D = 64 is bound by vector instructions (270 a step and wave against 48 MFMAs
 // of 16 cycles; half of them split the streamed rows).
 //
@@ -407,15 +413,15 @@ __device__ __forceinline__ float dot_vo(const HotRows& p, bool of32) {
 // (2^-24 of |dO| |V|) would be all that is left of the difference; V - O is small there
 // and exact to O's own rounding.  (Left to the difference, dQ and dK of rows with a weight
 // of 0.9 or more were 2.4 to 4.9 times as far off.)
-// The check and the list cost dK/dV 2 to 5% and dQ 0 to 4% where no row is dominated (144
-// -> 149 and 115 -> 116 us for float32 [2, 2048, 8, 64]; 589 -> 600 and 254 -> 264 for
-// bfloat16 [1, 4096, 8, 256]); at 1/4 instead of 1/2 they found no error to take away.
+// Where no row is dominated the check and the list cost dK/dV 1 to 2% and dQ nothing that
+// three traces resolve (float32 [2, 2048, 8, 64] dK/dV 148 -> 150 us, dQ 116 -> 115, at
+// D = 128 255 -> 260 and 237 -> 236); at 1/4 instead of 1/2 they found no error to take away.
 // A step leaves its hot pairs out of dS and notes them, up to MAX for each of the wave's
 // rows; they are added after the walk, when its operands' registers are free and all 16
 // rows have theirs formed at once (dK/dV of such float32 rows at D = 64, one dominant key
-// each: 207 us; formed in each step, 16 rows of one pair: 236).  A query (dQ) has no more than two.  A key that more
-// than eight queries lean on (the first one of a sequence, often) has the rest formed in
-// their step, hot_rest().
+// each: 207 us; formed in each step, 16 rows of one pair: 236).  A query (dQ) has no more
+// than two.  A key that more than eight queries lean on (the first one of a sequence,
+// often) has the rest formed in their step, hot_rest().
 constexpr float HOT = 0.5f;
 constexpr int HOT_Q = 2, HOT_K = 8;
 template <int MAX>
