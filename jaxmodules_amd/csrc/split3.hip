@@ -524,7 +524,11 @@ __device__ __forceinline__ void add_hot(f32x4 (&acc)[D / 16], HotList<MAX>& list
 // there forms its 16 rows again in plain float32, pair by allowed pair, which gives the
 // infinities and NaNs that the arithmetic of the inputs has.  Lanes as before: l16 the row,
 // g its columns 16 j + 4 g .. + 3.  (g is re-defined for each pair, so that the own row's
-// columns are not held over the loop.)
+// columns are not held over the loop.)  A pair takes a wave about 1.4 us, most of it
+// waiting, so this is slow: the causal steps above 2.4 and 16 ms with an Inf in one row of
+// V (0.43 and 1.1 without).  NaN stays NaN whatever is added, so a wave whose rows are NaN
+// throughout is done: NaN everywhere, a diverged problem's state, 0.5 and 1.5 ms (walked
+// to the end 10.6 and 91).
 template <int N>
 __device__ __forceinline__ bool not_finite(const f32x4 (&acc)[N]) {
   float t = 0.f;
@@ -534,10 +538,21 @@ __device__ __forceinline__ bool not_finite(const f32x4 (&acc)[N]) {
     for (int e = 0; e < 4; ++e) t = fmaf(acc[i][e], 0.f, t);
   return __builtin_expect(__any(!(t == 0.f)), 0);
 }
+template <int N>
+__device__ __forceinline__ bool all_nan(const f32x4 (&acc)[N]) {
+  bool r = true;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r &= !(acc[i][e] == acc[i][e]);
+  return r;
+}
 // f(other, on): every position `other` < n of the present tiles of a map row (or column)
-// with an allowed pair in the wave, on where the lane's own row has it
-template <class F>
-__device__ __forceinline__ void each_pair(const int* ent, int e0, int e1, const uint64_t* bits, int row, int n, F&& f) {
+// with an allowed pair in the wave, on where the lane's own row has it; looks every 16
+// positions whether all lanes are done()
+template <class F, class E>
+__device__ __forceinline__ void each_pair(const int* ent, int e0, int e1, const uint64_t* bits, int row, int n, F&& f,
+                                          E&& done) {
 #pragma unroll 1
   for (int e = e0; e < e1; ++e) {
     const int first = ent[2 * e] * TILE, mask = ent[2 * e + 1];
@@ -548,6 +563,7 @@ __device__ __forceinline__ void each_pair(const int* ent, int e0, int e1, const 
       for (int i = 0; i < 64 && first + 64 * half + i < n; ++i) {
         const bool on = (w >> i) & 1u;
         if (__any(on)) f(first + 64 * half + i, on);
+        if (i % 16 == 15 && __all(done())) return;
       }
     }
   }
@@ -579,7 +595,8 @@ __device__ __forceinline__ void clear(f32x4 (&acc)[N]) {
   for (int i = 0; i < N; ++i) acc[i] = f32x4{};
 }
 // The wave's 16 rows from row0 (of tile qt or kt: TILE t + row0) once more.
-// forward: O times the weights' sum l, and lse
+// forward: O times the weights' sum l, and lse.  l and lse come in as the walk had them: a
+// finite l says that every score was finite, and then both hold whatever V is.
 template <int D, class IT>
 __device__ __forceinline__ void plain_fwd(const KArgs& a, int b, int h, int qt, int row0, f32x4 (&acc)[D / 16], float& l,
                                           float& lse) {
@@ -588,6 +605,8 @@ __device__ __forceinline__ void plain_fwd(const KArgs& a, int b, int h, int qt, 
   const char* qb = head_base(a.q, a.qs, b, h, elt_bytes<IT>());
   const char* kb = head_base(a.k, a.ks, b, hk, elt_bytes<IT>());
   const char* vb = head_base(a.v, a.vs, b, hk, elt_bytes<IT>());
+  const float l0 = l;
+  const bool held = l0 * 0.f == 0.f;
   float m = NEG_INF;
   l = 0.f;
   clear(acc);
@@ -601,8 +620,9 @@ __device__ __forceinline__ void plain_fwd(const KArgs& a, int b, int h, int qt, 
 #pragma unroll
     for (int i = 0; i < D / 16; ++i) acc[i] *= alpha;
     add_plain<D, IT>(acc, p, row_at<IT>(vb, a.vs[1], key, g), on);
-  });
-  lse = l > 0.f ? fmaf(m, a.scale_log2, __builtin_log2f(l)) : NEG_INF;
+  }, [&] { return all_nan(acc) && (held || !(l == l)); });
+  if (held && all_nan(acc)) l = l0;
+  else lse = l > 0.f ? fmaf(m, a.scale_log2, __builtin_log2f(l)) : NEG_INF;
 }
 // dQ (without its scale)
 template <int D, class IT, class GT>
@@ -624,7 +644,7 @@ __device__ __forceinline__ void plain_dq(const KArgs& a, int b, int h, int qt, i
     const float x = dot_vo<2, D, IT, GT>(HotRows{row_at<GT>(gb, a.dos[1], qc, g), row_at<IT>(vb, a.vs[1], key, g),
                                                  ob + (of32 ? 4 : 2) * ((int64_t)qc * a.os[1] + 4 * g), kr}, of32);
     add_plain<D, IT>(acc, fast_exp2(fmaf(s, a.scale_log2, -lse)) * x, kr, on);
-  });
+  }, [&] { return all_nan(acc); });
 }
 // PART: 1 = dV, 2 = dK (without its scale)
 template <int D, class IT, class GT, int PART>
@@ -652,7 +672,7 @@ __device__ __forceinline__ void plain_dkdv(const KArgs& a, int b, int hk, int kt
                                                      ob + (of32 ? 4 : 2) * ((int64_t)q * a.os[1] + 4 * g), qr}, of32);
         add_plain<D, IT>(acc, p * x, qr, on);
       }
-    });
+    }, [&] { return all_nan(acc); });
   }
 }
 

@@ -61,3 +61,32 @@ def test_values_that_are_not_finite(dtype, d, what, value):
         assert torch.equal(a[inf], b[inf]), name
         fits = b.isfinite()
         assert ((a - b)[fits].norm() <= rel * b[fits].norm()).item(), name
+
+
+@pytest.mark.parametrize("dtype,d", KINDS)
+@pytest.mark.parametrize("what", ["q", "v", "do", "v and k", "q and k and v"])
+def test_tensors_of_nan(dtype, d, what):
+    """NaN wherever an allowed pair is, 0 in the rows and columns that have none (1 query in
+    7, 1 key in 5), and a log-sum-exp that is right where only V is NaN: dV is finite."""
+    import jaxmodules_amd as jm
+
+    N, H, dt = 150, 2, getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(d + 1)
+    t = {n: torch.randn((1, N, H, d), generator=gen, device="cuda").to(dt if n != "do" else torch.float32)
+         for n in ("q", "k", "v", "do")}
+    for n in what.split(" and "):
+        t[n].fill_(float("nan"))
+    if what == "v and k":  # (one key: the queries before it have finite scores)
+        t["k"].nan_to_num_(1.0)[0, 70, 1, 5] = INF
+    i = torch.arange(N, device="cuda")
+    allowed = (i[:, None] >= i[None, :]) & (i[:, None] % 7 != 3) & (i[None, :] % 5 != 2)
+    q, k, v = (t[n].requires_grad_() for n in ("q", "k", "v"))
+    o = jm.masked_attention_via_map(q, k, v, mask_fn=lambda b, h, q, k: (q >= k) & (q % 7 != 3) & (k % 5 != 2))
+    got = [o, *torch.autograd.grad(o, (q, k, v), t["do"])]
+    want = _reference(*(t[n].detach()[0] for n in ("q", "k", "v", "do")), allowed)
+    rel = 1e-5 if dtype == "float32" else 4e-3
+    for name, a, b in zip(("O", "dQ", "dK", "dV"), got, want):
+        a = a.detach()[0].double()
+        fits = b.isfinite()
+        assert torch.equal(a.isfinite(), fits), name
+        assert ((a - b)[fits].norm() <= rel * b[fits].norm()).item(), name
